@@ -8,7 +8,12 @@ structure-of-arrays in HBM.  One bench step is one loop of the three tasks
 metric is wire-updates/s = wires x loops / wall time, inputs resident in HBM.
 Policy (default): SCALED, with the ATOMIC reduction fused into
 calc_new_currents; --policy selects EXACT (bit-identical to the oracle), RECIP
-or FAST, and `detail.policies` times all four.
+or FAST, and `detail.policies` times all four.  The timed loops execute every
+one of the 10000 inner steps (OPT_ALL_STEPS), so that the rate and the
+roofline are those of the work the metric counts; the library's default, which
+ends a wave's steps where its state repeats itself (same bits), is
+`detail.early_end`, and is what the batched, served, FP64 and calling-form
+rows run.
 
 Printed: one JSON line (rank 0) with the metric, a `roofline` object for the
 dominant kernel (calc_new_currents, FP32 VALU-bound: executed flops over the
@@ -649,6 +654,7 @@ def main():
     log(f"[bench] generated+uploaded {W} wires / {N} nodes / {P} pieces in "
         f"{time.perf_counter() - t0:.1f} s")
     ctx.set_timing(True)
+    ctx.set_option(C.OPT_ALL_STEPS, 1)
     if args.warmup:
         ctx.run_loops(args.warmup, policy=policy, mode=mode)
     log(f"[bench] warmup {args.warmup} loops done; timing {args.steps} loops")
@@ -680,7 +686,8 @@ def main():
         "data": f"synthetic (load_circuit generator, seed 12345, {args.profile} profile)",
         "config": {"workload": f"{P} pieces x {N // P} nodes x {W // P} wires/piece "
                                f"({W} wires, {N} nodes), 95% in-piece, seed 12345, "
-                               f"WIRE_SEGMENTS=10, 10000 inner steps/loop, FP32, SoA",
+                               f"WIRE_SEGMENTS=10, 10000 inner steps/loop, all executed, "
+                               f"FP32, SoA",
                    "policy": args.policy, "reduction": args.mode,
                    "parallelism": "single GPU"},
         # calc_new_currents is FP32 vector-ALU bound.  `achieved` is the FP32
@@ -762,6 +769,7 @@ def main():
         ctx_s = C.Context(0)
         ctx_s.generate_device(C.GenParams(**wl, profile=C.PROFILE_STABLE))
         ctx_s.set_timing(True)
+        ctx_s.set_option(C.OPT_ALL_STEPS, 1)
         ctx_s.run_loops(1, policy=policy, mode=mode)
         r5, w5, k5 = time_loops(C, ctx_s, 4, policy, mode)
         ms = k5[C.CALC_NEW_CURRENTS][0]
@@ -770,6 +778,17 @@ def main():
             "tflops_executed": ef * C.STEPS * W / ms / 1e9,
             "tflops_reference_equivalent": FLOPS_PER_WIRE_STEP * C.STEPS * W / ms / 1e9}
         log(f"[bench] stable profile: {detail['stable_profile']}")
+        # The default: a wave's steps end where its state repeats itself.
+        early = {}
+        for prof, cx in (("reference", ctx), ("stable", ctx_s)):
+            cx.set_option(C.OPT_ALL_STEPS, 0)
+            for name in ("exact", "recip", "fast", "scaled"):
+                cx.run_loops(2, policy=policy_of(C, name), mode=mode)
+                r7, w7, k7 = time_loops(C, cx, 10, policy_of(C, name), mode)
+                early[f"{prof}/{name}"] = {"wire_updates_per_s": W * 10 / w7,
+                                           "cnc_ms": k7[C.CALC_NEW_CURRENTS][0]}
+        detail["early_end"] = early
+        log(f"[bench] early end: {early}")
         ctx_s.close()
     out["detail"] = detail
     ctx.close()

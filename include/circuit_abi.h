@@ -116,8 +116,8 @@ enum {
  *           loop and fused multiply-adds; voltages materialised every step.
  *   FAST  : RECIP with the internal-voltage update substituted into the next
  *           step's current update (a tridiagonal update of the 10 currents per
- *           step: 20 FMAs and 8 adds).  Every step's currents are computed; internal
- *           voltages are formed from the final currents.
+ *           step: 20 FMAs and 8 adds).  Internal voltages are formed from the
+ *           final currents.
  *   SCALED: FAST's update iterated as the deviation from its fixed point (one
  *           tridiagonal solve per wire and loop), scaled by the coupling
  *           coefficient and split into its mirror-symmetric and
@@ -125,6 +125,9 @@ enum {
  *           each step is 6 adds and 10 FMAs, plus 10 multiplies per 4 steps.
  *           Used for wires shown to contract or to diverge; other wires take
  *           FAST's step.
+ * Every policy stops stepping a wave of wires early where their states repeat
+ * themselves, with the same bits as if every step were executed
+ * (CKT_OPT_ALL_STEPS); a server with EXACT executes every step.
  * RECIP, FAST and SCALED are not bit-exact; their error is checked against
  * 1e-5.  FAST and SCALED write a wire whose currents left the finite range as
  * all NaN, which is where the reference recurrence ends such a wire. */
@@ -347,8 +350,12 @@ enum {
                                     wires; each lane relaxes that many one after another */
   CKT_OPT_TILE_SPAN = 7,         /* 0 (default): tiles end at piece ends; 1: adjacent pieces
                                     of a circuit form one run, only its last tile is partial */
-  CKT_OPT_TILE_ORDER = 8         /* 0 (default): runs in the order given; 1: longest run
+  CKT_OPT_TILE_ORDER = 8,        /* 0 (default): runs in the order given; 1: longest run
                                     first; 2: interleaved, tile k of every run before tile k+1 */
+  CKT_OPT_ALL_STEPS = 9          /* 0 (default): the wires of a wave stop stepping once the
+                                    state of each is found, bit for bit, to repeat itself, so
+                                    that the steps left cannot change the result; 1: every step
+                                    is executed.  Results are the same bits either way. */
 };
 int ckt_ctx_set_option(ckt_ctx_t* ctx, int option, int64_t value);
 

@@ -37,7 +37,7 @@ POLICY_EXACT, POLICY_RECIP, POLICY_FAST, POLICY_SCALED = 0, 1, 2, 3
 REDUCE_ATOMIC, REDUCE_CSR, REDUCE_CSR_KAHAN64 = 0, 1, 2
 PROFILE_REFERENCE, PROFILE_STABLE = 0, 1
 (OPT_STEPS, OPT_CNC_BLOCK, OPT_PERSISTENT, OPT_WAVES_PER_SIMD, OPT_DSC_ATOMIC_IMPL,
- OPT_FUSE_DSC, OPT_WIRES_PER_LANE, OPT_TILE_SPAN, OPT_TILE_ORDER) = range(9)
+ OPT_FUSE_DSC, OPT_WIRES_PER_LANE, OPT_TILE_SPAN, OPT_TILE_ORDER, OPT_ALL_STEPS) = range(10)
 
 # CircuitNode / CircuitWire / CircuitPiece records (circuit.h:35-70).
 NODE = np.dtype([("charge", "<f4"), ("voltage", "<f4"), ("capacitance", "<f4"),

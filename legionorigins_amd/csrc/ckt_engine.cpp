@@ -754,9 +754,10 @@ int Engine::cnc(const std::vector<PieceRef>& refs, int policy, bool fuse_dsc) {
     int grid = num_cus_ * 4 * waves / waves_per_block;
     if (grid > (int)t.n) grid = (int)t.n;
     e = launch_cnc_persistent(policy, fuse_dsc, d_table_, (const Tile*)t.p, t.n, block, grid,
-                              d_counters_, steps_, stream_);
+                              d_counters_, steps_, all_steps_ != 0, stream_);
   } else {
-    e = launch_cnc(policy, fuse_dsc, d_table_, (const Tile*)t.p, t.n, block, steps_, stream_);
+    e = launch_cnc(policy, fuse_dsc, d_table_, (const Tile*)t.p, t.n, block, steps_,
+                   all_steps_ != 0, stream_);
   }
   if (e != hipSuccess) return hip_fail(e, "calc_new_currents launch");
   return timed_end(CKT_CALC_NEW_CURRENTS, a);
@@ -1001,9 +1002,10 @@ int Engine::run_graph(const std::vector<PieceRef>& refs, int policy, int mode, i
   int st;
   if ((st = ensure_table())) return st;
   uint64_t key = fnv(1469598103934665603ull, refs.data(), refs.size() * sizeof(PieceRef));
-  const int64_t cfg[12] = {policy,           mode,       steps_,          cnc_block_,
+  const int64_t cfg[13] = {policy,           mode,       steps_,          cnc_block_,
                            persistent_,      waves_per_simd_, dsc_atomic_impl_, fuse_dsc_,
-                           wires_per_lane_,  tile_span_, tile_order_,     (int64_t)generation_};
+                           wires_per_lane_,  tile_span_, tile_order_,     all_steps_,
+                           (int64_t)generation_};
   key = fnv(key, cfg, sizeof(cfg));
   auto it = graphs_.find(key);
   hipGraphExec_t exec = nullptr;
@@ -1067,6 +1069,7 @@ int Engine::set_option(int opt, int64_t v) {
       if (v < 0 || v > 2) return fail(CKT_ERR_INVALID_ARG, "tile order must be 0, 1 or 2");
       tile_order_ = (int)v;
       return CKT_OK;
+    case OPT_ALL_STEPS: all_steps_ = v ? 1 : 0; return CKT_OK;
     default: return fail(CKT_ERR_INVALID_ARG, "unknown option");
   }
 }
@@ -1082,6 +1085,7 @@ int64_t Engine::option(int opt) const {
     case OPT_WIRES_PER_LANE: return wires_per_lane_;
     case OPT_TILE_SPAN: return tile_span_;
     case OPT_TILE_ORDER: return tile_order_;
+    case OPT_ALL_STEPS: return all_steps_;
     default: return -1;
   }
 }

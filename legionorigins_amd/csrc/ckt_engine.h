@@ -96,6 +96,7 @@ enum EngineOption {
   OPT_WIRES_PER_LANE = 6,   // calc_new_currents tile = workgroup size x this (1, 2, 4) wires
   OPT_TILE_SPAN = 7,        // 0: tiles within a piece; 1: within runs of adjacent pieces
   OPT_TILE_ORDER = 8,       // 0: as given; 1: longest runs first; 2: runs interleaved
+  OPT_ALL_STEPS = 9,        // 1: every inner step is executed (no early end)
 };
 
 class Engine {
@@ -229,6 +230,7 @@ class Engine {
   int wires_per_lane_ = 1;
   int tile_span_ = 0;
   int tile_order_ = 0;
+  int all_steps_ = 0;
   bool timing_ = false;
   std::vector<Pending> pending_;
   std::vector<hipEvent_t> event_pool_;

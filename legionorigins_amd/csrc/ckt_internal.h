@@ -57,12 +57,13 @@ struct PieceTile {
 
 // Host launchers (defined in ckt_kernels.hip).  All are asynchronous on `s`.
 // fuse_dsc adds each wire's two charge contributions with float atomics at the
-// end of the relaxation (the ATOMIC distribute_charge, fused).
+// end of the relaxation (the ATOMIC distribute_charge, fused); all_steps
+// executes every step also where the state repeats itself.
 hipError_t launch_cnc(int policy, bool fuse_dsc, const DevCircuit* circuits, const Tile* tiles,
-                      uint32_t ntiles, int block, int steps, hipStream_t s);
+                      uint32_t ntiles, int block, int steps, bool all_steps, hipStream_t s);
 hipError_t launch_cnc_persistent(int policy, bool fuse_dsc, const DevCircuit* circuits,
                                  const Tile* tiles, uint32_t ntiles, int block, int grid,
-                                 uint32_t* counters, int steps, hipStream_t s);
+                                 uint32_t* counters, int steps, bool all_steps, hipStream_t s);
 hipError_t launch_dsc_atomic(const DevCircuit* circuits, const Tile* tiles, uint32_t ntiles,
                              int block, hipStream_t s);
 // Dynamic LDS bytes of the LDS-privatised reduction for pieces of up to

@@ -82,6 +82,113 @@ __device__ __forceinline__ void div_fixed_group(float (&q)[N], const float (&a)[
 // cycles; running the tail on a wire that could skip it is also correct).
 __device__ __forceinline__ bool wave_all(bool p) { return __all(p); }
 
+// ---------------------------------------------------------------------------
+// The end of a loop whose state repeats itself.
+//
+// After its first step a wire's state is its ten currents: the internal
+// voltages are the same function of the currents in every later step, so the
+// step maps currents to currents and nothing else.  If the currents after
+// step j are, bit for bit, those after step j - k, they go through the same k
+// values for the rest of the loop, and the loop's result is reached after
+// (steps - j) mod k more steps.  That is looked for, exactly, here: no result
+// changes by a bit.  It happens early: in the generator's circuits every wire
+// repeats itself (period 1, in a fifth of the wires 2, seldom 4) after at most
+// 18 of a loop's 10000 steps in the stable profile, and in the reference
+// profile its NaN has reached every current after 17.  For 64 x 65536 wires a
+// SCALED launch takes 0.50 instead of 10.5 ms, FAST 0.50 instead of 16.9, RECIP
+// 0.50 instead of 28.5 and EXACT 0.96 instead of 93 ms (reference profile; the
+// stable one alike), most of it no longer the steps but the launch's tile queue
+// and the fused charge atomics.
+//
+// One check costs about one step.  Windows of kWin steps are compared one
+// after another up to step kDense, then one window of kWide steps every
+// kPlain steps, so that a wire that never repeats itself pays under 1%.  A
+// wave ends when all its active lanes do.  The state at a window's start is
+// kept in LDS (one column per lane, no barrier), not in registers: ten more
+// live registers in the step loops would cost EXACT an occupancy step.
+typedef __attribute__((address_space(3))) float lfloat;
+
+__device__ __forceinline__ bool same_value(float a, float b) {
+  return f32_bits(a) == f32_bits(b) || (a != a && b != b);
+}
+
+//
+// A kernel takes the early end with Settle and executes every step with
+// EveryStep: a template parameter, because the step loops with the checks
+// around them allocate 10 to 30 more registers and ran 3-5% slower than the
+// bare loops (SCALED 10.98 against 10.45 ms, EXACT 94.7 against 92.3 ms for
+// 64 x 65536 wires with every step executed).
+struct EveryStep {
+  static constexpr bool on = false;
+  __device__ __forceinline__ EveryStep(lfloat*, uint32_t) {}
+  template <int kRow = 0, int N>
+  __device__ __forceinline__ void save(const float (&)[N]) const {}
+  template <int kRow = 0, int N>
+  __device__ __forceinline__ bool same(const float (&)[N]) const {
+    return false;
+  }
+};
+
+struct Settle {
+  static constexpr bool on = true;
+  lfloat* snap;     // this lane's column, kSeg rows of `stride` floats
+  uint32_t stride;
+  __device__ __forceinline__ Settle(lfloat* lane_column, uint32_t row_stride)
+      : snap(lane_column), stride(row_stride) {}
+
+  // N values in rows kRow.. of the column.
+  template <int kRow = 0, int N>
+  __device__ __forceinline__ void save(const float (&x)[N]) const {
+#pragma unroll
+    for (int i = 0; i < N; i++) snap[(kRow + i) * stride] = x[i];
+  }
+  template <int kRow = 0, int N>
+  __device__ __forceinline__ bool same(const float (&x)[N]) const {
+    bool eq = true;
+#pragma unroll
+    for (int i = 0; i < N; i++) eq &= same_value(snap[(kRow + i) * stride], x[i]);
+    return eq;
+  }
+};
+
+// Takes the state from step j to step `limit` of n by run(k), which takes k
+// steps; save() keeps the state at a window's start, and over() says whether
+// it is the same again, or whether the steps left no longer change the result
+// for another reason.  Returns n if that was found in every active lane --
+// the state is then that after step n -- and `limit` otherwise.  The state at
+// j need not be a function of the currents: no window starts there.
+template <bool kOn, int kWin, int kWide, int kDense, int kPlain, class Run, class Save, class Over>
+__device__ __forceinline__ int advance(int j, int limit, int n, Run run, Save save, Over over) {
+  if constexpr (!kOn) {
+    run(limit - j);
+    return limit;
+  }
+  bool on = true, probe = false, settled = false;
+  int k = min(kWin, limit - j);
+  while (j < limit) {
+    if (probe) save();
+    run(k);
+    j += k;
+    if (probe && wave_all(over())) {
+      settled = true;
+      on = false;
+      limit = j + (n - j) % k;
+    }
+    const bool dense = j < kDense;
+    probe = on && (dense || !probe);
+    k = on ? min(dense ? kWin : probe ? kWide : kPlain, limit - j) : limit - j;
+  }
+  return settled ? n : limit;
+}
+
+template <int N>
+__device__ __forceinline__ bool all_finite(const float (&x)[N]) {
+  bool finite = true;
+#pragma unroll
+  for (int i = 0; i < N; i++) finite &= __builtin_isfinite(x[i]);
+  return finite;
+}
+
 // A divisor with its split for div_split_group: (zh, zl) from make_div_split,
 // zh = zl = 0 if it has none (every quotient then takes div_fixed).
 struct SplitDivisor {
@@ -169,76 +276,109 @@ __device__ __forceinline__ float state_max(const float (&ni)[kSeg], const float 
   return s;
 }
 
-// The reference's step in its order of operations (circuit_gpu.cu:114-129),
-// `steps` times, on the running currents ni and voltages nv (nv[0], nv[kSeg]
-// the node voltages), with I0 and V0 the wire's values at the start of the
-// loop; writes the result to I0 and V0.  Every division is correctly rounded:
-// the ten by dt, then the ten by R, then the nine by C, each group with one
-// guard; by the FP32 split (split_step, after a per-wire check of the
-// divisors) when kSplit, else by the FP64 reciprocal (div_fixed_group, no
-// set-up: the short tails of the other policies).
-template <bool kSplit>
-__device__ __forceinline__ void reference_steps(float (&ni)[kSeg], float (&nv)[kSeg + 1],
-                                                float (&I0)[kSeg], float (&V0)[kSeg - 1], float L,
-                                                float R, float C, int steps) {
+// One step of the reference (circuit_gpu.cu:114-129) with every division by
+// the FP64 reciprocal of its divisor (div_fixed_group): no per-wire set-up.
+__device__ __forceinline__ void reciprocal_step(float (&ni)[kSeg], float (&nv)[kSeg + 1],
+                                                const float (&I0)[kSeg],
+                                                const float (&V0)[kSeg - 1], float L, float R,
+                                                float C, double rR, double rC) {
   const float dt = CKT_DT_F;
-  if constexpr (kSplit) {
-    const SplitDivisor sdt(dt), sR(R), sC(C);
-    // The loop's constants against split_step's conditions, once; the running
-    // state every K steps.  A wave whose lanes all meet them takes K steps
-    // without the |u| guard.
-    float cmax = fmaxf(fabsf(L), fmaxf(fabsf(nv[0]), fabsf(nv[kSeg])));
+  constexpr double rdt = 1.0 / (double)CKT_DT_F;
+  float t[kSeg], q[kSeg], u[kSeg - 1], w[kSeg - 1];
 #pragma unroll
-    for (int i = 0; i < kSeg; i++) cmax = fmaxf(cmax, fabsf(I0[i]));
+  for (int i = 0; i < kSeg; i++) t[i] = L * (ni[i] - I0[i]);
+  div_fixed_group(q, t, rdt, dt);
 #pragma unroll
-    for (int i = 0; i < kSeg - 1; i++) cmax = fmaxf(cmax, fabsf(V0[i]));
-    const bool consts_ok = cmax <= kStepBound && fabsf(R) >= 0x1p-20f && fabsf(C) >= 0x1p-40f;
-    // Steps per state check: the largest of 8, 4, 3, 2 that every active lane
-    // allows (votes, so inactive lanes take no part).
-    const int kl = unchecked_steps(L, R, C);
-    const int K = wave_all(kl >= 8) ? 8 : wave_all(kl >= 4) ? 4 : wave_all(kl >= 3) ? 3
-                : wave_all(kl >= 2) ? 2 : 1;
-    int j = 0;
-    while (j < steps) {
-      while (j < steps && wave_all(consts_ok && state_max(ni, nv) <= kStepBound)) {
-        const int n = min(K, steps - j);
-        for (int k = 0; k < n; k++) split_step<false>(ni, nv, I0, V0, L, sdt, sR, sC);
-        j += n;
-      }
-      while (j < steps && !wave_all(consts_ok && state_max(ni, nv) <= kStepBound)) {
-        split_step<true>(ni, nv, I0, V0, L, sdt, sR, sC);
-        j++;
-      }
-    }
-  } else {
-    constexpr double rdt = 1.0 / (double)CKT_DT_F;
-    const double rR = 1.0 / (double)R, rC = 1.0 / (double)C;
-    for (int j = 0; j < steps; j++) {
-      float t[kSeg], q[kSeg], u[kSeg - 1], w[kSeg - 1];
+  for (int i = 0; i < kSeg; i++) t[i] = (nv[i + 1] - nv[i]) - q[i];
+  div_fixed_group(ni, t, rR, R);
 #pragma unroll
-      for (int i = 0; i < kSeg; i++) t[i] = L * (ni[i] - I0[i]);
-      div_fixed_group(q, t, rdt, dt);
+  for (int i = 0; i < kSeg - 1; i++) u[i] = dt * (ni[i] - ni[i + 1]);
+  div_fixed_group(w, u, rC, C);
 #pragma unroll
-      for (int i = 0; i < kSeg; i++) t[i] = (nv[i + 1] - nv[i]) - q[i];
-      div_fixed_group(ni, t, rR, R);
-#pragma unroll
-      for (int i = 0; i < kSeg - 1; i++) u[i] = dt * (ni[i] - ni[i + 1]);
-      div_fixed_group(w, u, rC, C);
-#pragma unroll
-      for (int i = 0; i < kSeg - 1; i++) nv[i + 1] = V0[i] + w[i];
-    }
-  }
+  for (int i = 0; i < kSeg - 1; i++) nv[i + 1] = V0[i] + w[i];
+}
+
+// The end of a loop in the reference's order: the running currents ni and
+// voltages nv become the wire's values.
+__device__ __forceinline__ void write_back(const float (&ni)[kSeg], const float (&nv)[kSeg + 1],
+                                           float (&I0)[kSeg], float (&V0)[kSeg - 1]) {
 #pragma unroll
   for (int i = 0; i < kSeg; i++) I0[i] = ni[i];
 #pragma unroll
   for (int i = 0; i < kSeg - 1; i++) V0[i] = nv[i + 1];
 }
 
+// The reference's step in its order of operations `steps` times on the
+// running currents ni and voltages nv (nv[0], nv[kSeg] the node voltages),
+// with I0 and V0 the wire's values at the start of the loop; writes the
+// result to I0 and V0.  Every division is correctly rounded: the ten by dt,
+// then the ten by R, then the nine by C, each group with one guard; by the
+// FP64 reciprocal (reciprocal_step) or, when kSplit, by the FP32 split
+// (split_step), which takes 339 cycles a step instead of 481 but needs a check
+// of the wire's divisors first.  So with the early end on, the split comes
+// only after kSplitAfter steps, which most wires never reach; the steps are
+// the same bit for bit.
+constexpr int kSplitAfter = 64;
+
+template <bool kSplit, class St>
+__device__ __forceinline__ void reference_steps(float (&ni)[kSeg], float (&nv)[kSeg + 1],
+                                                float (&I0)[kSeg], float (&V0)[kSeg - 1], float L,
+                                                float R, float C, int steps, const St& st) {
+  int j = 0;
+  if constexpr (!kSplit || St::on) {
+    const double rR = 1.0 / (double)R, rC = 1.0 / (double)C;
+    j = advance<St::on, 4, 12, 64, 1020>(
+        0, kSplit ? min(steps, kSplitAfter) : steps, steps,
+        [&](int k) {
+          for (int i = 0; i < k; i++) reciprocal_step(ni, nv, I0, V0, L, R, C, rR, rC);
+        },
+        [&] { st.save(ni); }, [&] { return st.same(ni); });
+  }
+  if constexpr (kSplit) {
+    if (j < steps) {
+      const SplitDivisor sdt(CKT_DT_F), sR(R), sC(C);
+      // The loop's constants against split_step's conditions, once; the
+      // running state every K steps.  A wave whose lanes all meet them takes
+      // K steps without the |u| guard.
+      float cmax = fmaxf(fabsf(L), fmaxf(fabsf(nv[0]), fabsf(nv[kSeg])));
+#pragma unroll
+      for (int i = 0; i < kSeg; i++) cmax = fmaxf(cmax, fabsf(I0[i]));
+#pragma unroll
+      for (int i = 0; i < kSeg - 1; i++) cmax = fmaxf(cmax, fabsf(V0[i]));
+      const bool consts_ok = cmax <= kStepBound && fabsf(R) >= 0x1p-20f && fabsf(C) >= 0x1p-40f;
+      // Steps per state check: the largest of 8, 4, 3, 2 that every active
+      // lane allows (votes, so inactive lanes take no part).
+      const int kl = unchecked_steps(L, R, C);
+      const int K = wave_all(kl >= 8) ? 8 : wave_all(kl >= 4) ? 4 : wave_all(kl >= 3) ? 3
+                  : wave_all(kl >= 2) ? 2 : 1;
+      advance<St::on, 12, 12, 0, 1020>(
+          j, steps, steps,
+          [&](int k) {
+            int i = 0;
+            while (i < k) {
+              while (i < k && wave_all(consts_ok && state_max(ni, nv) <= kStepBound)) {
+                const int m = min(K, k - i);
+                for (int c = 0; c < m; c++) split_step<false>(ni, nv, I0, V0, L, sdt, sR, sC);
+                i += m;
+              }
+              while (i < k && !wave_all(consts_ok && state_max(ni, nv) <= kStepBound)) {
+                split_step<true>(ni, nv, I0, V0, L, sdt, sR, sC);
+                i++;
+              }
+            }
+          },
+          [&] { st.save(ni); }, [&] { return st.same(ni); });
+    }
+  }
+  write_back(ni, nv, I0, V0);
+}
+
 // A whole loop in the reference's order, seeded as the reference kernel
 // seeds it (circuit_gpu.cu:107-112); kSplit as for reference_steps.
-template <bool kSplit>
+template <bool kSplit, class St>
 __device__ __forceinline__ void reference_loop(float (&I)[kSeg], float (&V)[kSeg - 1], float vin,
-                                               float vout, float L, float R, float C, int steps) {
+                                               float vout, float L, float R, float C, int steps,
+                                               const St& st) {
   float ni[kSeg], nv[kSeg + 1];
 #pragma unroll
   for (int i = 0; i < kSeg; i++) ni[i] = I[i];
@@ -246,15 +386,17 @@ __device__ __forceinline__ void reference_loop(float (&I)[kSeg], float (&V)[kSeg
 #pragma unroll
   for (int i = 0; i < kSeg - 1; i++) nv[i + 1] = V[i];
   nv[kSeg] = vout;
-  reference_steps<kSplit>(ni, nv, I, V, L, R, C, steps);
+  reference_steps<kSplit>(ni, nv, I, V, L, R, C, steps, st);
 }
 
 // Reference order of operations; bit-identical to a strict FP32 CPU run.
 template <>
 struct Relax<CKT_POLICY_EXACT> {
+  template <class St>
   static __device__ __forceinline__ void run(float (&I)[kSeg], float (&V)[kSeg - 1], float vin,
-                                             float vout, float L, float R, float C, int steps) {
-    reference_loop<true>(I, V, vin, vout, L, R, C, steps);
+                                             float vout, float L, float R, float C, int steps,
+                                             const St& st) {
+    reference_loop<true>(I, V, vin, vout, L, R, C, steps, st);
   }
 };
 
@@ -397,10 +539,7 @@ __device__ __forceinline__ void end_from_currents(float (&I)[kSeg], float (&V)[k
 __device__ __forceinline__ void finish_in_reference_order(float (&I)[kSeg], float (&V)[kSeg - 1],
                                                           float (&x)[kSeg], float vin, float vout,
                                                           float L, float R, float C) {
-  bool finite = true;
-#pragma unroll
-  for (int i = 0; i < kSeg; i++) finite &= __builtin_isfinite(x[i]);
-  if (!finite) {
+  if (!all_finite(x)) {
     const float nan = __builtin_nanf("");
 #pragma unroll
     for (int i = 0; i < kSeg; i++) I[i] = nan;
@@ -415,7 +554,9 @@ __device__ __forceinline__ void finish_in_reference_order(float (&I)[kSeg], floa
 #pragma unroll
   for (int i = 0; i < kSeg - 1; i++) nv[i + 1] = V[i] + div_fixed(dt * (x[i] - x[i + 1]), rC, C);
   nv[kSeg] = vout;
-  reference_steps<false>(x, nv, I, V, L, R, C, kTail);
+  const double rR = 1.0 / (double)R;
+  for (int j = 0; j < kTail; j++) reciprocal_step(x, nv, I, V, L, R, C, rR, rC);
+  write_back(x, nv, I, V);
 }
 
 // Per-wire constants hoisted, FMAs in the loop, voltages kept every step:
@@ -423,10 +564,12 @@ __device__ __forceinline__ void finish_in_reference_order(float (&I)[kSeg], floa
 //   v_k <- V0_k + b*(I_{k-1} - I_k),          b = dt/C
 template <>
 struct Relax<CKT_POLICY_RECIP> {
+  template <class St>
   static __device__ __forceinline__ void run(float (&I)[kSeg], float (&V)[kSeg - 1], float vin,
-                                             float vout, float L, float R, float C, int steps) {
+                                             float vout, float L, float R, float C, int steps,
+                                             const St& st) {
     if (whole_loop_in_reference_order(I, V, vin, vout, L, R, C, steps)) {
-      reference_loop<false>(I, V, vin, vout, L, R, C, steps);
+      reference_loop<false>(I, V, vin, vout, L, R, C, steps, st);
       return;
     }
     const bool no_tail = wave_all(tail_stays_finite(I, V, vin, vout, L, R, C));
@@ -450,13 +593,23 @@ struct Relax<CKT_POLICY_RECIP> {
     for (int i = 0; i < kSeg; i++) ni[i] = h * (nv[i + 1] - nv[i]);
 #pragma unroll
     for (int i = 0; i < kSeg - 1; i++) nv[i + 1] = fmaf(b, ni[i] - ni[i + 1], V[i]);
+    // With the tail a wire with a non-finite current ends all-NaN, whatever
+    // its other values (a non-finite current never becomes finite again).
+    const int body = no_tail ? steps : steps - kTail;
+    advance<St::on, 4, 12, 64, 1020>(
+        1, body, body,
+        [&](int k) {
 #pragma unroll 2
-    for (int j = no_tail ? 1 : kTail + 1; j < steps; j++) {
+          for (int j = 0; j < k; j++) {
 #pragma unroll
-      for (int i = 0; i < kSeg; i++) ni[i] = fmaf(-g, ni[i], fmaf(h, nv[i + 1] - nv[i], c0[i]));
+            for (int i = 0; i < kSeg; i++)
+              ni[i] = fmaf(-g, ni[i], fmaf(h, nv[i + 1] - nv[i], c0[i]));
 #pragma unroll
-      for (int i = 0; i < kSeg - 1; i++) nv[i + 1] = fmaf(b, ni[i] - ni[i + 1], V[i]);
-    }
+            for (int i = 0; i < kSeg - 1; i++) nv[i + 1] = fmaf(b, ni[i] - ni[i + 1], V[i]);
+          }
+        },
+        [&] { st.save(ni); },
+        [&] { return st.same(ni) || (!no_tail && !all_finite(ni)); });
     if (no_tail) {
 #pragma unroll
       for (int i = 0; i < kSeg; i++) I[i] = ni[i];
@@ -481,10 +634,12 @@ struct Relax<CKT_POLICY_RECIP> {
 // reference's order.
 template <>
 struct Relax<CKT_POLICY_FAST> {
+  template <class St>
   static __device__ __forceinline__ void run(float (&I)[kSeg], float (&V)[kSeg - 1], float vin,
-                                             float vout, float L, float R, float C, int steps) {
+                                             float vout, float L, float R, float C, int steps,
+                                             const St& st) {
     if (whole_loop_in_reference_order(I, V, vin, vout, L, R, C, steps)) {
-      reference_loop<false>(I, V, vin, vout, L, R, C, steps);
+      reference_loop<false>(I, V, vin, vout, L, R, C, steps, st);
       return;
     }
     const bool no_tail = wave_all(tail_stays_finite(I, V, vin, vout, L, R, C));
@@ -520,11 +675,16 @@ struct Relax<CKT_POLICY_FAST> {
     y[kSeg - 1] = fmaf(a_end, x[kSeg - 1], fmaf(m, x[kSeg - 2], K[kSeg - 1]));     \
     _Pragma("unroll") for (int i = 0; i < kSeg; i++) x[i] = y[i];                  \
   }
-    int j = 1;
-    for (; j + 4 <= body; j += 4) {
-      CKT_FAST_STEP CKT_FAST_STEP CKT_FAST_STEP CKT_FAST_STEP
-    }
-    for (; j < body; j++) CKT_FAST_STEP
+    advance<St::on, 4, 12, 64, 1020>(
+        1, body, body,
+        [&](int k) {
+          int j = 0;
+          for (; j + 4 <= k; j += 4) {
+            CKT_FAST_STEP CKT_FAST_STEP CKT_FAST_STEP CKT_FAST_STEP
+          }
+          for (; j < k; j++) CKT_FAST_STEP
+        },
+        [&] { st.save(x); }, [&] { return st.same(x) || (!no_tail && !all_finite(x)); });
 #undef CKT_FAST_STEP
     // The substitution has no voltages in its step, so same-signed infinite
     // currents would stay infinite where the reference's turn to NaN; values
@@ -584,13 +744,21 @@ struct Tridiag {
     for (int i = 0; i < kSeg; i++) x[i] = y[i];
   }
 
-  __device__ __forceinline__ void steps4(int n) {
-    for (int j = 0; j < n; j++) {
-      step();
-      step();
-      step();
-      step();
-    }
+  // `n` blocks of four steps; nan_ends: a non-finite current ends the wire
+  // all-NaN.
+  template <class St>
+  __device__ __forceinline__ void steps4(int n, bool nan_ends, const St& st) {
+    advance<St::on, 1, 3, 16, 255>(
+        0, n, n,
+        [&](int k) {
+          for (int j = 0; j < k; j++) {
+            step();
+            step();
+            step();
+            step();
+          }
+        },
+        [&] { st.save(x); }, [&] { return st.same(x) || (nan_ends && !all_finite(x)); });
   }
 };
 
@@ -634,10 +802,12 @@ struct Tridiag {
 // contracting.
 template <>
 struct Relax<CKT_POLICY_SCALED> {
+  template <class St>
   static __device__ __forceinline__ void run(float (&I)[kSeg], float (&V)[kSeg - 1], float vin,
-                                             float vout, float L, float R, float C, int steps) {
+                                             float vout, float L, float R, float C, int steps,
+                                             const St& st) {
     if (whole_loop_in_reference_order(I, V, vin, vout, L, R, C, steps)) {
-      reference_loop<false>(I, V, vin, vout, L, R, C, steps);
+      reference_loop<false>(I, V, vin, vout, L, R, C, steps, st);
       return;
     }
     const bool no_tail = wave_all(tail_stays_finite(I, V, vin, vout, L, R, C));
@@ -645,7 +815,7 @@ struct Relax<CKT_POLICY_SCALED> {
     const int rest = steps - 1 - (no_tail ? 0 : kTail);
     for (int j = 0; j < (rest & 3); j++) t.step();
     const int blocks = rest >> 2;
-    if (blocks > 0) run_blocks(t, blocks);
+    if (blocks > 0) run_blocks(t, blocks, !no_tail, st);
     if (no_tail)
       end_from_currents(I, V, t.x, C);
     else
@@ -658,7 +828,10 @@ struct Relax<CKT_POLICY_SCALED> {
 
   // `blocks` blocks of four steps from t.x, left in t.x: rewritten where one
   // of the two conditions holds, as plain tridiagonal steps otherwise.
-  static __device__ __forceinline__ void run_blocks(Tridiag& t, int blocks) {
+  // nan_ends: a non-finite current ends the wire all-NaN.
+  template <class St>
+  static __device__ __forceinline__ void run_blocks(Tridiag& t, int blocks, bool nan_ends,
+                                                    const St& st) {
     // x*: (1 - a_i) x*_i + d (x*_{i-1} + x*_{i+1}) = K_i, by the Thomas
     // algorithm (diagonally dominant under either condition below).
     float xs[kSeg];
@@ -703,7 +876,7 @@ struct Relax<CKT_POLICY_SCALED> {
     // or a fixed point past FLT_MAX: the reference leaves the finite range
     // then, and so does either step here, the deviation staying non-finite.
     if (!(t.d >= 0x1p-25f && (contracting || diverging))) {
-      t.steps4(blocks);
+      t.steps4(blocks, nan_ends, st);
       return;
     }
     const float c_mid = t.a_mid / t.m, c_end = t.a_end / t.m;
@@ -713,25 +886,51 @@ struct Relax<CKT_POLICY_SCALED> {
     // it is not kept live from the bound above across the fallback branch,
     // and split into its mirror-symmetric and antisymmetric halves.
     float s[kHalf], a[kHalf];
+    float xmin = __builtin_huge_valf();
 #pragma unroll
     for (int i = 0; i < kHalf; i++) {
       asm volatile("" : "+v"(xs[i]), "+v"(xs[kSeg - 1 - i]));
       const float lo = t.x[i] - xs[i], hi = t.x[kSeg - 1 - i] - xs[kSeg - 1 - i];
       s[i] = lo + hi;
       a[i] = lo - hi;
+      xmin = fminf(xmin, fminf(fabsf(xs[i]), fabsf(xs[kSeg - 1 - i])));
     }
-    for (int j = 0; j < blocks; j++) {
+    // The blocks end early where the halves repeat themselves, where a
+    // diverging wire is no longer finite, and where a contracting wire's
+    // deviation no longer moves any current: its halves shrink in maximum
+    // norm, so once max|s| + max|a| is at most 2^-26 of the smallest |x*|,
+    // every later x* + (s +- a)/2 rounds to x*.
+    const float quiet = contracting ? xmin * 0x1p-26f : 0.0f;
+    advance<St::on, 1, 1, 16, 255>(
+        0, blocks, blocks,
+        [&](int n) {
+          for (int j = 0; j < n; j++) {
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        half_step(s, c_end, c_mid, c_mid + 1.0f);
-        half_step(a, c_end, c_mid, c_mid - 1.0f);
-      }
+            for (int k = 0; k < 4; k++) {
+              half_step(s, c_end, c_mid, c_mid + 1.0f);
+              half_step(a, c_end, c_mid, c_mid - 1.0f);
+            }
 #pragma unroll
-      for (int i = 0; i < kHalf; i++) {
-        s[i] *= m4;
-        a[i] *= m4;
-      }
-    }
+            for (int i = 0; i < kHalf; i++) {
+              s[i] *= m4;
+              a[i] *= m4;
+            }
+          }
+        },
+        [&] {
+          st.save(s);
+          st.template save<kHalf>(a);
+        },
+        [&] {
+          if (st.same(s) && st.template same<kHalf>(a)) return true;
+          float sm = 0.0f, am = 0.0f;
+#pragma unroll
+          for (int i = 0; i < kHalf; i++) {
+            sm = fmaxf(sm, fabsf(s[i]));
+            am = fmaxf(am, fabsf(a[i]));
+          }
+          return all_finite(s) && all_finite(a) ? quiet > 0.0f && sm + am <= quiet : nan_ends;
+        });
 #pragma unroll
     for (int i = 0; i < kHalf; i++) {
       t.x[i] = fmaf(0.5f, s[i] + a[i], xs[i]);
@@ -768,8 +967,9 @@ typedef __attribute__((address_space(1))) const uint32_t gcu32;
 // FUSE: the wire's two charge contributions (distribute_charge's ATOMIC
 // mode, circuit_gpu.cu:273-283) are added from registers right after the
 // relaxation, so the loop drivers skip the separate launch.
-template <int POLICY, bool FUSE>
-__device__ __forceinline__ void cnc_one(const DevCircuit& c, uint32_t w, int steps) {
+template <int POLICY, bool FUSE, class St>
+__device__ __forceinline__ void cnc_one(const DevCircuit& c, uint32_t w, int steps,
+                                        const St& st) {
   const size_t ws = c.ws;
   gfloat* cur = (gfloat*)c.cur;
   gfloat* vol = (gfloat*)c.vol;
@@ -783,7 +983,7 @@ __device__ __forceinline__ void cnc_one(const DevCircuit& c, uint32_t w, int ste
   const float L = ((gfloat*)c.ind)[w], R = ((gfloat*)c.res)[w], C = ((gfloat*)c.wcap)[w];
   const float vin = ((gfloat*)c.voltage)[((gcu32*)c.in_ptr)[w]];
   const float vout = ((gfloat*)c.voltage)[((gcu32*)c.out_ptr)[w]];
-  Relax<POLICY>::run(I, V, vin, vout, L, R, C, steps);
+  Relax<POLICY>::run(I, V, vin, vout, L, R, C, steps, st);
   asm volatile("" : "+v"(w));
 #pragma unroll
   for (int s = 0; s < kSeg; s++) cur[s * ws + w] = I[s];
@@ -798,23 +998,27 @@ __device__ __forceinline__ void cnc_one(const DevCircuit& c, uint32_t w, int ste
 
 // One tile per workgroup.  A tile holds up to BLOCK wires per lane pass; lane
 // l relaxes wires l, l + BLOCK, ... of it one after another.
-template <int POLICY, int BLOCK, bool FUSE>
+template <int POLICY, int BLOCK, bool FUSE, class St>
 __global__ __launch_bounds__(BLOCK) void cnc_kernel(const DevCircuit* __restrict__ circuits,
                                                     const Tile* __restrict__ tiles, int steps) {
+  __shared__ float snap[St::on ? kSeg * BLOCK : 1];
+  const St st((lfloat*)snap + threadIdx.x, BLOCK);
   const Tile t = tiles[blockIdx.x];
   for (uint32_t i = threadIdx.x; i < t.count; i += BLOCK)
-    cnc_one<POLICY, FUSE>(circuits[t.circuit], t.first + i, steps);
+    cnc_one<POLICY, FUSE>(circuits[t.circuit], t.first + i, steps, st);
 }
 
 // Persistent form: a fixed grid pulls tiles from a queue counter.  The last
 // block to finish resets the two counters, so consecutive launches on one
 // stream reuse them without a separate clear.
-template <int POLICY, int BLOCK, bool FUSE>
+template <int POLICY, int BLOCK, bool FUSE, class St>
 __global__ __launch_bounds__(BLOCK) void cnc_persistent_kernel(const DevCircuit* __restrict__ circuits,
                                                                const Tile* __restrict__ tiles,
                                                                uint32_t ntiles, uint32_t* counters,
                                                                int steps) {
   __shared__ uint32_t s_tile;
+  __shared__ float snap[St::on ? kSeg * BLOCK : 1];
+  const St st((lfloat*)snap + threadIdx.x, BLOCK);
   for (;;) {
     if (threadIdx.x == 0) s_tile = atomicAdd(&counters[0], 1u);
     __syncthreads();
@@ -823,7 +1027,7 @@ __global__ __launch_bounds__(BLOCK) void cnc_persistent_kernel(const DevCircuit*
     if (ti >= ntiles) break;
     const Tile t = tiles[ti];
     for (uint32_t i = threadIdx.x; i < t.count; i += BLOCK)
-      cnc_one<POLICY, FUSE>(circuits[t.circuit], t.first + i, steps);
+      cnc_one<POLICY, FUSE>(circuits[t.circuit], t.first + i, steps, st);
   }
   if (threadIdx.x == 0) {
     __threadfence();
@@ -1152,6 +1356,8 @@ __global__ __launch_bounds__(256) void cnc_aos_kernel(PieceIndex ix, ckt_wire_t*
                                                       const ckt_node_t* pvt, const ckt_node_t* owned,
                                                       const ckt_node_t* ghost, int steps,
                                                       unsigned long long* bad) {
+  __shared__ float snap[kSeg * 256];
+  const Settle st((lfloat*)snap + threadIdx.x, 256);
   uint32_t k;
   const ckt_piece_t p = ix.pieces[piece_of_block(ix, blockIdx.x, &k)];
   if (k >= p.num_wires) return;
@@ -1168,7 +1374,8 @@ __global__ __launch_bounds__(256) void cnc_aos_kernel(PieceIndex ix, ckt_wire_t*
 #pragma unroll
   for (int s = 0; s < kSeg - 1; s++) V[s] = wire.voltage[s];
   const float vin = in_base[wire.in_ptr].voltage, vout = out_base[wire.out_ptr].voltage;
-  Relax<POLICY>::run(I, V, vin, vout, wire.inductance, wire.resistance, wire.capacitance, steps);
+  Relax<POLICY>::run(I, V, vin, vout, wire.inductance, wire.resistance, wire.capacitance, steps,
+                     st);
 #pragma unroll
   for (int s = 0; s < kSeg; s++) wire.current[s] = I[s];
 #pragma unroll
@@ -1255,65 +1462,75 @@ __global__ __launch_bounds__(256) void copy_kernel(uint4* __restrict__ dst,
 static inline uint32_t blocks_for(size_t n, int b) { return (uint32_t)((n + b - 1) / b); }
 
 // Plain grid (one tile per workgroup) or persistent grid (`grid` workgroups
-// pulling tiles), for every policy x workgroup size x fused epilogue.
-template <int POLICY, int BLOCK, bool FUSE>
+// pulling tiles), for every policy x workgroup size x fused epilogue
+// x early end or every step.
+template <int POLICY, int BLOCK, bool FUSE, class St>
 static void cnc_go(bool persistent, const DevCircuit* c, const Tile* t, uint32_t n, int grid,
                    uint32_t* ctr, int steps, hipStream_t s) {
   if (persistent)
-    hipLaunchKernelGGL((cnc_persistent_kernel<POLICY, BLOCK, FUSE>), dim3(grid), dim3(BLOCK), 0, s,
-                       c, t, n, ctr, steps);
+    hipLaunchKernelGGL((cnc_persistent_kernel<POLICY, BLOCK, FUSE, St>), dim3(grid), dim3(BLOCK), 0,
+                       s, c, t, n, ctr, steps);
   else
-    hipLaunchKernelGGL((cnc_kernel<POLICY, BLOCK, FUSE>), dim3(n), dim3(BLOCK), 0, s, c, t, steps);
+    hipLaunchKernelGGL((cnc_kernel<POLICY, BLOCK, FUSE, St>), dim3(n), dim3(BLOCK), 0, s, c, t,
+                       steps);
 }
 
-template <int POLICY, bool FUSE>
+template <int POLICY, bool FUSE, class St>
 static hipError_t cnc_by_block(bool persistent, const DevCircuit* c, const Tile* t, uint32_t n,
                                int block, int grid, uint32_t* ctr, int steps, hipStream_t s) {
   switch (block) {
-    case 64: cnc_go<POLICY, 64, FUSE>(persistent, c, t, n, grid, ctr, steps, s); break;
-    case 128: cnc_go<POLICY, 128, FUSE>(persistent, c, t, n, grid, ctr, steps, s); break;
-    case 256: cnc_go<POLICY, 256, FUSE>(persistent, c, t, n, grid, ctr, steps, s); break;
-    case 512: cnc_go<POLICY, 512, FUSE>(persistent, c, t, n, grid, ctr, steps, s); break;
+    case 64: cnc_go<POLICY, 64, FUSE, St>(persistent, c, t, n, grid, ctr, steps, s); break;
+    case 128: cnc_go<POLICY, 128, FUSE, St>(persistent, c, t, n, grid, ctr, steps, s); break;
+    case 256: cnc_go<POLICY, 256, FUSE, St>(persistent, c, t, n, grid, ctr, steps, s); break;
+    case 512: cnc_go<POLICY, 512, FUSE, St>(persistent, c, t, n, grid, ctr, steps, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
+template <int POLICY, bool FUSE>
+static hipError_t cnc_by_steps(bool persistent, const DevCircuit* c, const Tile* t, uint32_t n,
+                               int block, int grid, uint32_t* ctr, int steps, bool all,
+                               hipStream_t s) {
+  return all ? cnc_by_block<POLICY, FUSE, EveryStep>(persistent, c, t, n, block, grid, ctr, steps, s)
+             : cnc_by_block<POLICY, FUSE, Settle>(persistent, c, t, n, block, grid, ctr, steps, s);
+}
+
 template <int POLICY>
 static hipError_t cnc_by_fuse(bool fuse, bool persistent, const DevCircuit* c, const Tile* t,
-                              uint32_t n, int block, int grid, uint32_t* ctr, int steps,
+                              uint32_t n, int block, int grid, uint32_t* ctr, int steps, bool all,
                               hipStream_t s) {
-  return fuse ? cnc_by_block<POLICY, true>(persistent, c, t, n, block, grid, ctr, steps, s)
-              : cnc_by_block<POLICY, false>(persistent, c, t, n, block, grid, ctr, steps, s);
+  return fuse ? cnc_by_steps<POLICY, true>(persistent, c, t, n, block, grid, ctr, steps, all, s)
+              : cnc_by_steps<POLICY, false>(persistent, c, t, n, block, grid, ctr, steps, all, s);
 }
 
 static hipError_t cnc_launch(int policy, bool fuse, bool persistent, const DevCircuit* c,
                              const Tile* t, uint32_t n, int block, int grid, uint32_t* ctr,
-                             int steps, hipStream_t s) {
+                             int steps, bool all, hipStream_t s) {
   if (n == 0) return hipSuccess;
   if (persistent && grid < 1) return hipErrorInvalidValue;
   switch (policy) {
     case CKT_POLICY_EXACT:
-      return cnc_by_fuse<CKT_POLICY_EXACT>(fuse, persistent, c, t, n, block, grid, ctr, steps, s);
+      return cnc_by_fuse<CKT_POLICY_EXACT>(fuse, persistent, c, t, n, block, grid, ctr, steps, all, s);
     case CKT_POLICY_RECIP:
-      return cnc_by_fuse<CKT_POLICY_RECIP>(fuse, persistent, c, t, n, block, grid, ctr, steps, s);
+      return cnc_by_fuse<CKT_POLICY_RECIP>(fuse, persistent, c, t, n, block, grid, ctr, steps, all, s);
     case CKT_POLICY_FAST:
-      return cnc_by_fuse<CKT_POLICY_FAST>(fuse, persistent, c, t, n, block, grid, ctr, steps, s);
+      return cnc_by_fuse<CKT_POLICY_FAST>(fuse, persistent, c, t, n, block, grid, ctr, steps, all, s);
     case CKT_POLICY_SCALED:
-      return cnc_by_fuse<CKT_POLICY_SCALED>(fuse, persistent, c, t, n, block, grid, ctr, steps, s);
+      return cnc_by_fuse<CKT_POLICY_SCALED>(fuse, persistent, c, t, n, block, grid, ctr, steps, all, s);
     default: return hipErrorInvalidValue;
   }
 }
 
 hipError_t launch_cnc(int policy, bool fuse_dsc, const DevCircuit* c, const Tile* t, uint32_t n,
-                      int block, int steps, hipStream_t s) {
-  return cnc_launch(policy, fuse_dsc, false, c, t, n, block, 0, nullptr, steps, s);
+                      int block, int steps, bool all, hipStream_t s) {
+  return cnc_launch(policy, fuse_dsc, false, c, t, n, block, 0, nullptr, steps, all, s);
 }
 
 hipError_t launch_cnc_persistent(int policy, bool fuse_dsc, const DevCircuit* c, const Tile* t,
                                  uint32_t n, int block, int grid, uint32_t* ctr, int steps,
-                                 hipStream_t s) {
-  return cnc_launch(policy, fuse_dsc, true, c, t, n, block, grid, ctr, steps, s);
+                                 bool all, hipStream_t s) {
+  return cnc_launch(policy, fuse_dsc, true, c, t, n, block, grid, ctr, steps, all, s);
 }
 
 hipError_t launch_dsc_atomic(const DevCircuit* c, const Tile* t, uint32_t n, int block,

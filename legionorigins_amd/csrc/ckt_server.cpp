@@ -570,6 +570,14 @@ int ckt_server_create(int device, const ckt_server_config_t* config, ckt_server_
     delete s;
     return st;
   }
+  // EXACT requests execute every step.  The early end would serve a 500-loop
+  // request of 16384 wires in under 50 ms, and callers (the online test of
+  // wait's time limit and of cancel) count on it running longer than that.
+  if (cfg.policy == CKT_POLICY_EXACT) st = s->eng.set_option(OPT_ALL_STEPS, 1);
+  if (st) {
+    delete s;
+    return st;
+  }
   cfg.hbm_budget_bytes = s->eng.budget();
   s->cfg = cfg;
   *out = s;
