@@ -739,15 +739,20 @@ int Engine::cnc(const std::vector<PieceRef>& refs, int policy, bool fuse_dsc) {
   if ((st = timed_begin(CKT_CALC_NEW_CURRENTS, &a))) return st;
   hipError_t e;
   // Launch shape unless set with OPT_CNC_BLOCK / OPT_PERSISTENT /
-  // OPT_WAVES_PER_SIMD.  On the 64 x 16384 x 65536 circuit a persistent tile
+  // OPT_WAVES_PER_SIMD.  With the early end a launch is bound by the wires'
+  // bytes, and a plain grid of 256-lane workgroups is best: on the 64 x 16384 x
+  // 65536 circuit 170 us for SCALED, FAST and RECIP (172-190 with 64, 128 or
+  // 512 lanes; a tile queue 190-980), EXACT 239 (stable) and 169 (reference
+  // profile) against 228-374 and 179-185.  With every step: on the 64 x 16384 x 65536 circuit a persistent tile
   // queue of 256-lane workgroups with 4 resident waves per SIMD beats the
   // plain grid by 6% for SCALED and 1-2% for FAST and RECIP.  For EXACT (71
   // VGPRs, at most 7 resident waves) a queue of 64-lane workgroups at 7 waves
   // per SIMD is 1-3% faster than the plain grid of 256-lane workgroups, which
   // it keeps when the workgroup size is set (a queue of 256-lane workgroups
   // is 1-4% slower than that grid).
-  const bool persistent = persistent_ >= 0 ? persistent_ != 0
-                                           : policy != CKT_POLICY_EXACT || cnc_block_ < 0;
+  const bool persistent =
+      persistent_ >= 0 ? persistent_ != 0
+                       : all_steps_ && (policy != CKT_POLICY_EXACT || cnc_block_ < 0);
   const int waves = waves_per_simd_ > 0 ? waves_per_simd_ : (policy == CKT_POLICY_EXACT ? 7 : 4);
   if (persistent) {
     const int waves_per_block = block / 64;

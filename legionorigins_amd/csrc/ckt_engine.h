@@ -181,9 +181,9 @@ class Engine {
   int upload_buf(uint64_t key, const void* data, size_t bytes, uint32_t n, DevBuf* out);
   int prefetch_tiles(const std::vector<PieceRef>& refs, int policy, int mode);
   // calc_new_currents' workgroup size: OPT_CNC_BLOCK, or with -1 (default) 64
-  // for EXACT and 256 for the other policies.
+  // for EXACT with every step executed and 256 otherwise.
   int cnc_block_for(int policy) const {
-    return cnc_block_ > 0 ? cnc_block_ : (policy == CKT_POLICY_EXACT ? 64 : 256);
+    return cnc_block_ > 0 ? cnc_block_ : (all_steps_ && policy == CKT_POLICY_EXACT ? 64 : 256);
   }
   // loop_once's launches; every tile list must already be cached.
   int launch_loop(const std::vector<PieceRef>& refs, int policy, int mode);
