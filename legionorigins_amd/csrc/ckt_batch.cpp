@@ -259,10 +259,8 @@ int ckt_batch_add(ckt_batch_t* b, const ckt_node_t* nodes, uint32_t num_nodes,
   int st = check(b);
   if (st) return st;
   if (num_loops < 0) return fail(CKT_ERR_INVALID_ARG, "negative loop count");
-  SlabImage img;
-  if ((st = image_from_aos(img, nodes, num_nodes, wires, num_wires, locator, pieces, num_pieces)))
-    return st;
-  return b->eng.add(img, num_loops, id);
+  return b->eng.add_records(nodes, num_nodes, wires, num_wires, locator, pieces, num_pieces,
+                            num_loops, nullptr, id);
 }
 
 int ckt_batch_remove(ckt_batch_t* b, uint32_t id) {

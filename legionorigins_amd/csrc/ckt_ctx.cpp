@@ -113,10 +113,12 @@ int ckt_ctx_load(ckt_ctx_t* ctx, const ckt_node_t* nodes, uint32_t num_nodes,
                  const ckt_piece_t* pieces, uint32_t num_pieces) {
   CtxLock lk(ctx);
   if (!ctx) return fail(CKT_ERR_INVALID_ARG, "null context");
-  SlabImage img;
-  int st = image_from_aos(img, nodes, num_nodes, wires, num_wires, locator, pieces, num_pieces);
-  if (st) return st;
-  return install(ctx, img);
+  const bool had = ctx->loaded;
+  const uint32_t old = ctx->id;
+  const int st = ctx->eng.add_records(nodes, num_nodes, wires, num_wires, locator, pieces,
+                                      num_pieces, 0, had ? &old : nullptr, &ctx->id);
+  ctx->loaded = ctx->eng.find(ctx->id) != nullptr;
+  return st;
 }
 
 int ckt_ctx_generate(ckt_ctx_t* ctx, const ckt_gen_params_t* params) {

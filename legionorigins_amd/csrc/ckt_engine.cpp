@@ -1,6 +1,7 @@
 // ckt_engine.cpp -- device-resident circuits, tile lists and task launches.
 #include "ckt_engine.h"
 #include "ckt_index.h"
+#include "ckt_records.h"
 
 #include <algorithm>
 #include <cstring>
@@ -293,6 +294,154 @@ int Engine::add(SlabImage& img, int32_t loops, uint32_t* id) {
   return CKT_OK;
 }
 
+// Scratch of a load: what it found wrong, the piece table's workgroup numbers
+// (PieceIndex::first_block, over wires) and the index build's scratch.
+namespace {
+struct RecordScratch {
+  size_t first_block, index, bytes;
+  RecordScratch(uint32_t N, uint32_t W, uint32_t P)
+      : first_block(align_up(sizeof(LoadFaults), 256)),
+        index(align_up(first_block + 4 * ((size_t)P + 1), 256)),
+        bytes(index + index_scratch_bytes(N, W)) {}
+};
+// Scratch up to this size is kept with the engine for the next build.
+constexpr size_t kKeepScratch = 64u << 20;
+}  // namespace
+
+int Engine::build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, const int32_t* locator,
+                          const ckt_piece_t* pieces, const DevCircuit& c, void* scratch) {
+  const uint32_t N = c.num_nodes, W = c.num_wires, P = c.num_pieces;
+  const RecordScratch at(N, W, P);
+  LoadFaults* faults = (LoadFaults*)scratch;
+  uint32_t* d_blocks = (uint32_t*)((uint8_t*)scratch + at.first_block);
+  CKT_HIP(launch_fill_u32((uint32_t*)faults, 0xffffffffu, sizeof(LoadFaults) / 4, stream_));
+  int st;
+  if ((st = ring_.in(wires, sizeof(ckt_wire_t), W, device_, stream_,
+                     [&](void* slot, uint32_t first, uint32_t n) {
+                       return launch_unpack_wires((const ckt_wire_t*)slot, first, n, c, faults,
+                                                  stream_);
+                     })) ||
+      (st = ring_.in(nodes, sizeof(ckt_node_t), N, device_, stream_,
+                     [&](void* slot, uint32_t first, uint32_t n) {
+                       return launch_unpack_nodes((const ckt_node_t*)slot, first, n, c, stream_);
+                     })))
+    return st;
+  if (locator) {
+    if ((st = ring_.in(locator, sizeof(int32_t), N, device_, stream_,
+                       [&](void* slot, uint32_t first, uint32_t n) {
+                         return launch_unpack_locator((const int32_t*)slot, first, n, c, stream_);
+                       })))
+      return st;
+  } else {
+    CKT_HIP(launch_derive_locator(c, stream_));
+  }
+  // Pieces up to the first one that exceeds the circuit are checked for
+  // private nodes of other pieces that their wires reach.
+  std::vector<uint32_t> blocks(1, 0u);
+  uint32_t good = 0;
+  uint64_t total = 0;
+  while (good < P && (uint64_t)pieces[good].first_wire + pieces[good].num_wires <= W &&
+         (uint64_t)pieces[good].first_node + pieces[good].num_nodes <= N &&
+         total + ((uint64_t)pieces[good].num_wires + 255) / 256 <= 0x7fffffffu) {
+    total += ((uint64_t)pieces[good].num_wires + 255) / 256;
+    blocks.push_back((uint32_t)total);
+    good++;
+  }
+  const bool fits = good == P || (uint64_t)pieces[good].first_wire + pieces[good].num_wires > W ||
+                    (uint64_t)pieces[good].first_node + pieces[good].num_nodes > N;
+  if (!fits) return CKT_ERR_UNSUPPORTED;  // overlapping pieces past the grid's limit
+  if ((st = ring_.in(pieces, sizeof(ckt_piece_t), P, device_, stream_,
+                     [&](void* slot, uint32_t first, uint32_t n) {
+                       return launch_copy_words((uint32_t*)(c.pieces + first), (uint32_t*)slot,
+                                                4 * n, stream_);
+                     })) ||
+      (st = ring_.in(blocks.data(), sizeof(uint32_t), good + 1, device_, stream_,
+                     [&](void* slot, uint32_t first, uint32_t n) {
+                       return launch_copy_words(d_blocks + first, (uint32_t*)slot, n, stream_);
+                     })))
+    return st;
+  const PieceIndex ix{c.pieces, d_blocks, good};
+  CKT_HIP(launch_check_pieces(ix, (uint32_t)total, c, faults, stream_));
+  if ((st = index_enqueue(c, (uint8_t*)scratch + at.index, stream_))) return st;
+  LoadFaults f;
+  if ((st = ring_.out(&f, sizeof(f), 1, device_, stream_, [&](void* slot, uint32_t, uint32_t) {
+         return launch_copy_words((uint32_t*)slot, (const uint32_t*)faults, sizeof(f) / 4, stream_);
+       })))
+    return st;
+  // In the order in which a pass over wires, then pieces, meets them.
+  if (~f.location)
+    return fail(CKT_ERR_INVALID_ARG,
+                "wire " + std::to_string(f.location) + " has an invalid PointerLocation");
+  if (~f.pointer)
+    return fail(CKT_ERR_OUT_OF_RANGE,
+                "wire " + std::to_string(f.pointer) + " points past the last node");
+  if (~f.foreign)
+    return fail(CKT_ERR_INVALID_ARG, "wire " + std::to_string((uint32_t)f.foreign) + " of piece " +
+                                         std::to_string(f.foreign >> 32) +
+                                         " reaches a private node of another piece");
+  if (good < P)
+    return fail(CKT_ERR_OUT_OF_RANGE, "piece " + std::to_string(good) + " exceeds the circuit");
+  return CKT_OK;
+}
+
+int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* wires, uint32_t W,
+                        const int32_t* locator, const ckt_piece_t* pieces, uint32_t P,
+                        int32_t loops, const uint32_t* replaced, uint32_t* id) {
+  if ((N && !nodes) || (W && !wires) || (P && !pieces))
+    return fail(CKT_ERR_INVALID_ARG, "load: null array");
+  if (N == 0 || P == 0) return fail(CKT_ERR_INVALID_ARG, "load: need at least one node and one piece");
+  if (N >= kMaxElements || W >= kMaxElements)
+    return fail(CKT_ERR_OUT_OF_RANGE, "load: more than 2^30 nodes or wires");
+  CKT_HIP(hipSetDevice(device_));
+  int st;
+  const SlabLayout lay = SlabLayout::make(N, W, P);
+  const Circuit* old = replaced ? find(*replaced) : nullptr;
+  const uint64_t in_use = in_use_ - (old ? old->lay.total : 0);
+  // The device path holds the new circuit and its scratch beside the replaced
+  // one.  Where that does not fit, the records are unpacked and checked on the
+  // host and the replaced circuit leaves first.
+  void *slab = nullptr, *own = nullptr;
+  const size_t need = RecordScratch(N, W, P).bytes;
+  bool fits = !budget_ || in_use + lay.total <= budget_;
+  if (fits && need > devgen_scratch_cap_ && need <= kKeepScratch) {
+    // Builds already enqueued use the old scratch.
+    CKT_HIP(hipStreamSynchronize(stream_));
+    if (devgen_scratch_) CKT_HIP(hipFree(devgen_scratch_));
+    devgen_scratch_ = nullptr;
+    devgen_scratch_cap_ = 0;
+    fits = hipMalloc(&devgen_scratch_, need) == hipSuccess;
+    if (fits) devgen_scratch_cap_ = need;
+    else devgen_scratch_ = nullptr;
+  } else if (fits && need > devgen_scratch_cap_) {
+    fits = hipMalloc(&own, need) == hipSuccess;
+  }
+  fits = fits && hipMalloc(&slab, lay.total) == hipSuccess;
+  (void)hipGetLastError();
+  if (fits) {
+    st = build_records(nodes, wires, locator, pieces, device_view(slab, lay, N, W, P),
+                       own ? own : devgen_scratch_);
+    const hipError_t e = hipStreamSynchronize(stream_);
+    if (!st && e != hipSuccess) st = hip_fail(e, "load");
+    if (own) (void)hipFree(own);
+    if (st) (void)hipFree(slab);
+    if (st && st != CKT_ERR_UNSUPPORTED) return st;
+    if (!st && replaced && (st = remove(*replaced))) {
+      (void)hipFree(slab);
+      return st;
+    }
+    if (!st) {
+      attach(slab, lay, N, W, P, std::vector<ckt_piece_t>(pieces, pieces + P), loops, id);
+      return CKT_OK;
+    }
+  } else if (own) {
+    (void)hipFree(own);
+  }
+  SlabImage img;
+  if ((st = image_from_aos(img, nodes, N, wires, W, locator, pieces, P))) return st;
+  if (replaced && (st = remove(*replaced))) return st;
+  return add(img, loops, id);
+}
+
 int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loops, uint32_t* id) {
   uint32_t N, W, P;
   int st = gen_validate(params, &N, &W, &P);
@@ -315,21 +464,10 @@ int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loop
   return CKT_OK;
 }
 
-void Engine::attach(void* slab, const SlabLayout& L, uint32_t N, uint32_t W, uint32_t P,
-                    const std::vector<ckt_piece_t>& pieces, int32_t loops, uint32_t* id,
-                    bool stream_ordered) {
-  Circuit* c = new Circuit();
-  c->stream_ordered = stream_ordered;
-  c->id = next_id_++;
-  c->num_nodes = N;
-  c->num_wires = W;
-  c->num_pieces = P;
-  c->lay = L;
-  c->slab = slab;
-  c->pieces = pieces;
-  c->loops_left = loops;
+DevCircuit Engine::device_view(void* slab, const SlabLayout& L, uint32_t N, uint32_t W,
+                               uint32_t P) {
   uint8_t* b = (uint8_t*)slab;
-  DevCircuit& d = c->dev;
+  DevCircuit d{};
   d.cur = (float*)(b + L.cur);
   d.vol = (float*)(b + L.vol);
   d.ind = (float*)(b + L.ind);
@@ -351,6 +489,23 @@ void Engine::attach(void* slab, const SlabLayout& L, uint32_t N, uint32_t W, uin
   d.ws = L.ws;
   d.num_nodes = N;
   d.num_pieces = P;
+  return d;
+}
+
+void Engine::attach(void* slab, const SlabLayout& L, uint32_t N, uint32_t W, uint32_t P,
+                    const std::vector<ckt_piece_t>& pieces, int32_t loops, uint32_t* id,
+                    bool stream_ordered) {
+  Circuit* c = new Circuit();
+  c->stream_ordered = stream_ordered;
+  c->id = next_id_++;
+  c->num_nodes = N;
+  c->num_wires = W;
+  c->num_pieces = P;
+  c->lay = L;
+  c->slab = slab;
+  c->pieces = pieces;
+  c->loops_left = loops;
+  c->dev = device_view(slab, L, N, W, P);
   for (uint32_t k = 0; k < P; k++) c->piece_index.emplace(piece_key(pieces[k]), k);
   // Wires partitioned by the pieces -> the CSR modes apply; node ranges
   // disjoint -> the LDS-privatised reduction applies.
@@ -458,43 +613,26 @@ void Engine::all_refs(std::vector<PieceRef>& refs, bool only_active) const {
   }
 }
 
+// The records are put together on the device and written straight into
+// pinned slots; waits for the stream, behind which the kernels are queued.
 int Engine::store(uint32_t id, ckt_node_t* nodes, ckt_wire_t* wires) {
   Circuit* c = find(id);
   if (!c) return fail(CKT_ERR_NOT_FOUND, "no circuit with id " + std::to_string(id));
   CKT_HIP(hipSetDevice(device_));
+  int st;
+  if (wires &&
+      (st = ring_.out(wires, sizeof(ckt_wire_t), c->num_wires, device_, stream_,
+                      [&](void* slot, uint32_t first, uint32_t n) {
+                        return launch_pack_wires((ckt_wire_t*)slot, first, n, c->dev, stream_);
+                      })))
+    return st;
+  if (nodes &&
+      (st = ring_.out(nodes, sizeof(ckt_node_t), c->num_nodes, device_, stream_,
+                      [&](void* slot, uint32_t first, uint32_t n) {
+                        return launch_pack_nodes((ckt_node_t*)slot, first, n, c->dev, stream_);
+                      })))
+    return st;
   CKT_HIP(hipStreamSynchronize(stream_));
-  const SlabLayout& L = c->lay;
-  std::vector<uint8_t> img(L.total);
-  CKT_HIP(hipMemcpy(img.data(), c->slab, L.total, hipMemcpyDeviceToHost));
-  auto at = [&](size_t off) { return img.data() + off; };
-  const size_t ws = L.ws;
-  if (wires) {
-    const float* cur = (const float*)at(L.cur);
-    const float* vol = (const float*)at(L.vol);
-    const float *ind = (const float*)at(L.ind), *res = (const float*)at(L.res),
-                *wcap = (const float*)at(L.wcap);
-    const uint32_t *in_ptr = (const uint32_t*)at(L.in_ptr), *out_ptr = (const uint32_t*)at(L.out_ptr);
-    const uint8_t *in_loc = at(L.in_loc), *out_loc = at(L.out_loc);
-    for (uint32_t w = 0; w < c->num_wires; w++) {
-      ckt_wire_t& x = wires[w];
-      std::memset(&x, 0, sizeof(x));
-      x.in_ptr = in_ptr[w];
-      x.out_ptr = out_ptr[w];
-      x.in_loc = in_loc[w];
-      x.out_loc = out_loc[w];
-      x.inductance = ind[w];
-      x.resistance = res[w];
-      x.capacitance = wcap[w];
-      for (int s = 0; s < kSeg; s++) x.current[s] = cur[s * ws + w];
-      for (int s = 0; s < kSeg - 1; s++) x.voltage[s] = vol[s * ws + w];
-    }
-  }
-  if (nodes) {
-    const float *charge = (const float*)at(L.charge), *voltage = (const float*)at(L.voltage),
-                *ncap = (const float*)at(L.ncap), *leak = (const float*)at(L.leak);
-    for (uint32_t i = 0; i < c->num_nodes; i++)
-      nodes[i] = ckt_node_t{charge[i], voltage[i], ncap[i], leak[i]};
-  }
   return CKT_OK;
 }
 
@@ -502,18 +640,22 @@ int Engine::store_topology(uint32_t id, int32_t* locator, uint32_t* csr_row, uin
   Circuit* c = find(id);
   if (!c) return fail(CKT_ERR_NOT_FOUND, "no circuit with id " + std::to_string(id));
   CKT_HIP(hipSetDevice(device_));
+  int st;
+  auto words = [&](uint32_t* dst, const uint32_t* src, uint32_t count) {
+    return ring_.out(dst, sizeof(uint32_t), count, device_, stream_,
+                     [&](void* slot, uint32_t first, uint32_t n) {
+                       return launch_copy_words((uint32_t*)slot, src + first, n, stream_);
+                     });
+  };
+  if (locator &&
+      (st = ring_.out(locator, sizeof(int32_t), c->num_nodes, device_, stream_,
+                      [&](void* slot, uint32_t first, uint32_t n) {
+                        return launch_pack_locator((int32_t*)slot, first, n, c->dev, stream_);
+                      })))
+    return st;
+  if (csr_row && (st = words(csr_row, c->dev.csr_row, c->num_nodes + 1))) return st;
+  if (csr_ent && (st = words(csr_ent, c->dev.csr_ent, 2 * c->num_wires))) return st;
   CKT_HIP(hipStreamSynchronize(stream_));
-  const uint8_t* b = (const uint8_t*)c->slab;
-  const SlabLayout& L = c->lay;
-  if (locator) {
-    std::vector<uint8_t> loc(c->num_nodes);
-    CKT_HIP(hipMemcpy(loc.data(), b + L.locator, c->num_nodes, hipMemcpyDeviceToHost));
-    for (uint32_t i = 0; i < c->num_nodes; i++) locator[i] = loc[i];
-  }
-  if (csr_row)
-    CKT_HIP(hipMemcpy(csr_row, b + L.csr_row, ((size_t)c->num_nodes + 1) * 4, hipMemcpyDeviceToHost));
-  if (csr_ent && c->num_wires)
-    CKT_HIP(hipMemcpy(csr_ent, b + L.csr_ent, (size_t)c->num_wires * 8, hipMemcpyDeviceToHost));
   return CKT_OK;
 }
 

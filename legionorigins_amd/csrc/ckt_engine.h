@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "ckt_gen.h"
+#include "ckt_hostring.h"
 #include "ckt_internal.h"
 
 namespace ckt {
@@ -113,6 +114,12 @@ class Engine {
 
   // Circuits.
   int add(SlabImage& img, int32_t loops, uint32_t* id);
+  // A circuit from reference-layout records (ckt_ctx_load): streamed to the
+  // device, unpacked, checked and indexed there.  `replaced`, if not NULL, is
+  // the id of a circuit to remove once the new one is known to be valid.
+  int add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* wires, uint32_t W,
+                  const int32_t* locator, const ckt_piece_t* pieces, uint32_t P, int32_t loops,
+                  const uint32_t* replaced, uint32_t* id);
   // Generates the circuit on the device (no host image, no upload).
   int add_generated_on_device(const ckt_gen_params_t* params, int32_t loops, uint32_t* id);
   // Same circuit from a plan made earlier: the generation is only enqueued
@@ -176,6 +183,11 @@ class Engine {
   void attach(void* slab, const SlabLayout& L, uint32_t N, uint32_t W, uint32_t P,
               const std::vector<ckt_piece_t>& pieces, int32_t loops, uint32_t* id,
               bool stream_ordered = false);
+  static DevCircuit device_view(void* slab, const SlabLayout& L, uint32_t N, uint32_t W,
+                                uint32_t P);
+  // add_records' build into `slab`; `scratch` as record_scratch_bytes says.
+  int build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, const int32_t* locator,
+                    const ckt_piece_t* pieces, const DevCircuit& c, void* scratch);
   int ensure_table();
   int tiles_for(int kind, const std::vector<PieceRef>& refs, int block, DevBuf* out);
   int upload_buf(uint64_t key, const void* data, size_t bytes, uint32_t n, DevBuf* out);
@@ -246,6 +258,7 @@ class Engine {
   };
   std::vector<PinnedChunk> staging_;
   size_t staging_chunk_ = 0, staging_off_ = 0;
+  HostRing ring_;  // records between host memory and the device
   double acc_ms_[CKT_NUM_TASK_IDS] = {0};
   uint64_t acc_n_[CKT_NUM_TASK_IDS] = {0};
 };

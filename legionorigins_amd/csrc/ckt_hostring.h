@@ -1,0 +1,162 @@
+// ckt_hostring.h -- pinned slots through which records stream between the
+// caller's (pageable) memory and kernels that read or write them over PCIe.
+#pragma once
+
+#include <hip/hip_runtime_api.h>
+
+#include <algorithm>
+#include <cstring>
+#include <string>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+#include "ckt_internal.h"
+
+namespace ckt {
+
+// While a kernel reads or writes one slot over the bus, host threads copy
+// others: one core copies about 10 GB/s to or from pageable memory, the bus
+// carries about 50.  One transfer at a time (the caller's lock).  Slots are
+// allocated as large as they are first needed and kept, 32 MiB at most.
+class HostRing {
+ public:
+  HostRing() = default;
+  HostRing(const HostRing&) = delete;
+  HostRing& operator=(const HostRing&) = delete;
+  ~HostRing() {
+    for (Slot& sl : slots_) {
+      if (sl.busy) (void)hipEventSynchronize(sl.ev);
+      if (sl.p) (void)hipHostFree(sl.p);
+      if (sl.ev) (void)hipEventDestroy(sl.ev);
+    }
+  }
+
+  // Copies `count` records of `size` bytes from `src` into slots and calls
+  // launch(slot, first, n), which enqueues on `s` the kernel that reads them.
+  // Returns once every launch is made (`src` is free then); a slot's kernel is
+  // waited for where the slot is used again.
+  template <class Launch>
+  int in(const void* src, size_t size, uint32_t count, int device, hipStream_t s, Launch launch) {
+    const Plan p(size, count);
+    return team(p.workers, device, [&](int t) -> int {
+      int side = 0;
+      for (uint32_t c = (uint32_t)t; c < p.chunks; c += (uint32_t)p.workers, side ^= 1) {
+        const uint32_t first = c * p.per, n = std::min(p.per, count - first);
+        Slot& sl = slots_[2 * t + side];
+        if (int st = acquire(sl, n * size)) return st;
+        std::memcpy(sl.p, (const char*)src + (size_t)first * size, n * size);
+        if (hipError_t e = launch(sl.p, first, n)) return hip_fail(e, "reading records");
+        if (int st = mark(sl, s)) return st;
+      }
+      return CKT_OK;
+    });
+  }
+
+  // Calls launch(slot, first, n) for the kernels that write records into
+  // slots on `s`, and copies each slot to `dst` when its kernel has run.
+  // Returns when all records are there.
+  template <class Launch>
+  int out(void* dst, size_t size, uint32_t count, int device, hipStream_t s, Launch launch) {
+    const Plan p(size, count);
+    return team(p.workers, device, [&](int t) -> int {
+      auto begin = [&](uint32_t c, int side) -> int {
+        if (c >= p.chunks) return CKT_OK;
+        const uint32_t first = c * p.per, n = std::min(p.per, count - first);
+        Slot& sl = slots_[2 * t + side];
+        if (int st = acquire(sl, n * size)) return st;
+        if (hipError_t e = launch(sl.p, first, n)) return hip_fail(e, "writing records");
+        return mark(sl, s);
+      };
+      int side = 0;
+      int st = begin((uint32_t)t, side);
+      for (uint32_t c = (uint32_t)t; !st && c < p.chunks; c += (uint32_t)p.workers, side ^= 1) {
+        if ((st = begin(c + (uint32_t)p.workers, side ^ 1))) break;
+        Slot& sl = slots_[2 * t + side];
+        if ((st = wait(sl))) break;
+        const uint32_t first = c * p.per, n = std::min(p.per, count - first);
+        std::memcpy((char*)dst + (size_t)first * size, sl.p, n * size);
+      }
+      return st;
+    });
+  }
+
+ private:
+  static constexpr int kWorkers = 8;
+  static constexpr size_t kSlotBytes = 2u << 20;
+  struct Slot {
+    void* p = nullptr;
+    size_t cap = 0;
+    hipEvent_t ev = nullptr;
+    bool busy = false;  // ev is recorded and not yet waited for
+  };
+  Slot slots_[2 * kWorkers];
+
+  // A transfer's chunks (whole records, a multiple of four) and workers.
+  struct Plan {
+    uint32_t per, chunks;
+    int workers;
+    Plan(size_t size, uint32_t count)
+        : per((uint32_t)(kSlotBytes / size) & ~3u),
+          chunks((uint32_t)(((uint64_t)count + per - 1) / per)),
+          workers((int)std::min<uint32_t>(chunks, kWorkers)) {}
+  };
+
+  static int wait(Slot& sl) {
+    if (!sl.busy) return CKT_OK;
+    CKT_HIP(hipEventSynchronize(sl.ev));
+    sl.busy = false;
+    return CKT_OK;
+  }
+  // The slot, free and of at least `bytes`.
+  static int acquire(Slot& sl, size_t bytes) {
+    if (int st = wait(sl)) return st;
+    if (!sl.ev) CKT_HIP(hipEventCreateWithFlags(&sl.ev, hipEventDisableTiming));
+    if (bytes > sl.cap) {
+      if (sl.p) CKT_HIP(hipHostFree(sl.p));
+      sl.p = nullptr;
+      sl.cap = 0;
+      const size_t cap = std::min(kSlotBytes, std::max<size_t>(2 * bytes, 64u << 10));
+      CKT_HIP(hipHostMalloc(&sl.p, cap, hipHostMallocDefault));
+      sl.cap = cap;
+    }
+    return CKT_OK;
+  }
+  static int mark(Slot& sl, hipStream_t s) {
+    CKT_HIP(hipEventRecord(sl.ev, s));
+    sl.busy = true;
+    return CKT_OK;
+  }
+
+  // work(t) for t in [0, workers): the first on this thread, the others on
+  // threads of their own (or here too where none can be started).  Returns the
+  // first failure, with its message as this thread's.
+  template <class Work>
+  static int team(int workers, int device, Work work) {
+    if (workers <= 0) return CKT_OK;
+    int rc[kWorkers] = {0};
+    std::string err[kWorkers];
+    std::thread th[kWorkers];
+    auto one = [&](int t) {
+      const hipError_t e = hipSetDevice(device);
+      rc[t] = e != hipSuccess ? hip_fail(e, "hipSetDevice") : work(t);
+      if (rc[t]) err[t] = ckt_last_error();
+    };
+    for (int t = 1; t < workers; t++) {
+      try {
+        th[t] = std::thread(one, t);
+      } catch (const std::system_error&) {
+      }
+    }
+    one(0);
+    for (int t = 1; t < workers; t++) {
+      if (th[t].joinable()) th[t].join();
+      else one(t);
+    }
+    for (int t = 0; t < workers; t++)
+      if (rc[t]) return fail(rc[t], err[t]);
+    return CKT_OK;
+  }
+};
+
+}  // namespace ckt
