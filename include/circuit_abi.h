@@ -343,9 +343,13 @@ enum {
   CKT_OPT_WAVES_PER_SIMD = 3,    /* persistent grid: waves resident per SIMD (1..8);
                                     -1 (default): 7 for EXACT, 4 otherwise */
   CKT_OPT_DSC_ATOMIC_IMPL = 4,   /* ATOMIC reduction: 0 auto, 1 global atomics, 2 LDS */
-  CKT_OPT_FUSE_DSC = 5,          /* 1 (default): in ckt_run_loops (sync 0, per_piece 0),
-                                    batches and servers, the ATOMIC distribute_charge is
-                                    done by calc_new_currents' epilogue from registers */
+  CKT_OPT_FUSE_DSC = 5,          /* the ATOMIC distribute_charge in ckt_run_loops (sync 0,
+                                    per_piece 0), batches and servers: 1: done by
+                                    calc_new_currents' epilogue from registers; 0: a launch of
+                                    its own; -1 (default): the fastest form, for whole circuits
+                                    a sum over the node->wire index in one launch with
+                                    update_voltages (whose time kernel_time reports under
+                                    distribute_charge, as for the CSR modes in those loops) */
   /* calc_new_currents' tile schedule (results do not depend on it): */
   CKT_OPT_WIRES_PER_LANE = 6,    /* a tile holds workgroup size x this (1 default, 2, 4)
                                     wires; each lane relaxes that many one after another */

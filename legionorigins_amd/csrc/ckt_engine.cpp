@@ -525,14 +525,16 @@ void Engine::attach(void* slab, const SlabLayout& L, uint32_t N, uint32_t W, uin
     std::sort(ps.begin(), ps.end(), [](const ckt_piece_t& a, const ckt_piece_t& x) {
       return a.first_node < x.first_node;
     });
-    uint64_t end = 0;
+    uint64_t end = 0, covered = 0;
     ok = true;
     for (auto& p : ps) {
       if (p.num_nodes == 0) continue;
       if (p.first_node < end) ok = false;
       end = (uint64_t)p.first_node + p.num_nodes;
+      covered += p.num_nodes;
     }
     c->lds_ok = ok;
+    c->nodes_ok = ok && covered == N;
   }
   slots_.push_back(c);
   by_id_[c->id] = c;
@@ -779,8 +781,10 @@ int Engine::tiles_for(int kind, const std::vector<PieceRef>& refs, int block, De
   std::vector<Tile> t;
   if (kind == TK_CSR) {
     std::vector<uint32_t> seen;
-    for (const PieceRef& r : refs)
+    for (const PieceRef& r : refs) {  // usually grouped by circuit
+      if (!seen.empty() && seen.back() == r.slot) continue;
       if (std::find(seen.begin(), seen.end(), r.slot) == seen.end()) seen.push_back(r.slot);
+    }
     for (uint32_t s : seen) {
       const uint32_t N = slots_[s]->num_nodes;
       for (uint32_t off = 0; off < N; off += (uint32_t)block)
@@ -922,7 +926,9 @@ int Engine::prefetch_tiles(const std::vector<PieceRef>& refs, int policy, int mo
   if ((st = ensure_table())) return st;
   DevBuf t;
   if ((st = tiles_for(TK_CNC, refs, cnc_block_for(policy), &t))) return st;
-  if (mode == CKT_REDUCE_ATOMIC && !fuse_dsc_) {
+  const LoopForm form = loop_form(refs, mode);
+  if (form == kFusedNodes) return tiles_for(TK_CSR, refs, 256, &t);
+  if (mode == CKT_REDUCE_ATOMIC && form == kSeparate) {
     if ((st = tiles_for(TK_WIRES, refs, 256, &t))) return st;
     LdsPlan plan;
     if ((st = lds_plan(refs, &plan))) return st;
@@ -943,13 +949,58 @@ int Engine::loop_once(const std::vector<PieceRef>& refs, int policy, int mode) {
 
 int Engine::launch_loop(const std::vector<PieceRef>& refs, int policy, int mode) {
   int st;
-  if (fuse_dsc_ && mode == CKT_REDUCE_ATOMIC) {
-    if ((st = cnc(refs, policy, true))) return st;
-  } else {
-    if ((st = cnc(refs, policy))) return st;
-    if ((st = dsc(refs, mode))) return st;
-  }
+  const LoopForm form = loop_form(refs, mode);
+  if ((st = cnc(refs, policy, form == kFusedAtomic))) return st;
+  if (form == kFusedNodes) return csr(refs, mode, true);
+  if (form == kSeparate && (st = dsc(refs, mode))) return st;
   return upv(refs);
+}
+
+// The index form of distribute_charge leaves a node's whole charge in one
+// lane's register, so update_voltages rides along wherever the launch covers
+// every node of its circuits once.  ATOMIC's order of additions is unspecified,
+// and with the early end the index is the faster way to it too, except in small
+// launches (us a loop with the index / with the atomics in calc_new_currents /
+// with the LDS reduction as its own launch: 64 x 65536 wires 230 / 417 / 234, 16 x
+// 16384 21 / 34 / 29, 4 x 4096 11.9 / 10.7 / 18.7).  Where every step runs, the
+// atomics hide behind the steps of other waves and stay fused.  The options that
+// name an ATOMIC form get it.
+constexpr uint64_t kIndexSumWires = 32768;
+
+Engine::LoopForm Engine::loop_form(const std::vector<PieceRef>& refs, int mode) const {
+  if (mode == CKT_REDUCE_ATOMIC) {
+    if (fuse_dsc_ > 0 || (fuse_dsc_ < 0 && all_steps_)) return kFusedAtomic;
+    if (fuse_dsc_ == 0) return kSeparate;
+    if (dsc_atomic_impl_ != 0) return kFusedAtomic;
+    uint64_t wires = 0;
+    for (const PieceRef& r : refs) wires += slots_[r.slot]->pieces[r.piece].num_wires;
+    if (wires < kIndexSumWires) return kFusedAtomic;
+  }
+  // every piece of every circuit named, each once (refs are grouped by slot,
+  // as all_refs lists them)
+  bool whole = true;
+  for (size_t i = 0; whole && i < refs.size();) {
+    const Circuit* c = slots_[refs[i].slot];
+    whole = c->csr_ok && c->nodes_ok && refs.size() - i >= c->num_pieces;
+    for (uint32_t k = 0; whole && k < c->num_pieces; k++)
+      whole = refs[i + k].slot == refs[i].slot && refs[i + k].piece == k;
+    i += c->num_pieces;
+    whole = whole && (i >= refs.size() || refs[i].slot > refs[i - 1].slot);
+  }
+  if (whole) return kFusedNodes;
+  return mode == CKT_REDUCE_ATOMIC ? kFusedAtomic : kSeparate;
+}
+
+int Engine::csr(const std::vector<PieceRef>& refs, int mode, bool update) {
+  int st;
+  DevBuf t;
+  if ((st = tiles_for(TK_CSR, refs, 256, &t))) return st;
+  hipEvent_t a;
+  if ((st = timed_begin(CKT_DISTRIBUTE_CHARGE, &a))) return st;
+  const hipError_t e = launch_dsc_csr(mode == CKT_REDUCE_CSR_KAHAN64, update, d_table_,
+                                      (const Tile*)t.p, t.n, 256, stream_);
+  if (e != hipSuccess) return hip_fail(e, "distribute_charge launch");
+  return timed_end(CKT_DISTRIBUTE_CHARGE, a);
 }
 
 int Engine::csr_nodes_ok(const std::vector<PieceRef>& refs) const {
@@ -1031,9 +1082,7 @@ int Engine::dsc(const std::vector<PieceRef>& refs, int mode) {
     }
   } else {
     if ((st = csr_nodes_ok(refs))) return st;
-    if ((st = tiles_for(TK_CSR, refs, 256, &t))) return st;
-    if ((st = timed_begin(CKT_DISTRIBUTE_CHARGE, &a))) return st;
-    e = launch_dsc_csr(mode == CKT_REDUCE_CSR_KAHAN64, d_table_, (const Tile*)t.p, t.n, 256, stream_);
+    return csr(refs, mode, false);
   }
   if (e != hipSuccess) return hip_fail(e, "distribute_charge launch");
   return timed_end(CKT_DISTRIBUTE_CHARGE, a);
@@ -1203,7 +1252,7 @@ int Engine::set_option(int opt, int64_t v) {
       if (v < 0 || v > 2) return fail(CKT_ERR_INVALID_ARG, "atomic implementation must be 0, 1 or 2");
       dsc_atomic_impl_ = (int)v;
       return CKT_OK;
-    case OPT_FUSE_DSC: fuse_dsc_ = v ? 1 : 0; return CKT_OK;
+    case OPT_FUSE_DSC: fuse_dsc_ = v < 0 ? -1 : v ? 1 : 0; return CKT_OK;
     case OPT_WIRES_PER_LANE:
       if (v != 1 && v != 2 && v != 4) return fail(CKT_ERR_INVALID_ARG, "wires per lane must be 1, 2 or 4");
       wires_per_lane_ = (int)v;

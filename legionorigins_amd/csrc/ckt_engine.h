@@ -78,6 +78,7 @@ struct Circuit {
   std::unordered_map<uint64_t, uint32_t> piece_index;  // descriptor -> index
   bool csr_ok = false;   // the pieces partition the wires
   bool lds_ok = false;   // node ranges of the pieces are disjoint
+  bool nodes_ok = false; // the pieces partition the nodes
   bool stream_ordered = false;  // slab from the engine stream's memory pool
   int32_t loops_left = 0;
 };
@@ -93,7 +94,8 @@ enum EngineOption {
   OPT_PERSISTENT = 2,
   OPT_WAVES_PER_SIMD = 3,
   OPT_DSC_ATOMIC_IMPL = 4,  // 0 auto, 1 global atomics, 2 LDS per piece
-  OPT_FUSE_DSC = 5,         // loop drivers: ATOMIC distribute_charge fused into calc_new_currents
+  OPT_FUSE_DSC = 5,         // loop drivers: ATOMIC distribute_charge fused into
+                            // calc_new_currents (1), its own launch (0), or as is faster (-1)
   OPT_WIRES_PER_LANE = 6,   // calc_new_currents tile = workgroup size x this (1, 2, 4) wires
   OPT_TILE_SPAN = 7,        // 0: tiles within a piece; 1: within runs of adjacent pieces
   OPT_TILE_ORDER = 8,       // 0: as given; 1: longest runs first; 2: runs interleaved
@@ -158,8 +160,7 @@ class Engine {
   // `times` times.
   int run_graph(const std::vector<PieceRef>& refs, int policy, int mode, int times);
   // One loop of `refs`: calc_new_currents, distribute_charge, update_voltages
-  // (the first two as one fused launch when OPT_FUSE_DSC is on and the mode
-  // is ATOMIC).
+  // in two or three launches (loop_form).
   int loop_once(const std::vector<PieceRef>& refs, int policy, int mode);
 
   int set_option(int opt, int64_t value);
@@ -204,6 +205,16 @@ class Engine {
   int timed_begin(int task, hipEvent_t* a);
   int timed_end(int task, hipEvent_t a);
   int csr_nodes_ok(const std::vector<PieceRef>& refs) const;
+  // How a loop's launches share the tasks:
+  //   kFusedAtomic  calc_new_currents adds the charges with atomics; update_voltages
+  //   kFusedNodes   calc_new_currents; distribute_charge over the index and
+  //                 update_voltages in one launch
+  //   kSeparate     one launch per task
+  enum LoopForm { kFusedAtomic, kFusedNodes, kSeparate };
+  LoopForm loop_form(const std::vector<PieceRef>& refs, int mode) const;
+  // distribute_charge over the index, with update_voltages of the same nodes
+  // if `update`.
+  int csr(const std::vector<PieceRef>& refs, int mode, bool update);
   // The LDS-privatised ATOMIC reduction over `refs`: whether it applies, its
   // LDS bytes, the subranges per piece and the floats of partial sums it
   // needs (allocated here, before any launch or capture).
@@ -238,7 +249,7 @@ class Engine {
   int persistent_ = -1;      // -1: chosen per policy (launch_shape)
   int waves_per_simd_ = -1;  // -1: chosen per policy
   int dsc_atomic_impl_ = 0;
-  int fuse_dsc_ = 1;
+  int fuse_dsc_ = -1;
   int wires_per_lane_ = 1;
   int tile_span_ = 0;
   int tile_order_ = 0;

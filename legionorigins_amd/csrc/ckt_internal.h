@@ -76,8 +76,9 @@ size_t dsc_lds_bytes(uint32_t max_nodes);
 hipError_t launch_dsc_lds(const DevCircuit* circuits, const PieceTile* ptiles, uint32_t n,
                           uint32_t splits, uint32_t max_nodes, float* partial, size_t lds_bytes,
                           hipStream_t s);
-hipError_t launch_dsc_csr(int kahan, const DevCircuit* circuits, const Tile* node_tiles,
-                          uint32_t ntiles, int block, hipStream_t s);
+// update: update_voltages of the same nodes in the same launch.
+hipError_t launch_dsc_csr(int kahan, bool update, const DevCircuit* circuits,
+                          const Tile* node_tiles, uint32_t ntiles, int block, hipStream_t s);
 // nontemporal: streaming accesses for node arrays larger than the last-level
 // cache.
 hipError_t launch_upv(const DevCircuit* circuits, const Tile* node_tiles, uint32_t ntiles,

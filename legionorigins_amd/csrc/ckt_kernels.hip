@@ -1185,57 +1185,92 @@ __global__ __launch_bounds__(256) void dsc_lds_sum_kernel(const DevCircuit* __re
   c.charge[n] = c.charge[n] + v;
 }
 
-// One lane per node: the node's contributions in (wire, in-before-out) order,
-// added one at a time to its charge -- the order in which the reference's
-// CPU tasks apply them when run one piece after another.
-// Node tiles in XCD-contiguous order (xcd_tile): neighbouring node tiles --
-// whose wires, and so whose gathered currents, lie in the same piece -- share
-// an L2.
-template <bool KAHAN>
-__global__ __launch_bounds__(256) void dsc_csr_kernel(const DevCircuit* __restrict__ circuits,
-                                                      const Tile* __restrict__ tiles) {
-  const Tile t = tiles[xcd_tile(blockIdx.x, gridDim.x)];
-  if (threadIdx.x >= t.count) return;
-  const DevCircuit& c = circuits[t.circuit];
-  const uint32_t n = t.first + threadIdx.x;
-  if (!CKT_IN_BOUNDS(n < c.num_nodes)) return;
-  const float dt = CKT_DT_F;
-  const float* cur0 = c.cur;
-  const float* cur9 = c.cur + (size_t)(kSeg - 1) * c.ws;
-  const uint32_t k0 = c.csr_row[n], k1 = c.csr_row[n + 1];
-  if (!CKT_IN_BOUNDS(k0 <= k1 && k1 <= 2ull * c.num_wires)) return;
-  if (!KAHAN || c.locator[n]) {
-    float acc = c.charge[n];
-    for (uint32_t k = k0; k < k1; k++) {
-      const uint32_t e = c.csr_ent[k];
-      const uint32_t w = e >> 1;
-      if (!CKT_IN_BOUNDS(w < c.num_wires)) continue;
-      const float v = (e & 1u) ? dt * cur9[w] : -dt * cur0[w];
-      acc += v;
-    }
-    c.charge[n] = acc;
-  } else {
-    double s = (double)c.charge[n], comp = 0.0;
-    for (uint32_t k = k0; k < k1; k++) {
-      const uint32_t e = c.csr_ent[k];
-      const uint32_t w = e >> 1;
-      if (!CKT_IN_BOUNDS(w < c.num_wires)) continue;
-      const float v = (e & 1u) ? dt * cur9[w] : -dt * cur0[w];
-      const double y = (double)v - comp;
-      const double tt = s + y;
-      comp = (tt - s) - y;
-      s = tt;
-    }
-    c.charge[n] = (float)s;
-  }
-}
-
 // ---------------------------------------------------------------------------
 // update_voltages (circuit_gpu.cu:330-345; circuit.cc:1299-1302).
 
 __device__ __forceinline__ float upv_one(float v, float q, float C, float lk) {
   v = v + q / C;
   return v * (1.f - lk);
+}
+
+// ---------------------------------------------------------------------------
+// One lane per node: the node's contributions in (wire, in-before-out) order,
+// added one at a time to its charge -- the order in which the reference's
+// CPU tasks apply them when run one piece after another -- and, with UPDATE,
+// the node's update_voltages right after, its charge still in a register.
+// Node tiles in XCD-contiguous order (xcd_tile): neighbouring node tiles --
+// whose wires, and so whose gathered currents, lie in the same piece -- share
+// an L2.
+//
+// Bound by the gathers of currents: a cache line from L2 per contribution (40 of
+// 68 us for 64 x 65536 wires and 64 x 16384 nodes; with the same bytes read in
+// order it takes 29).  A tile's contributions are one contiguous range of the
+// index: the workgroup gathers them kChunk at a time into LDS, eight independent
+// loads in flight per lane, and each lane then adds its node's own part in
+// order.  (One lane walking its node's list by itself keeps one dependent pair
+// of loads in flight: 73 us for that circuit, 65 so, and 68 with the update,
+// which takes 8 us as its own launch; 16 x 16384 wires 10.8 + 6.3 and 9.2 us.)
+template <bool KAHAN, bool UPDATE>
+__global__ __launch_bounds__(256) void dsc_csr_kernel(const DevCircuit* __restrict__ circuits,
+                                                      const Tile* __restrict__ tiles) {
+  constexpr uint32_t kChunk = 2048;
+  __shared__ float part[kChunk];
+  const Tile t = tiles[xcd_tile(blockIdx.x, gridDim.x)];
+  const DevCircuit& c = circuits[t.circuit];
+  const uint32_t tid = threadIdx.x;
+  if (!CKT_IN_BOUNDS((uint64_t)t.first + t.count <= c.num_nodes && t.count <= 256u)) return;
+  const float dt = CKT_DT_F;
+  const gfloat* cur0 = (const gfloat*)c.cur;
+  const gfloat* cur9 = cur0 + (size_t)(kSeg - 1) * c.ws;
+  const gcu32* ent = (const gcu32*)c.csr_ent;
+  const gcu32* row = (const gcu32*)c.csr_row;
+  [[maybe_unused]] const uint32_t num_wires = c.num_wires;
+  const bool live = tid < t.count;
+  const uint32_t n = t.first + (live ? tid : 0u);
+  const uint32_t begin = row[t.first], end = row[t.first + t.count];
+  uint32_t k = row[n], k1 = live ? row[n + 1] : 0u;
+  if (!live) k = 0;
+  if (!CKT_IN_BOUNDS(begin <= end && end <= 2ull * num_wires && k <= k1 && k1 <= end)) return;
+  const bool kahan = KAHAN && !c.locator[n];
+  gfloat* charge = (gfloat*)c.charge;
+  float acc = charge[n];
+  double s = (double)acc, comp = 0.0;
+  for (uint32_t base = begin; base < end; base += kChunk) {
+    uint32_t e[kChunk / 256];
+#pragma unroll
+    for (uint32_t u = 0; u < kChunk / 256; u++) {
+      const uint32_t i = base + u * 256u + tid;
+      e[u] = ent[i < end ? i : begin];
+      if (!CKT_IN_BOUNDS((e[u] >> 1) < num_wires)) e[u] = 0;
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kChunk / 256; u++) {
+      const uint32_t w = e[u] >> 1;
+      part[u * 256u + tid] = (e[u] & 1u) ? dt * cur9[w] : -dt * cur0[w];
+    }
+    __syncthreads();
+    const uint32_t stop = k1 < base + kChunk ? k1 : base + kChunk;
+    if (!kahan) {
+      for (; k < stop; k++) acc += part[k - base];
+    } else {
+      for (; k < stop; k++) {
+        const double y = (double)part[k - base] - comp;
+        const double tt = s + y;
+        comp = (tt - s) - y;
+        s = tt;
+      }
+    }
+    __syncthreads();
+  }
+  if (!live) return;
+  if (kahan) acc = (float)s;
+  if constexpr (UPDATE) {
+    gfloat* voltage = (gfloat*)c.voltage;
+    voltage[n] = upv_one(voltage[n], acc, ((const gfloat*)c.ncap)[n], ((const gfloat*)c.leak)[n]);
+    charge[n] = 0.f;
+  } else {
+    charge[n] = acc;
+  }
 }
 
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -1591,13 +1626,16 @@ hipError_t launch_dsc_lds(const DevCircuit* c, const PieceTile* pt, uint32_t n, 
   return hipGetLastError();
 }
 
-hipError_t launch_dsc_csr(int kahan, const DevCircuit* c, const Tile* t, uint32_t n, int block,
-                          hipStream_t s) {
+hipError_t launch_dsc_csr(int kahan, bool update, const DevCircuit* c, const Tile* t, uint32_t n,
+                          int block, hipStream_t s) {
   if (n == 0) return hipSuccess;
   if (block != 256) return hipErrorInvalidValue;
-  if (kahan) hipLaunchKernelGGL(dsc_csr_kernel<true>, dim3(n), dim3(256), 0, s, c, t);
-  else hipLaunchKernelGGL(dsc_csr_kernel<false>, dim3(n), dim3(256), 0, s, c, t);
-  return hipGetLastError();
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(n), dim3(256), 0, s, c, t);
+    return hipGetLastError();
+  };
+  if (kahan) return update ? go(dsc_csr_kernel<true, true>) : go(dsc_csr_kernel<true, false>);
+  return update ? go(dsc_csr_kernel<false, true>) : go(dsc_csr_kernel<false, false>);
 }
 
 hipError_t launch_upv(const DevCircuit* c, const Tile* t, uint32_t n, int block, bool nontemporal,
