@@ -964,6 +964,22 @@ struct Relax<CKT_POLICY_SCALED> {
 typedef __attribute__((address_space(1))) float gfloat;
 typedef __attribute__((address_space(1))) const uint32_t gcu32;
 
+// A wire's state is read and written once per loop, so with the early end, where
+// the launch is bound by those bytes, they are nontemporal: 64 x 65536 wires 157
+// us instead of 171 (stores alone gain nothing).  The two currents that the
+// charge reduction reads next stay ordinary stores, and are then still cached:
+// its launch takes 49.5 instead of 68 us, and the loop 201 instead of 230.
+template <bool kNt, class T>
+__device__ __forceinline__ T load_once(const __attribute__((address_space(1))) T* p) {
+  if constexpr (kNt) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool kNt>
+__device__ __forceinline__ void store_once(float v, gfloat* p) {
+  if constexpr (kNt) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
 // FUSE: the wire's two charge contributions (distribute_charge's ATOMIC
 // mode, circuit_gpu.cu:273-283) are added from registers right after the
 // relaxation, so the loop drivers skip the separate launch.
@@ -977,18 +993,21 @@ __device__ __forceinline__ void cnc_one(const DevCircuit& c, uint32_t w, int ste
     return;
   float I[kSeg], V[kSeg - 1];
 #pragma unroll
-  for (int s = 0; s < kSeg; s++) I[s] = cur[s * ws + w];
+  for (int s = 0; s < kSeg; s++) I[s] = load_once<St::on>(&cur[s * ws + w]);
 #pragma unroll
-  for (int s = 0; s < kSeg - 1; s++) V[s] = vol[s * ws + w];
+  for (int s = 0; s < kSeg - 1; s++) V[s] = load_once<St::on>(&vol[s * ws + w]);
   const float L = ((gfloat*)c.ind)[w], R = ((gfloat*)c.res)[w], C = ((gfloat*)c.wcap)[w];
   const float vin = ((gfloat*)c.voltage)[((gcu32*)c.in_ptr)[w]];
   const float vout = ((gfloat*)c.voltage)[((gcu32*)c.out_ptr)[w]];
   Relax<POLICY>::run(I, V, vin, vout, L, R, C, steps, st);
   asm volatile("" : "+v"(w));
 #pragma unroll
-  for (int s = 0; s < kSeg; s++) cur[s * ws + w] = I[s];
+  for (int s = 0; s < kSeg; s++) {
+    if (s == 0 || s == kSeg - 1) cur[s * ws + w] = I[s];
+    else store_once<St::on>(I[s], &cur[s * ws + w]);
+  }
 #pragma unroll
-  for (int s = 0; s < kSeg - 1; s++) vol[s * ws + w] = V[s];
+  for (int s = 0; s < kSeg - 1; s++) store_once<St::on>(V[s], &vol[s * ws + w]);
   if (FUSE) {
     const float dt = CKT_DT_F;
     unsafeAtomicAdd(&c.charge[c.in_ptr[w]], -dt * I[0]);
