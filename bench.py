@@ -602,7 +602,7 @@ def run_gen(C, args):
         log(f"[gen] {row}")
     print(json.dumps({"metric": "circuit generation (load_circuit) throughput", "unit": "wires/s",
                       "host": "generator on one host thread + slab upload",
-                      "device": "start-state chain on the host, draws/classification/index on the GPU",
+                      "device": "draws, classification and index on the GPU",
                       "rows": rows}))
 
 

@@ -276,9 +276,9 @@ int ckt_ctx_load(ckt_ctx_t* ctx, const ckt_node_t* nodes, uint32_t num_nodes,
 int ckt_ctx_generate(ckt_ctx_t* ctx, const ckt_gen_params_t* params);
 /* Same circuit, bit for bit, generated in HBM (load_circuit,
  * circuit.cc:1071-1288, without the host image or its upload): the host
- * walks the drand48 chain once to find each wire's first draw, the device
- * draws every node and wire, marks shared nodes, derives the locations and
- * sorts the node->wire index. */
+ * sends only the parameters; the device finds each wire's first draw in the
+ * drand48 sequence, draws every node and wire, marks shared nodes, derives the
+ * locations and sorts the node->wire index. */
 int ckt_ctx_generate_device(ckt_ctx_t* ctx, const ckt_gen_params_t* params);
 /* Download the current state back into the reference layouts (host memory;
  * either pointer may be NULL).  Waits for the stream. */
@@ -452,8 +452,7 @@ typedef struct ckt_server_config {
   int32_t max_active;          /* cap on resident circuits (0 = none) */
   int32_t policy;
   int32_t reduce_mode;
-  int32_t gen_threads;         /* host threads walking admitted circuits' generator chains (the
-                                  circuits themselves are generated on the device) */
+  int32_t gen_threads;         /* accepted and unused: circuits are generated on the device */
 } ckt_server_config_t;
 
 typedef struct ckt_request {

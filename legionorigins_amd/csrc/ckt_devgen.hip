@@ -4,22 +4,18 @@
 // The reference draws from one drand48 stream in a fixed order: three draws
 // per node, then per wire six (in-piece) or seven (cross-piece) draws.  A
 // node's first draw is a fixed jump from the seed, so every node is drawn
-// independently on the device.  A wire's first draw depends on how many
-// earlier wires were cross-piece, which is only known by walking the chain:
-// the host does that walk (two 48-bit multiply-adds per wire: jump to the
-// in-piece test, then jump to the next wire).  The synchronous build streams
-// the start states to the device in chunks, overlapped with the device
-// drawing the previous chunk; the planned build takes a walk done earlier
-// (on any thread) and only enqueues device work, so a server can issue it
-// behind a running iteration.  The device then marks shared nodes, derives
-// the locations, and builds the node -> (wire, end) index with a stable
-// radix sort.  The slab is bit-identical to the host generator's image
-// (ckt_generator.cpp + finalize_image).  The library is compiled with
-// -ffp-contract=off, so the double expressions round exactly as on the host.
+// independently.  A wire's first draw depends on how many earlier wires were
+// cross-piece; that chain is cut into spans of the draw sequence whose effect
+// on it is known for each of the seven ways in which it can enter them
+// (gen_spans, scan_spans), so that every span's wires are drawn independently
+// too.  The device then marks shared nodes, derives the locations, and builds
+// the node -> (wire, end) index with a stable radix sort.  The slab is
+// bit-identical to the host generator's image (ckt_generator.cpp +
+// finalize_image).  The library is compiled with -ffp-contract=off, so the
+// double expressions round exactly as on the host.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstring>
 #include <vector>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -33,7 +29,6 @@ namespace {
 
 constexpr uint64_t kMask48 = (1ull << 48) - 1;
 constexpr uint64_t kA = 0x5DEECE66Dull, kC = 0xBull;
-constexpr uint32_t kChunk = 1u << 22;  // wires per host -> device start-state chunk
 
 // s -> a*s + c (mod 2^48): a number of steps of the drand48 recurrence.
 struct Jump {
@@ -43,6 +38,11 @@ struct Jump {
 // Jumps of 3 * 2^k draws: node i starts 3*i draws after the seed.
 struct NodeJumps {
   Jump j[32];
+};
+
+// Jumps of 2^k draws (a circuit of 2^30 nodes and wires takes under 2^34).
+struct DrawJumps {
+  Jump j[34];
 };
 
 __host__ __device__ __forceinline__ uint64_t apply(const Jump& j, uint64_t s) {
@@ -85,21 +85,192 @@ __global__ __launch_bounds__(256) void gen_nodes(uint32_t N, uint64_t seed_state
   leak[i] = (float)((double)0.1f * draw(s));
 }
 
-// Wires first .. first+count-1 (circuit.cc:1147-1193); state[k] is wire
-// first+k's start state.  A cross-piece wire's out-node becomes shared.
-__global__ __launch_bounds__(256) void gen_wires(uint32_t first, uint32_t count, uint32_t P,
-                                                 uint32_t npp, uint32_t wpp, int32_t pct,
-                                                 int32_t stable, const uint64_t* __restrict__ state,
-                                                 float* __restrict__ ind, float* __restrict__ res,
-                                                 float* __restrict__ wcap,
+// The wires' draws, position 0 the first wire's first draw, are cut into spans
+// of kSpan positions, each into kSubs sub-spans.  A wire that starts at
+// position p starts the next wire at p + 6, or at p + 7 if it is cross-piece
+// (its fifth draw, circuit.cc:1167).  So a chain enters a sub-span at one of its
+// first seven positions, and for each of them the walk through it (about 21
+// wires, one dependent LDS read each) gives where it enters the next one and how
+// many wires it started.  For 4.2 M wires the spans take 69 us, their composition
+// 61 and the wires 98, bound by the walks' latency and the draws' 64-bit
+// multiplies; the whole circuit is built in 1.4 ms, where one host core's walk of
+// the chain made it 26.
+constexpr uint32_t kSpan = 1024, kSubs = 8, kSub = kSpan / kSubs, kEntries = 7;
+
+struct SpanScratch {
+  uint8_t cross[kSpan];                   // whether a wire that starts here is cross-piece
+  uint16_t step[kSubs][kEntries + 1];     // count << 3 | entry into the next sub-span
+};
+
+// Fills `sp` for span b: lane t takes positions 4 t .. 4 t + 3.  With `states`,
+// also each position's state (before its draw).
+template <bool kStates>
+__device__ __forceinline__ void walk_span(uint32_t b, uint64_t first_state, const DrawJumps& t,
+                                          const Jump& j5, int32_t pct, SpanScratch& sp,
+                                          uint64_t* states) {
+  const uint32_t p0 = 4u * threadIdx.x;
+  uint64_t s = first_state;
+  uint64_t m = (uint64_t)b * kSpan + p0;
+  for (uint32_t k = 0; m; k++, m >>= 1)
+    if (m & 1) s = apply(t.j[k], s);
+  if (kStates) {
+    uint64_t x = s;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) {
+      states[p0 + k] = x;
+      x = (kA * x + kC) & kMask48;
+    }
+  }
+  s = apply(j5, s);
+  uint32_t four = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; k++) {
+    const double u = (double)s * 0x1p-48;
+    four |= ((100 * u) < pct ? 0u : 1u) << (8 * k);
+    s = (kA * s + kC) & kMask48;
+  }
+  *(uint32_t*)(sp.cross + p0) = four;
+  __syncthreads();
+  if (threadIdx.x < kSubs * 8 && (threadIdx.x & 7u) < kEntries) {
+    const uint32_t sub = threadIdx.x >> 3, end = (sub + 1) * kSub;
+    uint32_t p = sub * kSub + (threadIdx.x & 7u), n = 0;
+    for (; p < end; n++) p += 6u + sp.cross[p];
+    sp.step[sub][threadIdx.x & 7u] = (uint16_t)(n << 3 | (p - end));
+  }
+  __syncthreads();
+}
+
+// Each span's step for each entry, as in SpanScratch::step, eight to a span.
+__global__ __launch_bounds__(256) void gen_spans(uint64_t first_state, DrawJumps t, Jump j5,
+                                                 int32_t pct, uint16_t* __restrict__ steps) {
+  __shared__ SpanScratch sp;
+  walk_span<false>(blockIdx.x, first_state, t, j5, pct, sp, nullptr);
+  if (threadIdx.x < kEntries) {
+    uint32_t e = threadIdx.x, n = 0;
+    for (uint32_t sub = 0; sub < kSubs; sub++) {
+      const uint32_t v = sp.step[sub][e];
+      n += v >> 3;
+      e = v & 7u;
+    }
+    steps[(size_t)blockIdx.x * 8 + threadIdx.x] = (uint16_t)(n << 3 | e);
+  }
+}
+
+// Where the chain that starts at position 0 enters each span and the wire it
+// starts first there.  One workgroup: lane t composes the steps of its share of
+// the spans, 32 lanes compose 32 lanes' shares each, one lane walks those 32, and
+// the same again downwards.
+__global__ __launch_bounds__(1024) void scan_spans(uint32_t spans, const uint16_t* __restrict__ steps,
+                                                   uint2* __restrict__ starts) {
+  __shared__ uint32_t count[1024][kEntries], group_count[32][kEntries];
+  __shared__ uint8_t exit_to[1024][kEntries], group_exit[32][kEntries];
+  __shared__ uint32_t enter[1024], first[1024], group_enter[32], group_first[32];
+  const uint32_t t = threadIdx.x, share = (spans + 1023u) / 1024u;
+  const uint32_t lo = t * share < spans ? t * share : spans;
+  const uint32_t hi = lo + share < spans ? lo + share : spans;
+  auto at = [](const uint4& v, uint32_t e) {  // entry e of a span's eight steps
+    const uint32_t w = e < 4 ? (e < 2 ? v.x : v.y) : (e < 6 ? v.z : v.w);
+    return (w >> (16u * (e & 1u))) & 0xffffu;
+  };
+  const uint4* spans4 = (const uint4*)steps;
+  uint32_t e[kEntries], n[kEntries];
+#pragma unroll
+  for (uint32_t k = 0; k < kEntries; k++) e[k] = k, n[k] = 0;
+  for (uint32_t b = lo; b < hi; b++) {
+    const uint4 v = spans4[b];
+#pragma unroll
+    for (uint32_t k = 0; k < kEntries; k++) {
+      const uint32_t x = at(v, e[k]);
+      n[k] += x >> 3;
+      e[k] = x & 7u;
+    }
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < kEntries; k++) {
+    count[t][k] = n[k];
+    exit_to[t][k] = (uint8_t)e[k];
+  }
+  __syncthreads();
+  if (t < 32 * 8 && (t & 7u) < kEntries) {
+    const uint32_t g = t >> 3;
+    uint32_t x = t & 7u, c = 0;
+    for (uint32_t k = g * 32; k < g * 32 + 32; k++) {
+      c += count[k][x];
+      x = exit_to[k][x];
+    }
+    group_count[g][t & 7u] = c;
+    group_exit[g][t & 7u] = (uint8_t)x;
+  }
+  __syncthreads();
+  if (t == 0) {
+    uint32_t x = 0, c = 0;
+    for (uint32_t g = 0; g < 32; g++) {
+      group_enter[g] = x;
+      group_first[g] = c;
+      c += group_count[g][x];
+      x = group_exit[g][x];
+    }
+  }
+  __syncthreads();
+  if (t < 32) {
+    uint32_t x = group_enter[t], c = group_first[t];
+    for (uint32_t k = t * 32; k < t * 32 + 32; k++) {
+      enter[k] = x;
+      first[k] = c;
+      c += count[k][x];
+      x = exit_to[k][x];
+    }
+  }
+  __syncthreads();
+  uint32_t x = enter[t], c = first[t];
+  for (uint32_t b = lo; b < hi; b++) {
+    starts[b] = make_uint2(x, c);
+    const uint32_t v = at(spans4[b], x);
+    c += v >> 3;
+    x = v & 7u;
+  }
+}
+
+// The wires that start in span blockIdx.x (circuit.cc:1147-1193).  A
+// cross-piece wire's out-node becomes shared.
+__global__ __launch_bounds__(256) void gen_wires(uint32_t W, uint64_t first_state, DrawJumps t,
+                                                 Jump j5, const uint2* __restrict__ starts,
+                                                 uint32_t P, uint32_t npp, uint32_t wpp, int32_t pct,
+                                                 int32_t stable, float* __restrict__ ind,
+                                                 float* __restrict__ res, float* __restrict__ wcap,
                                                  uint32_t* __restrict__ in_ptr,
                                                  uint32_t* __restrict__ out_ptr, uint8_t* locator) {
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
-  if (k >= count) return;
-  const uint32_t w = first + k;
+  __shared__ SpanScratch sp;
+  __shared__ uint64_t states[kSpan];
+  __shared__ uint16_t at[kSpan / 6 + 2];
+  __shared__ uint16_t sub_enter[kSubs], sub_first[kSubs + 1];
+  const uint2 start = starts[blockIdx.x];
+  if (start.y >= W) return;
+  walk_span<true>(blockIdx.x, first_state, t, j5, pct, sp, states);
+  if (threadIdx.x == 0) {
+    uint32_t e = start.x, n = 0;
+    for (uint32_t sub = 0; sub < kSubs; sub++) {
+      sub_enter[sub] = (uint16_t)e;
+      sub_first[sub] = (uint16_t)n;
+      const uint32_t v = sp.step[sub][e];
+      n += v >> 3;
+      e = v & 7u;
+    }
+    sub_first[kSubs] = (uint16_t)n;
+  }
+  __syncthreads();
+  if (threadIdx.x < kSubs) {
+    const uint32_t sub = threadIdx.x, end = (sub + 1) * kSub;
+    uint32_t k = sub_first[sub];
+    for (uint32_t p = sub * kSub + sub_enter[sub]; p < end; p += 6u + sp.cross[p])
+      at[k++] = (uint16_t)p;
+  }
+  __syncthreads();
+  if (threadIdx.x >= sub_first[kSubs] || threadIdx.x >= W - start.y) return;
+  const uint32_t w = start.y + threadIdx.x;
   const uint32_t n = w / wpp;
   const uint32_t base = n * npp;
-  uint64_t s = state[k];
+  uint64_t s = states[at[threadIdx.x]];
   float R, L, C;
   if (stable) {  // the same draws; inductance x 1e-6, capacitance U(0.001, 0.011)
     R = (float)(draw(s) * 10 + 1);
@@ -197,27 +368,6 @@ uint64_t seed_state_of(const ckt_gen_params_t* p) {
   return ((uint64_t)(uint32_t)p->random_seed << 16) | 0x330Eull;
 }
 
-// Start states of wires [0, W): the only sequential part of load_circuit.
-// Per chunk of up to `chunk` wires, fn.begin(first, n) returns where to write
-// the n states and fn.end(first, n) is called once they are written.
-template <class Sink>
-void walk_wire_states(const ckt_gen_params_t* p, uint32_t N, uint32_t W, size_t chunk, Sink&& fn) {
-  const Jump j5 = jump(5), j6 = jump(6), j7 = jump(7);
-  const int32_t pct = p->pct_wire_in_piece;
-  uint64_t x = apply(jump(3ull * N), seed_state_of(p));
-  for (uint32_t first = 0; first < W; first += (uint32_t)chunk) {
-    const uint32_t n = (uint32_t)std::min<size_t>(chunk, W - first);
-    uint64_t* h = fn.begin(first, n);
-    for (uint32_t i = 0; i < n; i++) {
-      h[i] = x;
-      // The wire's fifth draw is the in-piece test (circuit.cc:1167).
-      const double u = (double)apply(j5, x) * 0x1p-48;
-      x = ((100 * u) < pct) ? apply(j6, x) : apply(j7, x);
-    }
-    fn.end(first, n);
-  }
-}
-
 // Slab arrays the kernels write.
 struct SlabView {
   uint8_t* b;
@@ -245,14 +395,33 @@ int enqueue_nodes(const ckt_gen_params_t* p, uint32_t N, uint32_t P, const SlabV
   return CKT_OK;
 }
 
-int enqueue_wires(const ckt_gen_params_t* p, uint32_t P, uint32_t first, uint32_t n,
-                  const uint64_t* d_state, const SlabView& v, hipStream_t s) {
-  if (n == 0) return CKT_OK;
-  hipLaunchKernelGGL(gen_wires, dim3(grid_for(n)), dim3(256), 0, s, first, n, P,
-                     (uint32_t)p->nodes_per_piece, (uint32_t)p->wires_per_piece,
-                     p->pct_wire_in_piece, (int32_t)(p->profile == CKT_PROFILE_STABLE), d_state,
-                     v.f(v.L.ind), v.f(v.L.res), v.f(v.L.wcap), v.u(v.L.in_ptr), v.u(v.L.out_ptr),
-                     v.b + v.L.locator);
+uint32_t span_count(uint32_t W) { return (uint32_t)((7ull * W + kSpan - 1) / kSpan); }
+
+size_t align256(size_t x) { return (x + 255) / 256 * 256; }
+
+// Scratch of the wires' draws: eight steps and a start per span.
+size_t span_scratch_bytes(uint32_t W) {
+  return align256((size_t)span_count(W) * 8 * sizeof(uint16_t)) +
+         align256((size_t)span_count(W) * sizeof(uint2));
+}
+
+int enqueue_wires(const ckt_gen_params_t* p, uint32_t N, uint32_t W, uint32_t P, void* scratch,
+                  const SlabView& v, hipStream_t s) {
+  if (W == 0) return CKT_OK;
+  const uint32_t spans = span_count(W);
+  uint16_t* steps = (uint16_t*)scratch;
+  uint2* starts = (uint2*)((uint8_t*)scratch + align256((size_t)spans * 8 * sizeof(uint16_t)));
+  DrawJumps t{};
+  for (int k = 0; k < 34; k++) t.j[k] = jump(1ull << k);
+  const uint64_t first = apply(jump(3ull * N), seed_state_of(p));
+  const Jump j5 = jump(5);
+  const int32_t pct = p->pct_wire_in_piece;
+  hipLaunchKernelGGL(gen_spans, dim3(spans), dim3(256), 0, s, first, t, j5, pct, steps);
+  hipLaunchKernelGGL(scan_spans, dim3(1), dim3(1024), 0, s, spans, steps, starts);
+  hipLaunchKernelGGL(gen_wires, dim3(spans), dim3(256), 0, s, W, first, t, j5, starts, P,
+                     (uint32_t)p->nodes_per_piece, (uint32_t)p->wires_per_piece, pct,
+                     (int32_t)(p->profile == CKT_PROFILE_STABLE), v.f(v.L.ind), v.f(v.L.res),
+                     v.f(v.L.wcap), v.u(v.L.in_ptr), v.u(v.L.out_ptr), v.b + v.L.locator);
   CKT_HIP(hipGetLastError());
   return CKT_OK;
 }
@@ -269,8 +438,6 @@ unsigned key_bits(uint32_t N) {
   while (bits < 32 && (1ull << bits) < N) bits++;
   return bits;
 }
-
-size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
 // Bytes of scratch for N nodes and W wires; with `base`, carves it.
 int index_scratch(uint32_t N, uint32_t W, void* base, IndexScratch* sc, size_t* bytes) {
@@ -321,126 +488,7 @@ int enqueue_index(const ckt_gen_params_t* p, uint32_t N, uint32_t W, const SlabV
   return enqueue_sort(N, W, v.u(v.L.csr_row), v.u(v.L.csr_ent), sc, s);
 }
 
-// Temporary device and pinned buffers and events of one synchronous build;
-// released after the stream has drained.
-struct Temps {
-  hipStream_t s;
-  std::vector<void*> dev, host;
-  std::vector<hipEvent_t> events;
-  explicit Temps(hipStream_t st) : s(st) {}
-  ~Temps() {
-    (void)hipStreamSynchronize(s);
-    for (void* p : dev) (void)hipFree(p);
-    for (void* p : host) (void)hipHostFree(p);
-    for (hipEvent_t e : events) (void)hipEventDestroy(e);
-  }
-  hipError_t device(void** p, size_t bytes) {
-    hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 16));
-    if (e == hipSuccess) dev.push_back(*p);
-    return e;
-  }
-  hipError_t pinned(void** p, size_t bytes) {
-    hipError_t e = hipHostMalloc(p, std::max<size_t>(bytes, 16), hipHostMallocDefault);
-    if (e == hipSuccess) host.push_back(*p);
-    return e;
-  }
-  hipError_t event(hipEvent_t* ev) {
-    hipError_t e = hipEventCreateWithFlags(ev, hipEventDisableTiming);
-    if (e == hipSuccess) events.push_back(*ev);
-    return e;
-  }
-};
-
 }  // namespace
-
-// Synchronous build: the host walks the start-state chain in chunks of 2^22
-// wires, two chunks in flight, so copying and drawing chunk c overlaps the
-// walk over chunk c+1.
-int devgen_build(const ckt_gen_params_t* params, const SlabLayout& L, void* slab, hipStream_t s,
-                 std::vector<ckt_piece_t>& pieces) {
-  uint32_t N, W, P;
-  int st = gen_validate(params, &N, &W, &P);
-  if (st) return st;
-  const SlabView v{(uint8_t*)slab, L};
-  Temps tmp(s);
-  if ((st = enqueue_nodes(params, N, P, v, s))) return st;
-
-  uint64_t* h_ring[2] = {nullptr, nullptr};
-  uint64_t* d_ring[2] = {nullptr, nullptr};
-  hipEvent_t copied[2] = {nullptr, nullptr};
-  const size_t chunk = std::min<size_t>(kChunk, std::max<uint32_t>(W, 1));
-  for (int k = 0; k < 2; k++) {
-    CKT_HIP(tmp.pinned((void**)&h_ring[k], chunk * sizeof(uint64_t)));
-    CKT_HIP(tmp.device((void**)&d_ring[k], chunk * sizeof(uint64_t)));
-    CKT_HIP(tmp.event(&copied[k]));
-  }
-  struct RingSink {
-    uint64_t** h;
-    uint64_t** d;
-    hipEvent_t* ev;
-    hipStream_t s;
-    const ckt_gen_params_t* p;
-    uint32_t P;
-    const SlabView& v;
-    uint32_t c = 0;
-    int st = CKT_OK;
-    uint64_t* begin(uint32_t, uint32_t) {
-      // chunk c-2's copy must have left this buffer
-      if (c >= 2 && st == CKT_OK) {
-        hipError_t e = hipEventSynchronize(ev[c & 1]);
-        if (e != hipSuccess) st = hip_fail(e, "hipEventSynchronize");
-      }
-      return h[c & 1];
-    }
-    void end(uint32_t first, uint32_t n) {
-      const int k = (int)(c & 1);
-      c++;
-      if (st) return;
-      hipError_t e = hipMemcpyAsync(d[k], h[k], n * sizeof(uint64_t), hipMemcpyHostToDevice, s);
-      if (e == hipSuccess) e = hipEventRecord(ev[k], s);
-      if (e != hipSuccess) {
-        st = hip_fail(e, "wire start states upload");
-        return;
-      }
-      st = enqueue_wires(p, P, first, n, d[k], v, s);
-    }
-  } sink{h_ring, d_ring, copied, s, params, P, v};
-  walk_wire_states(params, N, W, chunk, sink);
-  if (sink.st) return sink.st;
-
-  size_t bytes = 0;
-  IndexScratch sc{};
-  if ((st = index_scratch(N, W, nullptr, nullptr, &bytes))) return st;
-  void* base = nullptr;
-  CKT_HIP(tmp.device(&base, bytes));
-  if ((st = index_scratch(N, W, base, &sc, &bytes))) return st;
-  if ((st = enqueue_index(params, N, W, v, sc, s))) return st;
-  pieces.resize(P);
-  for (uint32_t n = 0; n < P; n++)
-    pieces[n] = ckt_piece_t{n * (uint32_t)params->wires_per_piece,
-                            (uint32_t)params->wires_per_piece, n * (uint32_t)params->nodes_per_piece,
-                            (uint32_t)params->nodes_per_piece};
-  CKT_HIP(hipStreamSynchronize(s));
-  return CKT_OK;
-}
-
-int devgen_plan(const ckt_gen_params_t* params, DevgenPlan& plan) {
-  uint32_t N, W, P;
-  int st = gen_validate(params, &N, &W, &P);
-  if (st) return st;
-  plan.params = *params;
-  plan.N = N;
-  plan.W = W;
-  plan.P = P;
-  plan.wire_state.resize(W);
-  struct VecSink {
-    uint64_t* base;
-    uint64_t* begin(uint32_t first, uint32_t) { return base + first; }
-    void end(uint32_t, uint32_t) {}
-  } sink{plan.wire_state.data()};
-  walk_wire_states(params, N, W, std::max<uint32_t>(W, 1), sink);
-  return CKT_OK;
-}
 
 size_t index_scratch_bytes(uint32_t N, uint32_t W) {
   size_t bytes = 0;
@@ -460,32 +508,24 @@ int index_enqueue(const DevCircuit& c, void* scratch, hipStream_t s) {
 }
 
 size_t devgen_scratch_bytes(uint32_t N, uint32_t W) {
-  size_t bytes = 0;
-  if (index_scratch(N, W, nullptr, nullptr, &bytes)) return 0;
-  return align256((size_t)W * sizeof(uint64_t)) + bytes;
+  const size_t index = index_scratch_bytes(N, W);
+  return index ? span_scratch_bytes(W) + index : 0;
 }
 
-int devgen_enqueue(const DevgenPlan& plan, const uint64_t* staged_state, const SlabLayout& L,
-                   void* slab, void* scratch, hipStream_t s, std::vector<ckt_piece_t>& pieces) {
-  const ckt_gen_params_t* p = &plan.params;
+int devgen_enqueue(const ckt_gen_params_t* p, const SlabLayout& L, void* slab, void* scratch,
+                   hipStream_t s, std::vector<ckt_piece_t>& pieces) {
+  uint32_t N, W, P;
+  int st = gen_validate(p, &N, &W, &P);
+  if (st) return st;
   const SlabView v{(uint8_t*)slab, L};
-  int st;
-  if ((st = enqueue_nodes(p, plan.N, plan.P, v, s))) return st;
-  uint64_t* d_state = (uint64_t*)scratch;
-  if (plan.W) {
-    CKT_HIP(hipMemcpyAsync(d_state, staged_state, (size_t)plan.W * sizeof(uint64_t),
-                           hipMemcpyHostToDevice, s));
-    if ((st = enqueue_wires(p, plan.P, 0, plan.W, d_state, v, s))) return st;
-  }
+  if ((st = enqueue_nodes(p, N, P, v, s))) return st;
+  if ((st = enqueue_wires(p, N, W, P, scratch, v, s))) return st;
   size_t bytes = 0;
   IndexScratch sc{};
-  if ((st = index_scratch(plan.N, plan.W, (uint8_t*)scratch +
-                                               align256((size_t)plan.W * sizeof(uint64_t)),
-                          &sc, &bytes)))
-    return st;
-  if ((st = enqueue_index(p, plan.N, plan.W, v, sc, s))) return st;
-  pieces.resize(plan.P);
-  for (uint32_t n = 0; n < plan.P; n++)
+  if ((st = index_scratch(N, W, (uint8_t*)scratch + span_scratch_bytes(W), &sc, &bytes))) return st;
+  if ((st = enqueue_index(p, N, W, v, sc, s))) return st;
+  pieces.resize(P);
+  for (uint32_t n = 0; n < P; n++)
     pieces[n] = ckt_piece_t{n * (uint32_t)p->wires_per_piece, (uint32_t)p->wires_per_piece,
                             n * (uint32_t)p->nodes_per_piece, (uint32_t)p->nodes_per_piece};
   return CKT_OK;

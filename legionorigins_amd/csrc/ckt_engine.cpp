@@ -262,9 +262,9 @@ int Engine::init(int device, uint64_t budget_bytes) {
   lds_limit_ = lds;
   budget_ = budget_bytes ? budget_bytes : (uint64_t)(0.9 * (double)hbm);
   CKT_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
-  // Planned circuits come from the device's default memory pool; keep what
-  // they release for reuse instead of returning it at each synchronisation.
-  // Without pool support, planned circuits use plain allocations instead.
+  // Asynchronously generated circuits come from the device's default memory
+  // pool; keep what they release for reuse instead of returning it at each
+  // synchronisation.  Without pool support they use plain allocations.
   hipMemPool_t pool = nullptr;
   uint64_t keep = UINT64_MAX;
   pool_ok_ = hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess &&
@@ -307,6 +307,24 @@ struct RecordScratch {
 // Scratch up to this size is kept with the engine for the next build.
 constexpr size_t kKeepScratch = 64u << 20;
 }  // namespace
+
+int Engine::build_scratch(size_t need, void** scratch, void** own) {
+  *scratch = *own = nullptr;
+  if (need > devgen_scratch_cap_ && need <= kKeepScratch) {
+    // Builds already enqueued use the old scratch.
+    CKT_HIP(hipStreamSynchronize(stream_));
+    if (devgen_scratch_) CKT_HIP(hipFree(devgen_scratch_));
+    devgen_scratch_ = nullptr;
+    devgen_scratch_cap_ = 0;
+    if (hipMalloc(&devgen_scratch_, need) == hipSuccess) devgen_scratch_cap_ = need;
+    else devgen_scratch_ = nullptr;
+  }
+  if (need <= devgen_scratch_cap_) *scratch = devgen_scratch_;
+  else if (hipMalloc(own, need) == hipSuccess) *scratch = *own;
+  else *own = nullptr;
+  (void)hipGetLastError();
+  return CKT_OK;
+}
 
 int Engine::build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, const int32_t* locator,
                           const ckt_piece_t* pieces, const DevCircuit& c, void* scratch) {
@@ -403,23 +421,14 @@ int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* w
   void *slab = nullptr, *own = nullptr;
   const size_t need = RecordScratch(N, W, P).bytes;
   bool fits = !budget_ || in_use + lay.total <= budget_;
-  if (fits && need > devgen_scratch_cap_ && need <= kKeepScratch) {
-    // Builds already enqueued use the old scratch.
-    CKT_HIP(hipStreamSynchronize(stream_));
-    if (devgen_scratch_) CKT_HIP(hipFree(devgen_scratch_));
-    devgen_scratch_ = nullptr;
-    devgen_scratch_cap_ = 0;
-    fits = hipMalloc(&devgen_scratch_, need) == hipSuccess;
-    if (fits) devgen_scratch_cap_ = need;
-    else devgen_scratch_ = nullptr;
-  } else if (fits && need > devgen_scratch_cap_) {
-    fits = hipMalloc(&own, need) == hipSuccess;
-  }
+  void* scratch = nullptr;
+  if (fits && (st = build_scratch(need, &scratch, &own))) return st;
+  fits = fits && scratch;
   fits = fits && hipMalloc(&slab, lay.total) == hipSuccess;
   (void)hipGetLastError();
   if (fits) {
     st = build_records(nodes, wires, locator, pieces, device_view(slab, lay, N, W, P),
-                       own ? own : devgen_scratch_);
+                       scratch);
     const hipError_t e = hipStreamSynchronize(stream_);
     if (!st && e != hipSuccess) st = hip_fail(e, "load");
     if (own) (void)hipFree(own);
@@ -455,8 +464,16 @@ int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loop
   hipError_t e = hipMalloc(&slab, lay.total);
   if (e != hipSuccess) return hip_fail(e, "hipMalloc(circuit)");
   std::vector<ckt_piece_t> pieces;
-  if ((st = devgen_build(params, lay, slab, stream_, pieces))) {
-    (void)hipStreamSynchronize(stream_);
+  void *scratch = nullptr, *own = nullptr;
+  const size_t need = devgen_scratch_bytes(N, W);
+  if (!need) st = fail(CKT_ERR_HIP, "device generator scratch size query failed");
+  else if (!(st = build_scratch(need, &scratch, &own)) && !scratch)
+    st = fail(CKT_ERR_NO_MEMORY, "device generator: no memory for its scratch");
+  if (!st) st = devgen_enqueue(params, lay, slab, scratch, stream_, pieces);
+  e = hipStreamSynchronize(stream_);
+  if (!st && e != hipSuccess) st = hip_fail(e, "device generator");
+  if (own) (void)hipFree(own);
+  if (st) {
     (void)hipFree(slab);
     return st;
   }
@@ -1154,14 +1171,16 @@ int Engine::stage(const void* src, size_t bytes, void** out) {
   return CKT_OK;
 }
 
-int Engine::add_planned(const DevgenPlan& plan, int32_t loops, uint32_t* id) {
+int Engine::add_generated_async(const ckt_gen_params_t* params, int32_t loops, uint32_t* id) {
+  uint32_t N, W, P;
+  int st = gen_validate(params, &N, &W, &P);
+  if (st) return st;
   CKT_HIP(hipSetDevice(device_));
-  const SlabLayout lay = SlabLayout::make(plan.N, plan.W, plan.P);
+  const SlabLayout lay = SlabLayout::make(N, W, P);
   if (budget_ && in_use_ + lay.total > budget_)
     return fail(CKT_ERR_BUDGET, "circuit needs " + std::to_string(lay.total) +
                                     " bytes; budget has " + std::to_string(budget_ - in_use_) + " left");
-  if (plan.wire_state.size() != plan.W) return fail(CKT_ERR_INVALID_ARG, "incomplete generator plan");
-  const size_t need = devgen_scratch_bytes(plan.N, plan.W);
+  const size_t need = devgen_scratch_bytes(N, W);
   if (need == 0) return fail(CKT_ERR_HIP, "device generator scratch size query failed");
   if (need > devgen_scratch_cap_) {
     // Builds already enqueued use the old scratch.
@@ -1172,25 +1191,20 @@ int Engine::add_planned(const DevgenPlan& plan, int32_t loops, uint32_t* id) {
     CKT_HIP(hipMalloc(&devgen_scratch_, need));
     devgen_scratch_cap_ = need;
   }
-  void* staged = nullptr;
-  int st;
-  if (plan.W && (st = stage(plan.wire_state.data(), (size_t)plan.W * sizeof(uint64_t), &staged)))
-    return st;
   // From the stream's memory pool: allocated and, at removal, released in
   // stream order, without waiting for the device.
   void* slab = nullptr;
   hipError_t e = pool_ok_ ? hipMallocAsync(&slab, lay.total, stream_) : hipMalloc(&slab, lay.total);
   if (e != hipSuccess) return hip_fail(e, "allocating a circuit");
   std::vector<ckt_piece_t> pieces;
-  if ((st = devgen_enqueue(plan, (const uint64_t*)staged, lay, slab, devgen_scratch_, stream_,
-                           pieces))) {
+  if ((st = devgen_enqueue(params, lay, slab, devgen_scratch_, stream_, pieces))) {
     (void)hipStreamSynchronize(stream_);
     if (pool_ok_) (void)hipFreeAsync(slab, stream_);
     else (void)hipFree(slab);
     (void)hipStreamSynchronize(stream_);
     return st;
   }
-  attach(slab, lay, plan.N, plan.W, plan.P, pieces, loops, id, pool_ok_);
+  attach(slab, lay, N, W, P, pieces, loops, id, pool_ok_);
   return CKT_OK;
 }
 

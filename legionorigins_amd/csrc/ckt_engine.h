@@ -47,26 +47,12 @@ int image_from_aos(SlabImage& img, const ckt_node_t* nodes, uint32_t N, const ck
 int image_from_gen(SlabImage& img, const ckt_gen_params_t* params);
 
 // Generates the circuit `params` describes straight into a device slab of
-// layout `L` (ckt_devgen.hip), bit-identical to image_from_gen; fills
-// `pieces`.  Synchronises `s` before returning.
-int devgen_build(const ckt_gen_params_t* params, const SlabLayout& L, void* slab, hipStream_t s,
-                 std::vector<ckt_piece_t>& pieces);
-
-// The host part of the device generator, done ahead of time (thread-safe):
-// every wire's drand48 state at its first draw.
-struct DevgenPlan {
-  ckt_gen_params_t params{};
-  uint32_t N = 0, W = 0, P = 0;
-  std::vector<uint64_t> wire_state;
-};
-int devgen_plan(const ckt_gen_params_t* params, DevgenPlan& plan);
-// Device scratch a planned build of N nodes and W wires needs.
+// layout `L` (ckt_devgen.hip), bit-identical to image_from_gen: enqueued on `s`
+// without waiting, with `scratch` (devgen_scratch_bytes) untouched by others
+// until `s` has run it.  Fills `pieces`.
 size_t devgen_scratch_bytes(uint32_t N, uint32_t W);
-// Enqueues the planned build on `s` without waiting: `staged_state` (pinned
-// host memory holding plan.wire_state) and `scratch` (devgen_scratch_bytes)
-// must stay untouched until `s` has run the enqueued work.  Fills `pieces`.
-int devgen_enqueue(const DevgenPlan& plan, const uint64_t* staged_state, const SlabLayout& L,
-                   void* slab, void* scratch, hipStream_t s, std::vector<ckt_piece_t>& pieces);
+int devgen_enqueue(const ckt_gen_params_t* params, const SlabLayout& L, void* slab, void* scratch,
+                   hipStream_t s, std::vector<ckt_piece_t>& pieces);
 
 struct Circuit {
   uint32_t id = 0;
@@ -124,11 +110,9 @@ class Engine {
                   const uint32_t* replaced, uint32_t* id);
   // Generates the circuit on the device (no host image, no upload).
   int add_generated_on_device(const ckt_gen_params_t* params, int32_t loops, uint32_t* id);
-  // Same circuit from a plan made earlier: the generation is only enqueued
-  // on the engine stream (after whatever runs there), nothing waits.  The
-  // plan's start states are copied into pinned staging memory that sync()
-  // recycles, so the plan may be dropped on return.
-  int add_planned(const DevgenPlan& plan, int32_t loops, uint32_t* id);
+  // The same, only enqueued on the engine stream (after whatever runs there)
+  // into a slab from the stream's memory pool: nothing waits.
+  int add_generated_async(const ckt_gen_params_t* params, int32_t loops, uint32_t* id);
   int remove(uint32_t id);
   int remove_many(const uint32_t* ids, size_t n);
   Circuit* find(uint32_t id);
@@ -153,7 +137,7 @@ class Engine {
   int upv(const std::vector<PieceRef>& refs);
   int sanity(const std::vector<PieceRef>& refs, uint64_t* bad);
   int nop();
-  // Waits for the engine stream; recycles the staging memory of planned adds.
+  // Waits for the engine stream; recycles the staging memory of tile lists.
   int sync();
 
   // One loop (cnc, dsc, upv) of `refs` captured in a graph and replayed
@@ -186,6 +170,10 @@ class Engine {
               bool stream_ordered = false);
   static DevCircuit device_view(void* slab, const SlabLayout& L, uint32_t N, uint32_t W,
                                 uint32_t P);
+  // Scratch of `need` bytes for a build: the engine's own (grown, after the
+  // builds already enqueued) up to kKeepScratch, else, or where that fails, an
+  // allocation in *own that the caller frees; NULL if there is no memory.
+  int build_scratch(size_t need, void** scratch, void** own);
   // add_records' build into `slab`; `scratch` as record_scratch_bytes says.
   int build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, const int32_t* locator,
                     const ckt_piece_t* pieces, const DevCircuit& c, void* scratch);
@@ -257,9 +245,9 @@ class Engine {
   bool timing_ = false;
   std::vector<Pending> pending_;
   std::vector<hipEvent_t> event_pool_;
-  // Planned device generation: one device scratch (grow-only; the builds on
-  // the stream run one after another) and pinned staging chunks for the
-  // start states, recycled at sync().
+  // Device scratch of circuit builds (grow-only; the builds on the stream run
+  // one after another), and pinned staging chunks for tile lists and the
+  // descriptor table, recycled at sync().
   bool pool_ok_ = false;  // the device's default memory pool is usable
   void* devgen_scratch_ = nullptr;
   size_t devgen_scratch_cap_ = 0;

@@ -7,12 +7,9 @@
 //   arrival   -> FIFO queue
 //   admission -> when the HBM budget, the resident-circuit cap and the
 //                per-iteration wire cap allow, the request's device footprint
-//                is reserved and a host thread walks its generator chain
-//                (each wire's first drand48 state, 8 bytes per wire)
-//   generate  -> the device generator is enqueued behind the running
-//                iteration (the GPU draws the circuit in HBM; nothing is
-//                uploaded but the start states); the circuit joins the next
-//                iteration
+//                is reserved and the device generator is enqueued behind the
+//                running iteration (the GPU draws the circuit in HBM; nothing
+//                is uploaded); the circuit joins the next iteration
 //   iteration -> one loop (calc_new_currents, distribute_charge,
 //                update_voltages) of every resident circuit with loops left,
 //                each task one launch over all of them
@@ -46,7 +43,7 @@ using namespace ckt;
 
 namespace {
 
-enum RecState { kQueued = 0, kPlanning = 1, kResident = 2, kDone = 3 };
+enum RecState { kQueued = 0, kResident = 1, kDone = 2 };
 
 // One submitted request.  gen, loops, timeout_s, need and wires are fixed at
 // submission; the rest belongs to the scheduler thread and is read by other
@@ -79,7 +76,7 @@ struct ckt_server {
 
   // Shared with the scheduler thread, under mu.
   std::mutex mu;
-  std::condition_variable wake;      // scheduler: submissions, cancels, stop, finished plans
+  std::condition_variable wake;      // scheduler: submissions, cancels, stop
   std::condition_variable finished;  // ckt_server_wait
   uint64_t wake_seq = 0;
   std::deque<Rec> recs;              // by request id; references stay valid as it grows
@@ -109,76 +106,6 @@ double now_s() {
   clock_gettime(CLOCK_MONOTONIC, &t);
   return (double)t.tv_sec + 1e-9 * (double)t.tv_nsec;
 }
-
-struct Ready {
-  uint32_t id;
-  std::unique_ptr<DevgenPlan> plan;
-  int status;
-  std::string error;
-};
-
-// Host threads that walk admitted requests' generator chains; each finished
-// plan wakes the scheduler.
-class GenPool {
- public:
-  GenPool(int threads, ckt_server* s) : s_(s) {
-    for (int i = 0; i < threads; i++) th_.emplace_back([this] { work(); });
-  }
-  ~GenPool() {
-    {
-      std::lock_guard<std::mutex> g(mu_);
-      stop_ = true;
-    }
-    cv_.notify_all();
-    for (auto& t : th_) t.join();
-  }
-  void submit(uint32_t id, const ckt_gen_params_t& gen) {
-    {
-      std::lock_guard<std::mutex> g(mu_);
-      jobs_.emplace_back(id, gen);
-    }
-    cv_.notify_one();
-  }
-  void take(std::vector<Ready>& out) {
-    std::lock_guard<std::mutex> g(mu_);
-    for (auto& r : done_) out.push_back(std::move(r));
-    done_.clear();
-  }
-
- private:
-  void work() {
-    for (;;) {
-      std::pair<uint32_t, ckt_gen_params_t> job;
-      {
-        std::unique_lock<std::mutex> g(mu_);
-        cv_.wait(g, [this] { return stop_ || !jobs_.empty(); });
-        if (stop_) return;
-        job = jobs_.front();
-        jobs_.pop_front();
-      }
-      Ready r;
-      r.id = job.first;
-      r.plan.reset(new DevgenPlan());
-      r.status = devgen_plan(&job.second, *r.plan);
-      if (r.status) {
-        r.error = ckt_last_error();
-        r.plan.reset();
-      }
-      {
-        std::lock_guard<std::mutex> g(mu_);
-        done_.push_back(std::move(r));
-      }
-      s_->poke();
-    }
-  }
-  ckt_server* s_;
-  std::vector<std::thread> th_;
-  std::mutex mu_;
-  std::condition_variable cv_;
-  std::deque<std::pair<uint32_t, ckt_gen_params_t>> jobs_;
-  std::vector<Ready> done_;
-  bool stop_ = false;
-};
 
 // Grow-only pinned host buffer (device-to-host copies into it are
 // asynchronous); grown only when no copy into it is pending.
@@ -253,13 +180,11 @@ void schedule(ckt_server* s) {
   const ckt_server_config_t cfg = s->cfg;
   int st = CKT_OK;
   if (hipSetDevice(E.device()) != hipSuccess) st = fail(CKT_ERR_HIP, "server: hipSetDevice");
-  GenPool pool(cfg.gen_threads, s);
   std::deque<uint32_t> queue;       // arrived, not admitted
   uint64_t reserved = 0;            // bytes of admitted, not retired requests
   uint64_t admitted_wires = 0;      // wires of admitted, not retired requests
   int32_t admitted = 0;             // admitted, not retired requests
   std::vector<uint32_t> request_of_circuit;
-  std::vector<Ready> ready;
   std::vector<uint32_t> in_flight;  // requests advanced by the running iteration
   // Circuits finishing with an iteration, as (circuit id, offset in that
   // iteration's download buffer).  Two buffers alternate: the voltages of the
@@ -312,8 +237,6 @@ void schedule(ckt_server* s) {
     if (stop && !drain) {
       for (uint32_t id : queue) cancels.push_back(id);
       for (Circuit* c : E.slots()) cancels.push_back(request_of_circuit[c->id]);
-      for (uint32_t id = 0; id < recp.size(); id++)
-        if (recp[id] && rec(id).state == kPlanning) cancels.push_back(id);
     }
     for (uint32_t id : cancels) {
       Rec& r = rec(id);
@@ -323,8 +246,6 @@ void schedule(ckt_server* s) {
           queue.erase(q);
           retire(id, CKT_ERR_CANCELLED, 0);
         }
-      } else if (r.state == kPlanning) {
-        r.cancel = true;  // retired when its plan comes back
       } else if (r.state == kResident && !r.cancel) {
         // Leaves before the next iteration, unless its last one has run.
         Circuit* c = E.find(r.circuit);
@@ -438,15 +359,23 @@ void schedule(ckt_server* s) {
       reserved += r.need;
       admitted_wires += r.wires;
       admitted++;
-      {
-        std::lock_guard<std::mutex> g(s->mu);
-        rec(i).state = kPlanning;
+      // Its generation is enqueued behind the running iteration.
+      uint32_t id = 0;
+      if (int as = E.add_generated_async(&r.gen, r.loops, &id)) {
+        release(i);
+        retire(i, as, 0);
+        continue;
       }
-      pool.submit(i, r.gen);
+      if (request_of_circuit.size() <= id) request_of_circuit.resize(id + 1, 0);
+      request_of_circuit[id] = i;
+      std::lock_guard<std::mutex> g(s->mu);
+      rec(i).circuit = id;
+      rec(i).state = kResident;
+      rec(i).res.admit_s = clock();
     }
     // With nothing on the GPU, sleep until something changes: a submission,
-    // a cancel, a stop, a finished plan or the next admission deadline.
-    if (refs.empty()) {
+    // a cancel, a stop or the next admission deadline.
+    if (refs.empty() && E.count() == 0) {
       std::unique_lock<std::mutex> g(s->mu);
       const bool idle_done = s->stop && queue.empty() && admitted == 0 && E.count() == 0 &&
                              s->incoming.empty();
@@ -454,32 +383,6 @@ void schedule(ckt_server* s) {
       const double wait = std::max(0.0, std::min(0.05, next_deadline - clock()));
       s->wake.wait_for(g, std::chrono::duration<double>(wait),
                        [&] { return s->wake_seq != seen; });
-    }
-    // Overlap: enqueue the generation of planned circuits behind the
-    // running iteration.
-    ready.clear();
-    pool.take(ready);
-    for (Ready& r : ready) {
-      Rec& q = rec(r.id);
-      if (q.cancel || r.status) {
-        release(r.id);
-        retire(r.id, q.cancel ? CKT_ERR_CANCELLED : r.status, 0);
-        continue;
-      }
-      uint32_t id = 0;
-      int as = E.add_planned(*r.plan, q.loops, &id);
-      r.plan.reset();
-      if (as) {
-        release(r.id);
-        retire(r.id, as, 0);
-        continue;
-      }
-      if (request_of_circuit.size() <= id) request_of_circuit.resize(id + 1, 0);
-      request_of_circuit[id] = r.id;
-      q.circuit = id;
-      std::lock_guard<std::mutex> g(s->mu);
-      q.state = kResident;
-      q.res.admit_s = clock();
     }
     s->max_resident = std::max<int32_t>(s->max_resident, (int32_t)E.count());
     if (!refs.empty()) {
@@ -563,7 +466,6 @@ int ckt_server_create(int device, const ckt_server_config_t* config, ckt_server_
     return fail(CKT_ERR_INVALID_ARG, "server: unknown policy");
   if (cfg.reduce_mode < CKT_REDUCE_ATOMIC || cfg.reduce_mode > CKT_REDUCE_CSR_KAHAN64)
     return fail(CKT_ERR_INVALID_ARG, "server: unknown reduction mode");
-  if (cfg.gen_threads <= 0) cfg.gen_threads = 8;
   ckt_server_t* s = new ckt_server_t();
   int st = s->eng.init(device, cfg.hbm_budget_bytes);
   if (st) {
