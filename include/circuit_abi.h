@@ -221,10 +221,10 @@ int ckt_sanity_check_wires_gpu(const ckt_piece_t* piece, const ckt_wire_t* wires
  * (circuit.cc:250-251,276-277,298-299) on the same instances, with the
  * results of one call per piece in piece order (distribute_charge's float
  * atomics aside, whose order is unspecified in either form) and one wait at
- * the end.  The per-piece calls are this form with a table of one.  Each
- * call allocates a few bytes of device scratch per piece (the piece table and
- * a bad-record counter) from the stream-ordered allocator on `stream` and
- * releases it before returning. */
+ * the end.  The per-piece calls are this form with a table of one.  A call
+ * over more than 64 pieces allocates a few bytes of device scratch per piece
+ * (the piece table and a bad-record counter) from the stream-ordered allocator
+ * on `stream` and releases it before returning. */
 int ckt_calc_new_currents_index_gpu(const ckt_piece_t* pieces, uint32_t num_pieces,
                                     ckt_wire_t* wires, const ckt_node_t* pvt,
                                     const ckt_node_t* owned, const ckt_node_t* ghost, int flag,

@@ -111,15 +111,17 @@ static int run_indexed(const ckt_piece_t* pieces, uint32_t n, bool over_nodes, u
   uint32_t blocks = 0;
   int st = stage_index(pieces, n, over_nodes, image, &blocks);
   if (st) return st;
-  const PieceIndex ix{(const ckt_piece_t*)(dev + lay.pieces),
-                      (const uint32_t*)(dev + lay.first_block), n};
+  PieceArgs ix;
+  ix.ix = PieceIndex{(const ckt_piece_t*)(dev + lay.pieces),
+                     (const uint32_t*)(dev + lay.first_block), n};
+  ix.inlined = 0;
   unsigned long long* d_bad = (unsigned long long*)dev;
   unsigned long long h_bad = 0;
   hipError_t e = hipMemcpyAsync(dev, image, 4 * ((size_t)n + 5), hipMemcpyHostToDevice, s);
   if (e == hipSuccess)
     e = hipMemcpyAsync(dev + lay.pieces, pieces, sizeof(ckt_piece_t) * n, hipMemcpyHostToDevice,
                        s);
-  if (e == hipSuccess) e = launch(ix, blocks, d_bad);
+  if (e == hipSuccess) e = launch(ix, blocks, BadRecords{d_bad, nullptr});
   if (e == hipSuccess && nbad)
     e = hipMemcpyAsync(&h_bad, d_bad, sizeof(h_bad), hipMemcpyDeviceToHost, s);
   // The copies read and write host memory the caller owns: wait in every case.
@@ -130,13 +132,94 @@ static int run_indexed(const ckt_piece_t* pieces, uint32_t n, bool over_nodes, u
   return CKT_OK;
 }
 
+// Flags in pinned host memory for launches that report invalid records: one
+// page for the process, a word to a call while it runs, 64 bytes apart.
+class FlagPool {
+ public:
+  // A cleared word, or NULL if there is none.
+  uint32_t* take() {
+    std::lock_guard<std::mutex> g(mu_);
+    if (!page_ && !failed_) {
+      void* p = nullptr;
+      failed_ = hipHostMalloc(&p, 64 * kWords, hipHostMallocPortable) != hipSuccess;
+      if (failed_) (void)hipGetLastError();
+      else page_ = (uint32_t*)p;
+    }
+    if (!page_ || !~used_) return nullptr;
+    const int k = __builtin_ctzll(~used_);
+    used_ |= 1ull << k;
+    uint32_t* w = page_ + 16 * k;
+    __atomic_store_n(w, 0u, __ATOMIC_RELEASE);
+    return w;
+  }
+  void give(uint32_t* w) {
+    std::lock_guard<std::mutex> g(mu_);
+    used_ &= ~(1ull << ((w - page_) / 16));
+  }
+
+ private:
+  static constexpr int kWords = 64;
+  std::mutex mu_;
+  uint32_t* page_ = nullptr;
+  uint64_t used_ = 0;
+  bool failed_ = false;
+};
+static FlagPool g_flags;
+
+// One accessor-form task over a table of up to kInlinePieces pieces: the
+// table goes with the launch's arguments and invalid records raise a flag in
+// host memory, so that a call is a launch and a wait, without a copy or an
+// allocation (those made a call over one small piece take 46-55 us, a launch
+// and a wait take 15-26).  Only a raised flag makes a second launch, which
+// counts the records.  `wires` is NULL for a task that reports none.
+template <class Launch>
+static int run_inlined(const ckt_piece_t* pieces, uint32_t n, bool over_nodes, uint32_t* image,
+                       const ckt_wire_t* wires, hipStream_t s, const char* what, uint32_t* flag,
+                       uint64_t* nbad, Launch launch) {
+  uint32_t blocks = 0;
+  if (int st = stage_index(pieces, n, over_nodes, image, &blocks)) return st;
+  PieceArgs ix;
+  ix.ix = PieceIndex{nullptr, nullptr, 0};
+  ix.inlined = n;
+  std::copy(image + 4, image + 5 + n, ix.first_block);
+  std::copy(pieces, pieces + n, ix.pieces);
+  const hipError_t e = launch(ix, blocks, BadRecords{nullptr, flag});
+  const hipError_t w = hipStreamSynchronize(s);
+  if (e != hipSuccess) return hip_fail(e, what);
+  if (w != hipSuccess) return hip_fail(w, what);
+  if (!wires || !__atomic_load_n(flag, __ATOMIC_ACQUIRE)) return CKT_OK;
+  unsigned long long* d_bad = nullptr;
+  unsigned long long h_bad = 0;
+  CKT_HIP(hipMallocAsync((void**)&d_bad, sizeof(*d_bad), s));
+  hipError_t c = hipMemcpyAsync(d_bad, &h_bad, sizeof(h_bad), hipMemcpyHostToDevice, s);
+  if (c == hipSuccess) c = launch_count_bad(ix, blocks, wires, d_bad, s);
+  if (c == hipSuccess) c = hipMemcpyAsync(&h_bad, d_bad, sizeof(h_bad), hipMemcpyDeviceToHost, s);
+  const hipError_t f = hipFreeAsync(d_bad, s);
+  const hipError_t y = hipStreamSynchronize(s);
+  for (hipError_t x : {c, f, y})
+    if (x != hipSuccess) return hip_fail(x, what);
+  *nbad = h_bad;
+  return CKT_OK;
+}
+
+// One accessor-form task: run_inlined where the table is short, else
 // run_indexed with its scratch from the stream-ordered allocator, released
 // behind the call.
 template <class Launch>
-static int run_indexed_alloc(const ckt_piece_t* pieces, uint32_t n, bool over_nodes, hipStream_t s,
-                             const char* what, uint64_t* nbad, Launch launch) {
+static int run_indexed_alloc(const ckt_piece_t* pieces, uint32_t n, bool over_nodes,
+                             const ckt_wire_t* wires, hipStream_t s, const char* what,
+                             uint64_t* nbad, Launch launch) {
   std::vector<uint32_t> image((size_t)n + 5);
   if (int st = check_disjoint(pieces, n, over_nodes, image.data(), what)) return st;
+  if (n >= 1 && n <= kInlinePieces) {
+    uint32_t* flag = wires ? g_flags.take() : nullptr;
+    if (flag || !wires) {
+      const int st = run_inlined(pieces, n, over_nodes, image.data(), wires, s, what, flag, nbad,
+                                 launch);
+      if (flag) g_flags.give(flag);
+      return st;
+    }
+  }
   unsigned char* dev = nullptr;
   CKT_HIP(hipMallocAsync((void**)&dev, IndexLayout(n).bytes, s));
   const int st = run_indexed(pieces, n, over_nodes, dev, image.data(), s, what, nbad, launch);
@@ -275,8 +358,8 @@ int ckt_calc_new_currents_index_gpu(const ckt_piece_t* pieces, uint32_t num_piec
     return fail(CKT_ERR_INVALID_ARG, "calc_new_currents: flag is not a CKT_POLICY_*");
   hipStream_t s = (hipStream_t)stream;
   uint64_t nbad = 0;
-  int st = run_indexed_alloc(pieces, num_pieces, false, s, what, &nbad,
-                             [&](const PieceIndex& ix, uint32_t blocks, unsigned long long* bad) {
+  int st = run_indexed_alloc(pieces, num_pieces, false, wires, s, what, &nbad,
+                             [&](const PieceArgs& ix, uint32_t blocks, const BadRecords& bad) {
                                return launch_cnc_aos(flag, ix, blocks, wires, pvt, owned, ghost,
                                                      CKT_STEPS, bad, s);
                              });
@@ -305,7 +388,7 @@ int ckt_calc_new_currents_index_gpu_noalloc(const ckt_piece_t* pieces, uint32_t 
   hipStream_t s = (hipStream_t)stream;
   uint64_t nbad = 0;
   int st = run_indexed(pieces, num_pieces, false, dev, image, s, what, &nbad,
-                       [&](const PieceIndex& ix, uint32_t blocks, unsigned long long* bad) {
+                       [&](const PieceArgs& ix, uint32_t blocks, const BadRecords& bad) {
                          return launch_cnc_aos(flag, ix, blocks, wires, pvt, owned, ghost,
                                                CKT_STEPS, bad, s);
                        });
@@ -329,8 +412,8 @@ int ckt_distribute_charge_index_gpu(const ckt_piece_t* pieces, uint32_t num_piec
   if (flag != 0) return fail(CKT_ERR_INVALID_ARG, "distribute_charge: flag must be 0");
   hipStream_t s = (hipStream_t)stream;
   uint64_t nbad = 0;
-  int st = run_indexed_alloc(pieces, num_pieces, false, s, what, &nbad,
-                             [&](const PieceIndex& ix, uint32_t blocks, unsigned long long* bad) {
+  int st = run_indexed_alloc(pieces, num_pieces, false, wires, s, what, &nbad,
+                             [&](const PieceArgs& ix, uint32_t blocks, const BadRecords& bad) {
                                return launch_dsc_aos(ix, blocks, wires, pvt, owned_fold,
                                                      ghost_fold, bad, s);
                              });
@@ -353,8 +436,8 @@ int ckt_update_voltages_index_gpu(const ckt_piece_t* pieces, uint32_t num_pieces
   if (int st = check_pieces(pieces, num_pieces, what)) return st;
   if (flag != 0) return fail(CKT_ERR_INVALID_ARG, "update_voltages: flag must be 0");
   hipStream_t s = (hipStream_t)stream;
-  return run_indexed_alloc(pieces, num_pieces, true, s, what, nullptr,
-                           [&](const PieceIndex& ix, uint32_t blocks, unsigned long long*) {
+  return run_indexed_alloc(pieces, num_pieces, true, nullptr, s, what, nullptr,
+                           [&](const PieceArgs& ix, uint32_t blocks, const BadRecords&) {
                              return launch_upv_aos(ix, blocks, pvt, owned, locator, s);
                            });
 }

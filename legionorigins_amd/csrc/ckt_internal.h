@@ -99,15 +99,35 @@ struct PieceIndex {
   uint32_t num_pieces;
 };
 
+// The piece table as a kernel argument: tables of up to kInlinePieces by
+// value (no copy to the device goes before the launch), longer ones by `ix`.
+constexpr uint32_t kInlinePieces = 64;
+struct PieceArgs {
+  PieceIndex ix;
+  uint32_t inlined;  // pieces below, 0 if `ix` holds the table
+  uint32_t first_block[kInlinePieces + 1];
+  ckt_piece_t pieces[kInlinePieces];
+};
+
+// Where a launch reports records with an invalid PointerLocation: a counter
+// in device memory, or, if that is NULL, a flag in pinned host memory.
+struct BadRecords {
+  unsigned long long* count;
+  uint32_t* flag;
+};
+
 // Accessor-form (reference AoS layout) launchers over a piece table;
-// `blocks` = first_block[num_pieces].
-hipError_t launch_cnc_aos(int policy, const PieceIndex& ix, uint32_t blocks, ckt_wire_t* wires,
+// `blocks` is its workgroup count.
+hipError_t launch_cnc_aos(int policy, const PieceArgs& ix, uint32_t blocks, ckt_wire_t* wires,
                           const ckt_node_t* pvt, const ckt_node_t* owned, const ckt_node_t* ghost,
-                          int steps, unsigned long long* bad, hipStream_t s);
-hipError_t launch_dsc_aos(const PieceIndex& ix, uint32_t blocks, const ckt_wire_t* wires,
+                          int steps, const BadRecords& bad, hipStream_t s);
+hipError_t launch_dsc_aos(const PieceArgs& ix, uint32_t blocks, const ckt_wire_t* wires,
                           ckt_node_t* pvt, float* owned_fold, float* ghost_fold,
-                          unsigned long long* bad, hipStream_t s);
-hipError_t launch_upv_aos(const PieceIndex& ix, uint32_t blocks, ckt_node_t* pvt,
+                          const BadRecords& bad, hipStream_t s);
+// Adds to *bad the wires that the two above report.
+hipError_t launch_count_bad(const PieceArgs& ix, uint32_t blocks, const ckt_wire_t* wires,
+                            unsigned long long* bad, hipStream_t s);
+hipError_t launch_upv_aos(const PieceArgs& ix, uint32_t blocks, ckt_node_t* pvt,
                           ckt_node_t* owned, const int32_t* locator, hipStream_t s);
 hipError_t launch_sanity_aos(const ckt_piece_t piece, const ckt_wire_t* wires,
                              uint32_t num_nodes_total, unsigned long long* bad, hipStream_t s);

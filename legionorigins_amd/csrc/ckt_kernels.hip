@@ -1411,27 +1411,36 @@ __device__ __forceinline__ const ckt_node_t* pick_instance(int32_t loc, const ck
 // The accessor-form kernels run over a piece table (an index-space launch;
 // a per-piece call is a table of one).  Workgroups are numbered across the
 // pieces: piece p owns workgroups [first_block[p], first_block[p + 1]), each
-// covering 256 consecutive elements (wires or nodes) of it.
-__device__ __forceinline__ uint32_t piece_of_block(const PieceIndex& ix, uint32_t b,
-                                                   uint32_t* elem) {
-  return piece_of_block(ix.first_block, ix.num_pieces, b, threadIdx.x, elem);
+// covering 256 consecutive elements (wires or nodes) of it.  Returns the piece
+// of workgroup b, from the launch's arguments or from the table in memory.
+__device__ __forceinline__ ckt_piece_t piece_of_block(const PieceArgs& a, uint32_t b,
+                                                      uint32_t* elem) {
+  if (a.inlined) return a.pieces[piece_of_block(a.first_block, a.inlined, b, threadIdx.x, elem)];
+  return a.ix.pieces[piece_of_block(a.ix.first_block, a.ix.num_pieces, b, threadIdx.x, elem)];
+}
+
+// A record with an invalid PointerLocation: counted, or only flagged in host
+// memory (a plain store: the bus need not carry atomics).
+__device__ __forceinline__ void report_bad(const BadRecords& bad) {
+  if (bad.count) atomicAdd(bad.count, 1ull);
+  else __hip_atomic_store(bad.flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <int POLICY>
-__global__ __launch_bounds__(256) void cnc_aos_kernel(PieceIndex ix, ckt_wire_t* __restrict__ wires,
+__global__ __launch_bounds__(256) void cnc_aos_kernel(PieceArgs ix, ckt_wire_t* __restrict__ wires,
                                                       const ckt_node_t* pvt, const ckt_node_t* owned,
                                                       const ckt_node_t* ghost, int steps,
-                                                      unsigned long long* bad) {
+                                                      BadRecords bad) {
   __shared__ float snap[kSeg * 256];
   const Settle st((lfloat*)snap + threadIdx.x, 256);
   uint32_t k;
-  const ckt_piece_t p = ix.pieces[piece_of_block(ix, blockIdx.x, &k)];
+  const ckt_piece_t p = piece_of_block(ix, blockIdx.x, &k);
   if (k >= p.num_wires) return;
   ckt_wire_t& wire = wires[p.first_wire + k];
   const ckt_node_t* in_base = pick_instance(wire.in_loc, pvt, owned, ghost);
   const ckt_node_t* out_base = pick_instance(wire.out_loc, pvt, owned, ghost);
   if (!in_base || !out_base) {
-    atomicAdd(bad, 1ull);
+    report_bad(bad);
     return;
   }
   float I[kSeg], V[kSeg - 1];
@@ -1458,26 +1467,37 @@ __device__ __forceinline__ bool reduce_local(int32_t loc, uint32_t ptr, float v,
   }
 }
 
-__global__ __launch_bounds__(256) void dsc_aos_kernel(PieceIndex ix,
+__global__ __launch_bounds__(256) void dsc_aos_kernel(PieceArgs ix,
                                                       const ckt_wire_t* __restrict__ wires,
                                                       ckt_node_t* pvt, float* owned_fold,
-                                                      float* ghost_fold, unsigned long long* bad) {
+                                                      float* ghost_fold, BadRecords bad) {
   uint32_t k;
-  const ckt_piece_t p = ix.pieces[piece_of_block(ix, blockIdx.x, &k)];
+  const ckt_piece_t p = piece_of_block(ix, blockIdx.x, &k);
   if (k >= p.num_wires) return;
   const ckt_wire_t& wire = wires[p.first_wire + k];
   const float dt = CKT_DT_F;
   bool ok = reduce_local(wire.in_loc, wire.in_ptr, -dt * wire.current[0], pvt, owned_fold, ghost_fold);
   ok = reduce_local(wire.out_loc, wire.out_ptr, dt * wire.current[kSeg - 1], pvt, owned_fold,
                     ghost_fold) && ok;
-  if (!ok) atomicAdd(bad, 1ull);
+  if (!ok) report_bad(bad);
 }
 
-__global__ __launch_bounds__(256) void upv_aos_kernel(PieceIndex ix, ckt_node_t* pvt,
+// The wires that either kernel above reports.
+__global__ __launch_bounds__(256) void count_bad_kernel(PieceArgs ix,
+                                                        const ckt_wire_t* __restrict__ wires,
+                                                        unsigned long long* bad) {
+  uint32_t k;
+  const ckt_piece_t p = piece_of_block(ix, blockIdx.x, &k);
+  if (k >= p.num_wires) return;
+  const ckt_wire_t& wire = wires[p.first_wire + k];
+  if ((uint32_t)wire.in_loc > 2u || (uint32_t)wire.out_loc > 2u) atomicAdd(bad, 1ull);
+}
+
+__global__ __launch_bounds__(256) void upv_aos_kernel(PieceArgs ix, ckt_node_t* pvt,
                                                       ckt_node_t* owned,
                                                       const int32_t* __restrict__ locator) {
   uint32_t k;
-  const ckt_piece_t p = ix.pieces[piece_of_block(ix, blockIdx.x, &k)];
+  const ckt_piece_t p = piece_of_block(ix, blockIdx.x, &k);
   if (k >= p.num_nodes) return;
   const uint32_t i = p.first_node + k;
   ckt_node_t& nd = locator[i] ? pvt[i] : owned[i];
@@ -1685,9 +1705,9 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_cnc_aos(int policy, const PieceIndex& ix, uint32_t blocks, ckt_wire_t* wires,
+hipError_t launch_cnc_aos(int policy, const PieceArgs& ix, uint32_t blocks, ckt_wire_t* wires,
                           const ckt_node_t* pvt, const ckt_node_t* owned, const ckt_node_t* ghost,
-                          int steps, unsigned long long* bad, hipStream_t s) {
+                          int steps, const BadRecords& bad, hipStream_t s) {
   if (blocks == 0) return hipSuccess;
   const dim3 g(blocks), b(256);
   switch (policy) {
@@ -1708,16 +1728,23 @@ hipError_t launch_cnc_aos(int policy, const PieceIndex& ix, uint32_t blocks, ckt
   return hipGetLastError();
 }
 
-hipError_t launch_dsc_aos(const PieceIndex& ix, uint32_t blocks, const ckt_wire_t* wires,
+hipError_t launch_count_bad(const PieceArgs& ix, uint32_t blocks, const ckt_wire_t* wires,
+                            unsigned long long* bad, hipStream_t s) {
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(count_bad_kernel, dim3(blocks), dim3(256), 0, s, ix, wires, bad);
+  return hipGetLastError();
+}
+
+hipError_t launch_dsc_aos(const PieceArgs& ix, uint32_t blocks, const ckt_wire_t* wires,
                           ckt_node_t* pvt, float* owned_fold, float* ghost_fold,
-                          unsigned long long* bad, hipStream_t s) {
+                          const BadRecords& bad, hipStream_t s) {
   if (blocks == 0) return hipSuccess;
   hipLaunchKernelGGL(dsc_aos_kernel, dim3(blocks), dim3(256), 0, s, ix, wires, pvt, owned_fold,
                      ghost_fold, bad);
   return hipGetLastError();
 }
 
-hipError_t launch_upv_aos(const PieceIndex& ix, uint32_t blocks, ckt_node_t* pvt,
+hipError_t launch_upv_aos(const PieceArgs& ix, uint32_t blocks, ckt_node_t* pvt,
                           ckt_node_t* owned, const int32_t* locator, hipStream_t s) {
   if (blocks == 0) return hipSuccess;
   hipLaunchKernelGGL(upv_aos_kernel, dim3(blocks), dim3(256), 0, s, ix, pvt, owned, locator);
