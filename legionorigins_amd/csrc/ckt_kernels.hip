@@ -1294,6 +1294,8 @@ __global__ __launch_bounds__(256) void dsc_csr_kernel(const DevCircuit* __restri
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) v4f gv4f;
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(1))) v2f gv2f;
 
 template <bool NT>
 __device__ __forceinline__ v4f load4(const gv4f* p) {
@@ -1426,6 +1428,11 @@ __device__ __forceinline__ void report_bad(const BadRecords& bad) {
   else __hip_atomic_store(bad.flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// A lane takes one record.  With 128-byte records every access of a wave goes
+// to 64 lines, so what counts is how many accesses there are: seven of 16 bytes
+// read a record's 26 words and seven of 4 to 16 write the 19 that change, where
+// one per word took 45 (64 x 16384 wires: 96 us for the call, 82 so).
+// Instances that do not start on a 16-byte boundary go word by word.
 template <int POLICY>
 __global__ __launch_bounds__(256) void cnc_aos_kernel(PieceArgs ix, ckt_wire_t* __restrict__ wires,
                                                       const ckt_node_t* pvt, const ckt_node_t* owned,
@@ -1436,25 +1443,48 @@ __global__ __launch_bounds__(256) void cnc_aos_kernel(PieceArgs ix, ckt_wire_t* 
   uint32_t k;
   const ckt_piece_t p = piece_of_block(ix, blockIdx.x, &k);
   if (k >= p.num_wires) return;
-  ckt_wire_t& wire = wires[p.first_wire + k];
-  const ckt_node_t* in_base = pick_instance(wire.in_loc, pvt, owned, ghost);
-  const ckt_node_t* out_base = pick_instance(wire.out_loc, pvt, owned, ghost);
+  constexpr uint32_t kCur = 6, kCap = 16, kVol = 17, kEnd = 26;  // words of ckt_wire_t
+  gfloat* io = (gfloat*)(float*)(wires + p.first_wire + k);
+  const bool aligned = ((uintptr_t)wires & 15u) == 0;
+  float r[28];
+  if (aligned) {
+#pragma unroll
+    for (uint32_t i = 0; i < 28; i += 4) {
+      const v4f v = *(const gv4f*)(io + i);
+      r[i] = v.x, r[i + 1] = v.y, r[i + 2] = v.z, r[i + 3] = v.w;
+    }
+  } else {
+#pragma unroll
+    for (uint32_t i = 0; i < kEnd; i++) r[i] = io[i];
+  }
+  const ckt_node_t* in_base = pick_instance((int32_t)__float_as_uint(r[2]), pvt, owned, ghost);
+  const ckt_node_t* out_base = pick_instance((int32_t)__float_as_uint(r[3]), pvt, owned, ghost);
   if (!in_base || !out_base) {
     report_bad(bad);
     return;
   }
   float I[kSeg], V[kSeg - 1];
 #pragma unroll
-  for (int s = 0; s < kSeg; s++) I[s] = wire.current[s];
+  for (int s = 0; s < kSeg; s++) I[s] = r[kCur + s];
 #pragma unroll
-  for (int s = 0; s < kSeg - 1; s++) V[s] = wire.voltage[s];
-  const float vin = in_base[wire.in_ptr].voltage, vout = out_base[wire.out_ptr].voltage;
-  Relax<POLICY>::run(I, V, vin, vout, wire.inductance, wire.resistance, wire.capacitance, steps,
-                     st);
+  for (int s = 0; s < kSeg - 1; s++) V[s] = r[kVol + s];
+  const float vin = in_base[__float_as_uint(r[0])].voltage;
+  const float vout = out_base[__float_as_uint(r[1])].voltage;
+  Relax<POLICY>::run(I, V, vin, vout, r[4], r[5], r[kCap], steps, st);
+  if (aligned) {
+    *(gv2f*)(io + 6) = (v2f){I[0], I[1]};
+    *(gv4f*)(io + 8) = (v4f){I[2], I[3], I[4], I[5]};
+    *(gv4f*)(io + 12) = (v4f){I[6], I[7], I[8], I[9]};
+    io[17] = V[0];
+    *(gv2f*)(io + 18) = (v2f){V[1], V[2]};
+    *(gv4f*)(io + 20) = (v4f){V[3], V[4], V[5], V[6]};
+    *(gv2f*)(io + 24) = (v2f){V[7], V[8]};
+  } else {
 #pragma unroll
-  for (int s = 0; s < kSeg; s++) wire.current[s] = I[s];
+    for (int s = 0; s < kSeg; s++) io[kCur + s] = I[s];
 #pragma unroll
-  for (int s = 0; s < kSeg - 1; s++) wire.voltage[s] = V[s];
+    for (int s = 0; s < kSeg - 1; s++) io[kVol + s] = V[s];
+  }
 }
 
 __device__ __forceinline__ bool reduce_local(int32_t loc, uint32_t ptr, float v, ckt_node_t* pvt,
