@@ -258,6 +258,49 @@ static int noalloc_scratch(unsigned char** out) {
   return CKT_OK;
 }
 
+// Whether distribute_charge sums pieces' nodes in LDS, and how: `splits`
+// workgroups per piece (0: atomics per contribution), rows of `stride` nodes,
+// `bytes` of partial sums.
+//   Float atomics to memory complete ~21 a ns over the device, so a table of W
+// wires takes W / 10.5 ns with one per contribution: 429 us for a call over 64 x
+// 65536 wires, 168 with the LDS form, 121 and 62 for 64 x 16384.  The
+// LDS form has two launches, and an atomic per node with a contribution, so it
+// wants large tables with several wires per node; its two sums per node have
+// to fit in LDS, and the rows in 64 MiB.
+struct ChargePlan {
+  uint32_t splits = 0, stride = 0;
+  size_t bytes = 0;
+};
+static ChargePlan charge_plan(const ckt_piece_t* pieces, uint32_t n) {
+  ChargePlan plan;
+  uint64_t wires = 0, nodes = 0;
+  uint32_t most_wires = 0, most = 0;
+  for (uint32_t i = 0; i < n; i++) {
+    wires += pieces[i].num_wires;
+    nodes += pieces[i].num_nodes;
+    most_wires = std::max(most_wires, pieces[i].num_wires);
+    most = std::max(most, pieces[i].num_nodes);
+  }
+  if (wires < (1u << 18) || n > 0xffffu || most == 0 || 8ull * most > 160u * 1024u) return plan;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return plan;
+  }
+  // One workgroup per CU, two where their sums fit beside each other, none
+  // with under 2048 wires, 16 per piece at most.
+  const uint64_t want = (8ull * most <= 80u * 1024u ? 2u : 1u) * (uint64_t)cus;
+  const uint32_t splits = (uint32_t)std::max<uint64_t>(
+      1, std::min<uint64_t>({(want + n - 1) / n, most_wires / 2048u, 16u}));
+  const uint64_t sums = 2ull * most * splits * n;
+  if (sums > 4 * wires || 4 * sums > (64u << 20) || nodes > wires) return plan;
+  plan.splits = splits;
+  plan.stride = most;
+  plan.bytes = 4 * sums;
+  return plan;
+}
+
 static int check_pieces(const ckt_piece_t* pieces, uint32_t n, const char* what) {
   if (!pieces && n) return fail(CKT_ERR_INVALID_ARG, std::string(what) + ": null piece table");
   return CKT_OK;
@@ -412,11 +455,23 @@ int ckt_distribute_charge_index_gpu(const ckt_piece_t* pieces, uint32_t num_piec
   if (flag != 0) return fail(CKT_ERR_INVALID_ARG, "distribute_charge: flag must be 0");
   hipStream_t s = (hipStream_t)stream;
   uint64_t nbad = 0;
-  int st = run_indexed_alloc(pieces, num_pieces, false, wires, s, what, &nbad,
-                             [&](const PieceArgs& ix, uint32_t blocks, const BadRecords& bad) {
-                               return launch_dsc_aos(ix, blocks, wires, pvt, owned_fold,
-                                                     ghost_fold, bad, s);
-                             });
+  ChargePlan plan = charge_plan(pieces, num_pieces);
+  float* partial = nullptr;
+  if (plan.splits && hipMallocAsync((void**)&partial, plan.bytes, s) != hipSuccess) {
+    (void)hipGetLastError();
+    partial = nullptr;
+  }
+  int st = run_indexed_alloc(
+      pieces, num_pieces, false, wires, s, what, &nbad,
+      [&](const PieceArgs& ix, uint32_t blocks, const BadRecords& bad) {
+        return partial ? launch_dsc_aos_lds(ix, num_pieces, plan.splits, wires, pvt, owned_fold,
+                                            ghost_fold, partial, plan.stride, bad, s)
+                       : launch_dsc_aos(ix, blocks, wires, pvt, owned_fold, ghost_fold, bad, s);
+      });
+  if (partial) {
+    const hipError_t e = hipFreeAsync(partial, s);
+    if (!st && e != hipSuccess) st = hip_fail(e, what);
+  }
   return st ? st : bad_locations(nbad, what);
 }
 

@@ -124,7 +124,15 @@ hipError_t launch_cnc_aos(int policy, const PieceArgs& ix, uint32_t blocks, ckt_
 hipError_t launch_dsc_aos(const PieceArgs& ix, uint32_t blocks, const ckt_wire_t* wires,
                           ckt_node_t* pvt, float* owned_fold, float* ghost_fold,
                           const BadRecords& bad, hipStream_t s);
-// Adds to *bad the wires that the two above report.
+// The same with the n pieces' own nodes summed in LDS, `splits` workgroups per
+// piece; `stride` is the largest node count and `partial` holds n x splits rows
+// of 2 x stride floats.
+hipError_t launch_dsc_aos_lds(const PieceArgs& ix, uint32_t n, uint32_t splits,
+                              const ckt_wire_t* wires, ckt_node_t* pvt, float* owned_fold,
+                              float* ghost_fold, float* partial, uint32_t stride,
+                              const BadRecords& bad, hipStream_t s);
+// Adds to *bad the wires that the calc_new_currents and distribute_charge
+// launches report.
 hipError_t launch_count_bad(const PieceArgs& ix, uint32_t blocks, const ckt_wire_t* wires,
                             unsigned long long* bad, hipStream_t s);
 hipError_t launch_upv_aos(const PieceArgs& ix, uint32_t blocks, ckt_node_t* pvt,

@@ -1512,7 +1512,86 @@ __global__ __launch_bounds__(256) void dsc_aos_kernel(PieceArgs ix,
   if (!ok) report_bad(bad);
 }
 
-// The wires that either kernel above reports.
+// The same with a piece's own nodes summed in LDS.  Workgroup b takes wire
+// subrange b % splits (lds_subrange) of piece b / splits: contributions to the
+// piece's node range go to one of two LDS sums per node (private or shared),
+// all others to memory with atomics, and the sums are written as rows of
+// `partial` (`stride` private sums, then `stride` shared ones), which
+// dsc_aos_sum_kernel adds to the instances -- with atomics, because calls on
+// other streams may add to the same nodes.  Bound by the records: 64 bytes of
+// each cross the bus for the 24 in use.
+__global__ __launch_bounds__(1024) void dsc_aos_lds_kernel(PieceArgs ix, uint32_t splits,
+                                                           const ckt_wire_t* __restrict__ wires,
+                                                           ckt_node_t* pvt, float* owned_fold,
+                                                           float* ghost_fold, float* partial,
+                                                           uint32_t stride, BadRecords bad) {
+  extern __shared__ float acc[];
+  const uint32_t si = blockIdx.x % splits, pi = blockIdx.x / splits;
+  const ckt_piece_t p = ix.inlined ? ix.pieces[pi] : ix.ix.pieces[pi];
+  const uint32_t npp = p.num_nodes;
+  uint32_t k0, k1;
+  lds_subrange(p.num_wires, splits, si, &k0, &k1);
+  for (uint32_t i = threadIdx.x; i < 2 * npp; i += 1024) acc[i] = 0.f;
+  __syncthreads();
+  const float dt = CKT_DT_F;
+  const gfloat* base = (const gfloat*)(const float*)(wires + p.first_wire);
+  const bool aligned = ((uintptr_t)wires & 15u) == 0;
+  auto add = [&](uint32_t loc, uint32_t node, float q) {
+    const uint32_t l = node - p.first_node;
+    if (l < npp && loc == CKT_PRIVATE_PTR) atomicAdd(&acc[l], q);
+    else if (l < npp && loc == CKT_SHARED_PTR) atomicAdd(&acc[npp + l], q);
+    else return reduce_local((int32_t)loc, node, q, pvt, owned_fold, ghost_fold);
+    return true;
+  };
+  constexpr uint32_t kU = 4;
+  for (uint32_t first = k0 + threadIdx.x; first < k1; first += kU * 1024u) {
+    v4f head[kU];  // in_ptr, out_ptr, in_loc, out_loc
+    float q0[kU], q9[kU];
+#pragma unroll
+    for (uint32_t u = 0; u < kU; u++) {
+      const uint32_t k = first + u * 1024u;
+      const gfloat* r = base + (size_t)(k < k1 ? k : k0) * 32u;
+      if (aligned) head[u] = *(const gv4f*)r;
+      else head[u] = (v4f){r[0], r[1], r[2], r[3]};
+      q0[u] = -dt * r[6];
+      q9[u] = dt * r[15];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kU; u++) {
+      if (first + u * 1024u >= k1) break;
+      bool ok = add(__float_as_uint(head[u].z), __float_as_uint(head[u].x), q0[u]);
+      ok = add(__float_as_uint(head[u].w), __float_as_uint(head[u].y), q9[u]) && ok;
+      if (!ok) report_bad(bad);
+    }
+  }
+  __syncthreads();
+  float* row = partial + (size_t)blockIdx.x * 2u * stride;
+  for (uint32_t i = threadIdx.x; i < npp; i += 1024) {
+    row[i] = acc[i];
+    row[stride + i] = acc[npp + i];
+  }
+}
+
+// The rows of piece blockIdx.y added to its nodes.
+__global__ __launch_bounds__(256) void dsc_aos_sum_kernel(PieceArgs ix, uint32_t splits,
+                                                          ckt_node_t* pvt, float* owned_fold,
+                                                          const float* __restrict__ partial,
+                                                          uint32_t stride) {
+  const ckt_piece_t p = ix.inlined ? ix.pieces[blockIdx.y] : ix.ix.pieces[blockIdx.y];
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= p.num_nodes) return;
+  const float* row = partial + (size_t)blockIdx.y * splits * 2u * stride + i;
+  float a = 0.f, b = 0.f;
+  for (uint32_t s = 0; s < splits; s++, row += 2u * stride) {
+    a += row[0];
+    b += row[stride];
+  }
+  // a node without contributions is not touched
+  if (a != 0.f) unsafeAtomicAdd(&pvt[p.first_node + i].charge, a);
+  if (b != 0.f) unsafeAtomicAdd(&owned_fold[p.first_node + i], b);
+}
+
+// The wires that the kernels above report.
 __global__ __launch_bounds__(256) void count_bad_kernel(PieceArgs ix,
                                                         const ckt_wire_t* __restrict__ wires,
                                                         unsigned long long* bad) {
@@ -1771,6 +1850,23 @@ hipError_t launch_dsc_aos(const PieceArgs& ix, uint32_t blocks, const ckt_wire_t
   if (blocks == 0) return hipSuccess;
   hipLaunchKernelGGL(dsc_aos_kernel, dim3(blocks), dim3(256), 0, s, ix, wires, pvt, owned_fold,
                      ghost_fold, bad);
+  return hipGetLastError();
+}
+
+hipError_t launch_dsc_aos_lds(const PieceArgs& ix, uint32_t n, uint32_t splits,
+                              const ckt_wire_t* wires, ckt_node_t* pvt, float* owned_fold,
+                              float* ghost_fold, float* partial, uint32_t stride,
+                              const BadRecords& bad, hipStream_t s) {
+  // Allows dynamic LDS beyond the default limit where the runtime needs it.
+  (void)hipFuncSetAttribute((const void*)dsc_aos_lds_kernel,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(dsc_aos_lds_kernel, dim3(n * splits), dim3(1024), 8 * (size_t)stride, s, ix,
+                     splits, wires, pvt, owned_fold, ghost_fold, partial, stride, bad);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(dsc_aos_sum_kernel, dim3(blocks_for(stride, 256), n), dim3(256), 0, s, ix,
+                     splits, pvt, owned_fold, (const float*)partial, stride);
   return hipGetLastError();
 }
 

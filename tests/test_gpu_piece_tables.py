@@ -79,3 +79,65 @@ def test_concurrent_calls(C, O):
     for t in th:
         t.join()
     assert seen == [0, 20] * 4
+
+
+@pytest.mark.parametrize("P,npp,wpp,off", [
+    (4, 20480, 65537, 0),     # the largest node range whose sums fit in LDS; partial wire blocks
+    (4, 20481, 65537, 0),     # one more: atomics
+    (70, 5, 3745, 0),         # a table in device memory; far fewer nodes than lanes
+    (3, 1000, 87382, 4),      # records that start off a 16-byte boundary
+    (64, 4095, 4095, 0),      # just below the size from which LDS is used
+    (64, 4097, 4097, 0),      # above it, with as many nodes as wires
+])
+def test_large_tables_sum_charges(C, P, npp, wpp, off):
+    rng = np.random.default_rng(P + npp)
+    N, W = P * npp, P * wpp
+    w = np.zeros(W, C.WIRE)
+    piece = np.arange(W) // wpp
+    w["in_ptr"] = piece * npp + rng.integers(0, npp, W)
+    w["out_ptr"] = np.where(rng.random(W) < 0.8, piece * npp, rng.integers(0, P, W) * npp) + \
+        rng.integers(0, npp, W)
+    w["in_loc"], w["out_loc"] = rng.integers(0, 3, W), rng.integers(0, 3, W)
+    w["current"] = rng.standard_normal((W, 10))
+    pieces = np.zeros(P, C.PIECE)
+    k = np.arange(P)
+    pieces["first_wire"], pieces["num_wires"] = k * wpp, wpp
+    pieces["first_node"], pieces["num_nodes"] = k * npp, npp
+    n = np.zeros(N, C.NODE)
+    n["charge"] = rng.standard_normal(N) * 1e-6
+    raw = np.concatenate([np.zeros(off, np.uint8), w.view(np.uint8).reshape(-1),
+                          np.zeros(16 - off, np.uint8)])
+    dev = C.DeviceArray(raw)
+
+    class At:
+        ptr = type(dev.ptr)(dev.ptr.value + off)
+
+    dn = C.DeviceArray(n)
+    folds = [C.DeviceArray(np.zeros(N, np.float32)) for _ in range(2)]
+    want = [n["charge"].astype(np.float64), np.zeros(N), np.zeros(N)]
+    terms = [np.abs(want[0]), np.zeros(N), np.zeros(N)]
+    dt = np.float32(1e-6)
+    for ptr, loc, q in (("in_ptr", "in_loc", -dt * w["current"][:, 0]),
+                        ("out_ptr", "out_loc", dt * w["current"][:, 9])):
+        for kind in range(3):
+            m = w[loc] == kind
+            np.add.at(want[kind], w[ptr][m], q[m].astype(np.float64))
+            np.add.at(terms[kind], w[ptr][m], np.abs(q[m]).astype(np.float64))
+    C.distribute_charge_index_gpu(pieces, At, dn, *folds)
+    got = [dn.download()["charge"], folds[0].download(), folds[1].download()]
+    most = max(np.bincount(w["in_ptr"], minlength=N).max(), np.bincount(w["out_ptr"], minlength=N).max())
+    for g, x, t in zip(got, want, terms):
+        # each of at most 2 most + 1 additions rounds by 2^-24 of a partial sum
+        assert (np.abs(g - x) <= (2 * most + 1) * 2.0 ** -24 * t).all()
+    # the relaxation reads the same records (off the boundary word by word)
+    if off:
+        one = C.DeviceArray(w)
+        C.calc_new_currents_index_gpu(pieces, At, dn, dn, dn, flag=C.POLICY_FAST)
+        C.calc_new_currents_index_gpu(pieces, one, dn, dn, dn, flag=C.POLICY_FAST)
+        back = dev.download()[off:off + W * 128].view(C.WIRE)
+        assert back.tobytes() == one.download().tobytes()
+    bad = w.copy()
+    bad["in_loc"][[0, W - 1]] = 4
+    dev.upload(np.concatenate([raw[:off], bad.view(np.uint8).reshape(-1), raw[:16 - off]]))
+    with pytest.raises(C.CircuitError, match="2 wires"):
+        C.distribute_charge_index_gpu(pieces, At, dn, *folds)
