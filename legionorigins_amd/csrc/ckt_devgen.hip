@@ -321,24 +321,16 @@ __global__ __launch_bounds__(256) void gen_locations(uint32_t W, uint32_t npp, u
   vals[2 * w + 1] = (w << 1) | 1u;
 }
 
-// The index entries of a circuit whose pointers are given (an invalid pointer
-// is refused after the build; here it only has to stay in range).
-__global__ __launch_bounds__(256) void index_keys(DevCircuit c, uint32_t* __restrict__ keys,
-                                                  uint32_t* __restrict__ vals) {
-  const uint32_t w = blockIdx.x * 256u + threadIdx.x;
-  if (w >= c.num_wires) return;
-  const uint32_t a = c.in_ptr[w], b = c.out_ptr[w], last = c.num_nodes - 1;
-  *(uint2*)(keys + 2 * (size_t)w) = make_uint2(a < last ? a : last, b < last ? b : last);
-  *(uint2*)(vals + 2 * (size_t)w) = make_uint2(w << 1, (w << 1) | 1u);
-}
-
 // csr_row[n] = the first of the E sorted entries whose node is at least n, by
 // one binary search per row: 24 us for 8.4 M entries of 1 M nodes, where an
 // atomic count per entry and a scan of the counts took 296.
 __global__ __launch_bounds__(256) void index_rows(uint32_t N, uint32_t E,
                                                   const uint32_t* __restrict__ keys,
-                                                  uint32_t* __restrict__ row) {
+                                                  uint32_t* __restrict__ row,
+                                                  const LoadFaults* faults,
+                                                  LoadFaults* host_faults) {
   const uint32_t n = blockIdx.x * 256u + threadIdx.x;
+  if (n == 0 && faults) *host_faults = *faults;
   if (n > N) return;
   uint32_t lo = 0, hi = E;
   while (lo < hi) {
@@ -426,20 +418,39 @@ int enqueue_wires(const ckt_gen_params_t* p, uint32_t N, uint32_t W, uint32_t P,
   return CKT_OK;
 }
 
-// Scratch of the index build, carved from one buffer.
-struct IndexScratch {
-  uint32_t *keys, *vals, *keys_sorted;
-  void* work;
-  size_t sort_bytes;
-};
-
 unsigned key_bits(uint32_t N) {
   unsigned bits = 1;
   while (bits < 32 && (1ull << bits) < N) bits++;
   return bits;
 }
 
-// Bytes of scratch for N nodes and W wires; with `base`, carves it.
+DevCircuit index_view(uint32_t N, uint32_t W, uint32_t* csr_row, uint32_t* csr_ent) {
+  DevCircuit c{};
+  c.num_nodes = N;
+  c.num_wires = W;
+  c.csr_row = csr_row;
+  c.csr_ent = csr_ent;
+  return c;
+}
+
+// Locations, then the index.
+int enqueue_index(const ckt_gen_params_t* p, uint32_t N, uint32_t W, const SlabView& v,
+                  const IndexScratch& sc, hipStream_t s) {
+  if (W) {
+    hipLaunchKernelGGL(gen_locations, dim3(grid_for(W)), dim3(256), 0, s, W,
+                       (uint32_t)p->nodes_per_piece, (uint32_t)p->wires_per_piece,
+                       v.u(v.L.in_ptr), v.u(v.L.out_ptr), v.b + v.L.locator, v.b + v.L.in_loc,
+                       v.b + v.L.out_loc, sc.keys, sc.vals);
+    CKT_HIP(hipGetLastError());
+  }
+  const DevCircuit c = index_view(N, W, v.u(v.L.csr_row), v.u(v.L.csr_ent));
+  if (int st = index_sort(c, sc, s)) return st;
+  CKT_HIP(launch_index_rows(c, sc, nullptr, nullptr, s));
+  return CKT_OK;
+}
+
+}  // namespace
+
 int index_scratch(uint32_t N, uint32_t W, void* base, IndexScratch* sc, size_t* bytes) {
   size_t sort_bytes = 0;
   if (W)
@@ -460,56 +471,25 @@ int index_scratch(uint32_t N, uint32_t W, void* base, IndexScratch* sc, size_t* 
   return CKT_OK;
 }
 
-// The node -> (wire, end) index from the entries in `sc`: a stable sort by
-// node keeps each node's entries in (wire, in-before-out) order, and the rows
-// are searched for in the sorted nodes.
-int enqueue_sort(uint32_t N, uint32_t W, uint32_t* csr_row, uint32_t* csr_ent,
-                 const IndexScratch& sc, hipStream_t s) {
+int index_sort(const DevCircuit& c, const IndexScratch& sc, hipStream_t s) {
   size_t sort_bytes = sc.sort_bytes;
-  if (W)
+  if (c.num_wires)
     CKT_HIP(rocprim::radix_sort_pairs(sc.work, sort_bytes, sc.keys, sc.keys_sorted, sc.vals,
-                                      csr_ent, (size_t)2 * W, 0, key_bits(N), s));
-  hipLaunchKernelGGL(index_rows, dim3(grid_for((size_t)N + 1)), dim3(256), 0, s, N, 2 * W,
-                     sc.keys_sorted, csr_row);
-  CKT_HIP(hipGetLastError());
+                                      c.csr_ent, (size_t)2 * c.num_wires, 0,
+                                      key_bits(c.num_nodes), s));
   return CKT_OK;
 }
 
-// Locations, then the index.
-int enqueue_index(const ckt_gen_params_t* p, uint32_t N, uint32_t W, const SlabView& v,
-                  const IndexScratch& sc, hipStream_t s) {
-  if (W) {
-    hipLaunchKernelGGL(gen_locations, dim3(grid_for(W)), dim3(256), 0, s, W,
-                       (uint32_t)p->nodes_per_piece, (uint32_t)p->wires_per_piece,
-                       v.u(v.L.in_ptr), v.u(v.L.out_ptr), v.b + v.L.locator, v.b + v.L.in_loc,
-                       v.b + v.L.out_loc, sc.keys, sc.vals);
-    CKT_HIP(hipGetLastError());
-  }
-  return enqueue_sort(N, W, v.u(v.L.csr_row), v.u(v.L.csr_ent), sc, s);
-}
-
-}  // namespace
-
-size_t index_scratch_bytes(uint32_t N, uint32_t W) {
-  size_t bytes = 0;
-  return index_scratch(N, W, nullptr, nullptr, &bytes) ? 0 : bytes;
-}
-
-int index_enqueue(const DevCircuit& c, void* scratch, hipStream_t s) {
-  size_t bytes = 0;
-  IndexScratch sc{};
-  if (int st = index_scratch(c.num_nodes, c.num_wires, scratch, &sc, &bytes)) return st;
-  if (c.num_wires) {
-    hipLaunchKernelGGL(index_keys, dim3(grid_for(c.num_wires)), dim3(256), 0, s, c, sc.keys,
-                       sc.vals);
-    CKT_HIP(hipGetLastError());
-  }
-  return enqueue_sort(c.num_nodes, c.num_wires, c.csr_row, c.csr_ent, sc, s);
+hipError_t launch_index_rows(const DevCircuit& c, const IndexScratch& sc, const LoadFaults* faults,
+                             LoadFaults* host_faults, hipStream_t s) {
+  hipLaunchKernelGGL(index_rows, dim3(grid_for((size_t)c.num_nodes + 1)), dim3(256), 0, s,
+                     c.num_nodes, 2 * c.num_wires, sc.keys_sorted, c.csr_row, faults, host_faults);
+  return hipGetLastError();
 }
 
 size_t devgen_scratch_bytes(uint32_t N, uint32_t W) {
-  const size_t index = index_scratch_bytes(N, W);
-  return index ? span_scratch_bytes(W) + index : 0;
+  size_t index = 0;
+  return index_scratch(N, W, nullptr, nullptr, &index) ? 0 : span_scratch_bytes(W) + index;
 }
 
 int devgen_enqueue(const ckt_gen_params_t* p, const SlabLayout& L, void* slab, void* scratch,

@@ -225,6 +225,11 @@ static uint64_t piece_key(const ckt_piece_t& p) {
   return fnv(1469598103934665603ull, &p, sizeof(p));
 }
 
+// Build scratch up to this size is kept with the engine for the next build,
+// and slabs up to this size come from the stream's memory pool.
+constexpr size_t kKeepScratch = 64u << 20;
+constexpr size_t kPooledSlab = 32u << 20;
+
 Engine::~Engine() {
   if (device_ < 0) return;
   (void)hipSetDevice(device_);
@@ -237,6 +242,10 @@ Engine::~Engine() {
   }
   if (stream_) (void)hipStreamSynchronize(stream_);
   slots_.clear();
+  // What the memory pool keeps of this engine's circuits goes back.
+  hipMemPool_t pool = nullptr;
+  if (pool_ok_ && hipDeviceGetDefaultMemPool(&pool, device_) == hipSuccess)
+    (void)hipMemPoolTrimTo(pool, 0);
   if (d_table_) (void)hipFree(d_table_);
   if (d_counters_) (void)hipFree(d_counters_);
   if (d_bad_) (void)hipFree(d_bad_);
@@ -298,14 +307,14 @@ int Engine::add(SlabImage& img, int32_t loops, uint32_t* id) {
 // (PieceIndex::first_block, over wires) and the index build's scratch.
 namespace {
 struct RecordScratch {
-  size_t first_block, index, bytes;
+  size_t first_block, index, bytes;  // bytes 0: the index's size query failed
   RecordScratch(uint32_t N, uint32_t W, uint32_t P)
       : first_block(align_up(sizeof(LoadFaults), 256)),
-        index(align_up(first_block + 4 * ((size_t)P + 1), 256)),
-        bytes(index + index_scratch_bytes(N, W)) {}
+        index(align_up(first_block + 4 * ((size_t)P + 1), 256)) {
+    size_t n = 0;
+    bytes = index_scratch(N, W, nullptr, nullptr, &n) ? 0 : index + n;
+  }
 };
-// Scratch up to this size is kept with the engine for the next build.
-constexpr size_t kKeepScratch = 64u << 20;
 }  // namespace
 
 int Engine::build_scratch(size_t need, void** scratch, void** own) {
@@ -332,27 +341,10 @@ int Engine::build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, cons
   const RecordScratch at(N, W, P);
   LoadFaults* faults = (LoadFaults*)scratch;
   uint32_t* d_blocks = (uint32_t*)((uint8_t*)scratch + at.first_block);
-  CKT_HIP(launch_fill_u32((uint32_t*)faults, 0xffffffffu, sizeof(LoadFaults) / 4, stream_));
   int st;
-  if ((st = ring_.in(wires, sizeof(ckt_wire_t), W, device_, stream_,
-                     [&](void* slot, uint32_t first, uint32_t n) {
-                       return launch_unpack_wires((const ckt_wire_t*)slot, first, n, c, faults,
-                                                  stream_);
-                     })) ||
-      (st = ring_.in(nodes, sizeof(ckt_node_t), N, device_, stream_,
-                     [&](void* slot, uint32_t first, uint32_t n) {
-                       return launch_unpack_nodes((const ckt_node_t*)slot, first, n, c, stream_);
-                     })))
-    return st;
-  if (locator) {
-    if ((st = ring_.in(locator, sizeof(int32_t), N, device_, stream_,
-                       [&](void* slot, uint32_t first, uint32_t n) {
-                         return launch_unpack_locator((const int32_t*)slot, first, n, c, stream_);
-                       })))
-      return st;
-  } else {
-    CKT_HIP(launch_derive_locator(c, stream_));
-  }
+  IndexScratch sc{};
+  size_t index_bytes = 0;
+  if ((st = index_scratch(N, W, (uint8_t*)scratch + at.index, &sc, &index_bytes))) return st;
   // Pieces up to the first one that exceeds the circuit are checked for
   // private nodes of other pieces that their wires reach.
   std::vector<uint32_t> blocks(1, 0u);
@@ -368,22 +360,54 @@ int Engine::build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, cons
   const bool fits = good == P || (uint64_t)pieces[good].first_wire + pieces[good].num_wires > W ||
                     (uint64_t)pieces[good].first_node + pieces[good].num_nodes > N;
   if (!fits) return CKT_ERR_UNSUPPORTED;  // overlapping pieces past the grid's limit
-  if ((st = ring_.in(pieces, sizeof(ckt_piece_t), P, device_, stream_,
+  const LoadRest rest(N, locator != nullptr, P, good + 1);
+  if (rest.bytes <= HostRing::kSlotBytes) {
+    if ((st = ring_.put(rest.bytes, stream_,
+                        [&](unsigned char* b) {
+                          std::memcpy(b, nodes, sizeof(ckt_node_t) * (size_t)N);
+                          if (locator) std::memcpy(b + rest.locator_at, locator, 4 * (size_t)N);
+                          std::memcpy(b + rest.pieces_at, pieces, sizeof(ckt_piece_t) * (size_t)P);
+                          std::memcpy(b + rest.blocks_at, blocks.data(), 4 * blocks.size());
+                        },
+                        [&](void* slot) {
+                          return launch_unpack_rest(slot, rest, c, d_blocks, faults, stream_);
+                        })))
+      return st;
+  } else {
+    CKT_HIP(launch_clear_faults(faults, stream_));
+    if ((st = ring_.in(nodes, sizeof(ckt_node_t), N, device_, stream_,
+                       [&](void* slot, uint32_t first, uint32_t n) {
+                         return launch_unpack_nodes((const ckt_node_t*)slot, first, n, c, stream_);
+                       })) ||
+        (locator &&
+         (st = ring_.in(locator, sizeof(int32_t), N, device_, stream_,
+                        [&](void* slot, uint32_t first, uint32_t n) {
+                          return launch_unpack_locator((const int32_t*)slot, first, n, c, stream_);
+                        }))) ||
+        (st = ring_.in(pieces, sizeof(ckt_piece_t), P, device_, stream_,
+                       [&](void* slot, uint32_t first, uint32_t n) {
+                         return launch_copy_words((uint32_t*)(c.pieces + first), (uint32_t*)slot,
+                                                  4 * n, stream_);
+                       })) ||
+        (st = ring_.in(blocks.data(), sizeof(uint32_t), good + 1, device_, stream_,
+                       [&](void* slot, uint32_t first, uint32_t n) {
+                         return launch_copy_words(d_blocks + first, (uint32_t*)slot, n, stream_);
+                       })))
+      return st;
+  }
+  if ((st = ring_.in(wires, sizeof(ckt_wire_t), W, device_, stream_,
                      [&](void* slot, uint32_t first, uint32_t n) {
-                       return launch_copy_words((uint32_t*)(c.pieces + first), (uint32_t*)slot,
-                                                4 * n, stream_);
-                     })) ||
-      (st = ring_.in(blocks.data(), sizeof(uint32_t), good + 1, device_, stream_,
-                     [&](void* slot, uint32_t first, uint32_t n) {
-                       return launch_copy_words(d_blocks + first, (uint32_t*)slot, n, stream_);
+                       return launch_unpack_wires((const ckt_wire_t*)slot, first, n, c, sc, faults,
+                                                  stream_);
                      })))
     return st;
+  if (!locator) CKT_HIP(launch_derive_locator(c, stream_));
   const PieceIndex ix{c.pieces, d_blocks, good};
   CKT_HIP(launch_check_pieces(ix, (uint32_t)total, c, faults, stream_));
-  if ((st = index_enqueue(c, (uint8_t*)scratch + at.index, stream_))) return st;
+  if ((st = index_sort(c, sc, stream_))) return st;
   LoadFaults f;
   if ((st = ring_.out(&f, sizeof(f), 1, device_, stream_, [&](void* slot, uint32_t, uint32_t) {
-         return launch_copy_words((uint32_t*)slot, (const uint32_t*)faults, sizeof(f) / 4, stream_);
+         return launch_index_rows(c, sc, faults, (LoadFaults*)slot, stream_);
        })))
     return st;
   // In the order in which a pass over wires, then pieces, meets them.
@@ -420,26 +444,31 @@ int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* w
   // host and the replaced circuit leaves first.
   void *slab = nullptr, *own = nullptr;
   const size_t need = RecordScratch(N, W, P).bytes;
-  bool fits = !budget_ || in_use + lay.total <= budget_;
+  bool fits = need && (!budget_ || in_use + lay.total <= budget_);
   void* scratch = nullptr;
   if (fits && (st = build_scratch(need, &scratch, &own))) return st;
   fits = fits && scratch;
-  fits = fits && hipMalloc(&slab, lay.total) == hipSuccess;
+  // Small slabs come from the stream's memory pool: allocating and freeing one
+  // takes 5 us there, 115 us (and a wait for the stream) otherwise.
+  const bool pooled = pool_ok_ && lay.total <= kPooledSlab;
+  fits = fits && (pooled ? hipMallocAsync(&slab, lay.total, stream_)
+                         : hipMalloc(&slab, lay.total)) == hipSuccess;
   (void)hipGetLastError();
+  auto free_slab = [&] { (void)(pooled ? hipFreeAsync(slab, stream_) : hipFree(slab)); };
   if (fits) {
     st = build_records(nodes, wires, locator, pieces, device_view(slab, lay, N, W, P),
                        scratch);
     const hipError_t e = hipStreamSynchronize(stream_);
     if (!st && e != hipSuccess) st = hip_fail(e, "load");
     if (own) (void)hipFree(own);
-    if (st) (void)hipFree(slab);
+    if (st) free_slab();
     if (st && st != CKT_ERR_UNSUPPORTED) return st;
     if (!st && replaced && (st = remove(*replaced))) {
-      (void)hipFree(slab);
+      free_slab();
       return st;
     }
     if (!st) {
-      attach(slab, lay, N, W, P, std::vector<ckt_piece_t>(pieces, pieces + P), loops, id);
+      attach(slab, lay, N, W, P, std::vector<ckt_piece_t>(pieces, pieces + P), loops, id, pooled);
       return CKT_OK;
     }
   } else if (own) {
@@ -461,8 +490,9 @@ int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loop
     return fail(CKT_ERR_BUDGET, "circuit needs " + std::to_string(lay.total) +
                                     " bytes; budget has " + std::to_string(budget_ - in_use_) + " left");
   void* slab = nullptr;
-  hipError_t e = hipMalloc(&slab, lay.total);
-  if (e != hipSuccess) return hip_fail(e, "hipMalloc(circuit)");
+  const bool pooled = pool_ok_ && lay.total <= kPooledSlab;
+  hipError_t e = pooled ? hipMallocAsync(&slab, lay.total, stream_) : hipMalloc(&slab, lay.total);
+  if (e != hipSuccess) return hip_fail(e, "allocating a circuit");
   std::vector<ckt_piece_t> pieces;
   void *scratch = nullptr, *own = nullptr;
   const size_t need = devgen_scratch_bytes(N, W);
@@ -474,10 +504,10 @@ int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loop
   if (!st && e != hipSuccess) st = hip_fail(e, "device generator");
   if (own) (void)hipFree(own);
   if (st) {
-    (void)hipFree(slab);
+    (void)(pooled ? hipFreeAsync(slab, stream_) : hipFree(slab));
     return st;
   }
-  attach(slab, lay, N, W, P, pieces, loops, id);
+  attach(slab, lay, N, W, P, pieces, loops, id, pooled);
   return CKT_OK;
 }
 
@@ -862,8 +892,10 @@ int Engine::timed_end(int task, hipEvent_t a) {
 }
 
 int Engine::kernel_time(int task, double* ms, uint64_t* launches) {
-  CKT_HIP(hipSetDevice(device_));
-  CKT_HIP(hipStreamSynchronize(stream_));
+  if (!pending_.empty()) {  // events to read: they have to have happened
+    CKT_HIP(hipSetDevice(device_));
+    CKT_HIP(hipStreamSynchronize(stream_));
+  }
   for (auto& p : pending_) {
     float t = 0.f;
     CKT_HIP(hipEventElapsedTime(&t, p.a, p.b));
@@ -1150,8 +1182,9 @@ int Engine::sync() {
   return CKT_OK;
 }
 
-// Copies `bytes` into pinned staging memory (new chunks of at least 64 MiB
-// as needed) and returns its address, valid until the next sync().
+// Copies `bytes` into pinned staging memory (new chunks as needed, 1 MiB and
+// then twice the last one: pinning 64 MiB at the first tile list took 203 us
+// and freeing it 692, 1 MiB takes 80 and 47) and returns its address, valid until the next sync().
 int Engine::stage(const void* src, size_t bytes, void** out) {
   while (staging_chunk_ < staging_.size() &&
          staging_off_ + bytes > staging_[staging_chunk_].cap) {
@@ -1159,7 +1192,8 @@ int Engine::stage(const void* src, size_t bytes, void** out) {
     staging_off_ = 0;
   }
   if (staging_chunk_ == staging_.size()) {
-    PinnedChunk c{nullptr, std::max<size_t>(bytes, 64ull << 20)};
+    const size_t grown = staging_.empty() ? 1ull << 20 : 2 * staging_.back().cap;
+    PinnedChunk c{nullptr, std::max(bytes, std::min<size_t>(grown, 64ull << 20))};
     CKT_HIP(hipHostMalloc(&c.p, c.cap, hipHostMallocDefault));
     staging_.push_back(c);
     staging_off_ = 0;

@@ -18,7 +18,7 @@ namespace ckt {
 // While a kernel reads or writes one slot over the bus, host threads copy
 // others: one core copies about 10 GB/s to or from pageable memory, the bus
 // carries about 50.  One transfer at a time (the caller's lock).  Slots are
-// allocated as large as they are first needed and kept, 32 MiB at most.
+// allocated as large as they are first needed and kept, 38 MiB at most.
 class HostRing {
  public:
   HostRing() = default;
@@ -39,11 +39,12 @@ class HostRing {
   template <class Launch>
   int in(const void* src, size_t size, uint32_t count, int device, hipStream_t s, Launch launch) {
     const Plan p(size, count);
+    Slot* const own = slots_for(p);
     return team(p.workers, device, [&](int t) -> int {
       int side = 0;
       for (uint32_t c = (uint32_t)t; c < p.chunks; c += (uint32_t)p.workers, side ^= 1) {
         const uint32_t first = c * p.per, n = std::min(p.per, count - first);
-        Slot& sl = slots_[2 * t + side];
+        Slot& sl = own[2 * t + side];
         if (int st = acquire(sl, n * size)) return st;
         std::memcpy(sl.p, (const char*)src + (size_t)first * size, n * size);
         if (hipError_t e = launch(sl.p, first, n)) return hip_fail(e, "reading records");
@@ -53,17 +54,29 @@ class HostRing {
     });
   }
 
+  // One slot of `bytes` (kSlotBytes at most): fill(slot) writes it, launch(slot)
+  // enqueues the kernel that reads it.
+  template <class Fill, class Launch>
+  int put(size_t bytes, hipStream_t s, Fill fill, Launch launch) {
+    Slot& sl = *small_slot();
+    if (int st = acquire(sl, bytes)) return st;
+    fill((unsigned char*)sl.p);
+    if (hipError_t e = launch(sl.p)) return hip_fail(e, "reading records");
+    return mark(sl, s);
+  }
+
   // Calls launch(slot, first, n) for the kernels that write records into
   // slots on `s`, and copies each slot to `dst` when its kernel has run.
   // Returns when all records are there.
   template <class Launch>
   int out(void* dst, size_t size, uint32_t count, int device, hipStream_t s, Launch launch) {
     const Plan p(size, count);
+    Slot* const own = slots_for(p);
     return team(p.workers, device, [&](int t) -> int {
       auto begin = [&](uint32_t c, int side) -> int {
         if (c >= p.chunks) return CKT_OK;
         const uint32_t first = c * p.per, n = std::min(p.per, count - first);
-        Slot& sl = slots_[2 * t + side];
+        Slot& sl = own[2 * t + side];
         if (int st = acquire(sl, n * size)) return st;
         if (hipError_t e = launch(sl.p, first, n)) return hip_fail(e, "writing records");
         return mark(sl, s);
@@ -72,7 +85,7 @@ class HostRing {
       int st = begin((uint32_t)t, side);
       for (uint32_t c = (uint32_t)t; !st && c < p.chunks; c += (uint32_t)p.workers, side ^= 1) {
         if ((st = begin(c + (uint32_t)p.workers, side ^ 1))) break;
-        Slot& sl = slots_[2 * t + side];
+        Slot& sl = own[2 * t + side];
         if ((st = wait(sl))) break;
         const uint32_t first = c * p.per, n = std::min(p.per, count - first);
         std::memcpy((char*)dst + (size_t)first * size, sl.p, n * size);
@@ -81,16 +94,18 @@ class HostRing {
     });
   }
 
- private:
-  static constexpr int kWorkers = 8;
   static constexpr size_t kSlotBytes = 2u << 20;
+
+ private:
+  static constexpr int kWorkers = 8, kSlots = 2 * kWorkers, kSmall = 3;
   struct Slot {
     void* p = nullptr;
     size_t cap = 0;
     hipEvent_t ev = nullptr;
     bool busy = false;  // ev is recorded and not yet waited for
   };
-  Slot slots_[2 * kWorkers];
+  Slot slots_[kSlots + kSmall];
+  int next_ = 0;
 
   // A transfer's chunks (whole records, a multiple of four) and workers.
   struct Plan {
@@ -101,6 +116,16 @@ class HostRing {
           chunks((uint32_t)(((uint64_t)count + per - 1) / per)),
           workers((int)std::min<uint32_t>(chunks, kWorkers)) {}
   };
+
+  // Slots 2 t and 2 t + 1 of the result are worker t's.  A transfer of one
+  // chunk gets one of a few slots of its own in turn, so that it does not wait
+  // for the kernel of the transfer just before it, and a program that only
+  // makes small transfers pins few of them.
+  Slot* slots_for(const Plan& p) { return p.chunks > 1 ? slots_ : small_slot(); }
+  Slot* small_slot() {
+    next_ = (next_ + 1) % kSmall;
+    return slots_ + kSlots + next_;
+  }
 
   static int wait(Slot& sl) {
     if (!sl.busy) return CKT_OK;

@@ -43,6 +43,28 @@ __global__ __launch_bounds__(256) void unpack_nodes_kernel(const float4* __restr
   c.leak[first + i] = v.w;
 }
 
+__global__ __launch_bounds__(256) void unpack_rest_kernel(const uint8_t* __restrict__ host,
+                                                          LoadRest r, DevCircuit c,
+                                                          uint32_t* __restrict__ blocks,
+                                                          LoadFaults* faults) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i == 0) *faults = LoadFaults{~0ull, ~0ull, ~0ull};
+  if (i < r.nodes) {
+    const float4 v = ((const float4*)host)[i];  // charge, voltage, capacitance, leakage
+    c.charge[i] = v.x;
+    c.voltage[i] = v.y;
+    c.ncap[i] = v.z;
+    c.leak[i] = v.w;
+    if (r.locator) c.locator[i] = ((const int32_t*)(host + r.locator_at))[i] ? 1 : 0;
+  }
+  if (i < r.pieces) ((uint4*)c.pieces)[i] = ((const uint4*)(host + r.pieces_at))[i];
+  if (i < r.blocks) blocks[i] = ((const uint32_t*)(host + r.blocks_at))[i];
+}
+
+__global__ void clear_faults_kernel(LoadFaults* faults) {
+  *faults = LoadFaults{~0ull, ~0ull, ~0ull};
+}
+
 __global__ __launch_bounds__(256) void pack_nodes_kernel(float4* __restrict__ host, uint32_t first,
                                                          uint32_t n, DevCircuit c) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
@@ -53,7 +75,8 @@ __global__ __launch_bounds__(256) void pack_nodes_kernel(float4* __restrict__ ho
 
 __global__ __launch_bounds__(256) void unpack_wires_kernel(const uint4* __restrict__ host,
                                                            uint32_t first, uint32_t n,
-                                                           DevCircuit c, LoadFaults* faults) {
+                                                           DevCircuit c, IndexScratch sc,
+                                                           LoadFaults* faults) {
   __shared__ uint32_t rec[kWords * kRow];
   const uint32_t base = blockIdx.x * kTile;
   const uint32_t here = base < n ? (n - base < kTile ? n - base : kTile) : 0u;
@@ -87,6 +110,11 @@ __global__ __launch_bounds__(256) void unpack_wires_kernel(const uint4* __restri
   c.in_loc[w] = (uint8_t)la;
   c.out_loc[w] = (uint8_t)lb;
   if (t < here) {
+    // an invalid pointer is refused after the build; its entry only has to
+    // stay in range
+    const uint32_t last = c.num_nodes - 1;
+    *(uint2*)(sc.keys + 2 * (size_t)w) = make_uint2(a < last ? a : last, b < last ? b : last);
+    *(uint2*)(sc.vals + 2 * (size_t)w) = make_uint2(w << 1, (w << 1) | 1u);
     if (la > 2u || lb > 2u) atomicMin(&faults->location, (unsigned long long)w);
     if (a >= c.num_nodes || b >= c.num_nodes) atomicMin(&faults->pointer, (unsigned long long)w);
   }
@@ -182,6 +210,20 @@ __global__ __launch_bounds__(256) void copy_words_kernel(uint32_t* __restrict__ 
   }
 }
 
+hipError_t launch_unpack_rest(const void* host, const LoadRest& r, const DevCircuit& c,
+                              uint32_t* blocks, LoadFaults* faults, hipStream_t s) {
+  uint32_t n = r.nodes > r.pieces ? r.nodes : r.pieces;
+  n = n > r.blocks ? n : r.blocks;
+  hipLaunchKernelGGL(unpack_rest_kernel, dim3(grid_for(n)), dim3(256), 0, s, (const uint8_t*)host, r,
+                     c, blocks, faults);
+  return hipGetLastError();
+}
+
+hipError_t launch_clear_faults(LoadFaults* faults, hipStream_t s) {
+  hipLaunchKernelGGL(clear_faults_kernel, dim3(1), dim3(1), 0, s, faults);
+  return hipGetLastError();
+}
+
 hipError_t launch_unpack_nodes(const ckt_node_t* host, uint32_t first, uint32_t n,
                                const DevCircuit& c, hipStream_t s) {
   hipLaunchKernelGGL(unpack_nodes_kernel, dim3(grid_for(n)), dim3(256), 0, s, (const float4*)host,
@@ -190,10 +232,11 @@ hipError_t launch_unpack_nodes(const ckt_node_t* host, uint32_t first, uint32_t 
 }
 
 hipError_t launch_unpack_wires(const ckt_wire_t* host, uint32_t first, uint32_t n,
-                               const DevCircuit& c, LoadFaults* faults, hipStream_t s) {
+                               const DevCircuit& c, const IndexScratch& sc, LoadFaults* faults,
+                               hipStream_t s) {
   const uint32_t lanes = first + n == c.num_wires ? c.ws - first : n;
   hipLaunchKernelGGL(unpack_wires_kernel, dim3(grid_for(lanes)), dim3(256), 0, s,
-                     (const uint4*)host, first, n, c, faults);
+                     (const uint4*)host, first, n, c, sc, faults);
   return hipGetLastError();
 }
 
