@@ -225,10 +225,9 @@ static uint64_t piece_key(const ckt_piece_t& p) {
   return fnv(1469598103934665603ull, &p, sizeof(p));
 }
 
-// Build scratch up to this size is kept with the engine for the next build,
-// and slabs up to this size come from the stream's memory pool.
+// Build scratch up to this size is kept with the engine for the next build.
 constexpr size_t kKeepScratch = 64u << 20;
-constexpr size_t kPooledSlab = 32u << 20;
+constexpr uint32_t kDeviceLoadWires = 512;
 
 Engine::~Engine() {
   if (device_ < 0) return;
@@ -242,10 +241,6 @@ Engine::~Engine() {
   }
   if (stream_) (void)hipStreamSynchronize(stream_);
   slots_.clear();
-  // What the memory pool keeps of this engine's circuits goes back.
-  hipMemPool_t pool = nullptr;
-  if (pool_ok_ && hipDeviceGetDefaultMemPool(&pool, device_) == hipSuccess)
-    (void)hipMemPoolTrimTo(pool, 0);
   if (d_table_) (void)hipFree(d_table_);
   if (d_counters_) (void)hipFree(d_counters_);
   if (d_bad_) (void)hipFree(d_bad_);
@@ -404,12 +399,17 @@ int Engine::build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, cons
   if (!locator) CKT_HIP(launch_derive_locator(c, stream_));
   const PieceIndex ix{c.pieces, d_blocks, good};
   CKT_HIP(launch_check_pieces(ix, (uint32_t)total, c, faults, stream_));
-  if ((st = index_sort(c, sc, stream_))) return st;
   LoadFaults f;
-  if ((st = ring_.out(&f, sizeof(f), 1, device_, stream_, [&](void* slot, uint32_t, uint32_t) {
-         return launch_index_rows(c, sc, faults, (LoadFaults*)slot, stream_);
-       })))
-    return st;
+  if (index_is_small(N, W)) {
+    st = ring_.out(&f, sizeof(f), 1, device_, stream_, [&](void* slot, uint32_t, uint32_t) {
+      return launch_index_small(c, faults, (LoadFaults*)slot, stream_);
+    });
+  } else if (!(st = index_sort(c, sc, stream_))) {
+    st = ring_.out(&f, sizeof(f), 1, device_, stream_, [&](void* slot, uint32_t, uint32_t) {
+      return launch_index_rows(c, sc, faults, (LoadFaults*)slot, stream_);
+    });
+  }
+  if (st) return st;
   // In the order in which a pass over wires, then pieces, meets them.
   if (~f.location)
     return fail(CKT_ERR_INVALID_ARG,
@@ -441,34 +441,31 @@ int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* w
   const uint64_t in_use = in_use_ - (old ? old->lay.total : 0);
   // The device path holds the new circuit and its scratch beside the replaced
   // one.  Where that does not fit, the records are unpacked and checked on the
-  // host and the replaced circuit leaves first.
+  // host and the replaced circuit leaves first; so are the smallest circuits,
+  // for which that is faster (256 wires 30 us against 54, 1024 wires 110 against
+  // 56).
   void *slab = nullptr, *own = nullptr;
   const size_t need = RecordScratch(N, W, P).bytes;
-  bool fits = need && (!budget_ || in_use + lay.total <= budget_);
+  bool fits = W >= kDeviceLoadWires && need && (!budget_ || in_use + lay.total <= budget_);
   void* scratch = nullptr;
   if (fits && (st = build_scratch(need, &scratch, &own))) return st;
   fits = fits && scratch;
-  // Small slabs come from the stream's memory pool: allocating and freeing one
-  // takes 5 us there, 115 us (and a wait for the stream) otherwise.
-  const bool pooled = pool_ok_ && lay.total <= kPooledSlab;
-  fits = fits && (pooled ? hipMallocAsync(&slab, lay.total, stream_)
-                         : hipMalloc(&slab, lay.total)) == hipSuccess;
+  fits = fits && hipMalloc(&slab, lay.total) == hipSuccess;
   (void)hipGetLastError();
-  auto free_slab = [&] { (void)(pooled ? hipFreeAsync(slab, stream_) : hipFree(slab)); };
   if (fits) {
     st = build_records(nodes, wires, locator, pieces, device_view(slab, lay, N, W, P),
                        scratch);
     const hipError_t e = hipStreamSynchronize(stream_);
     if (!st && e != hipSuccess) st = hip_fail(e, "load");
     if (own) (void)hipFree(own);
-    if (st) free_slab();
+    if (st) (void)hipFree(slab);
     if (st && st != CKT_ERR_UNSUPPORTED) return st;
     if (!st && replaced && (st = remove(*replaced))) {
-      free_slab();
+      (void)hipFree(slab);
       return st;
     }
     if (!st) {
-      attach(slab, lay, N, W, P, std::vector<ckt_piece_t>(pieces, pieces + P), loops, id, pooled);
+      attach(slab, lay, N, W, P, std::vector<ckt_piece_t>(pieces, pieces + P), loops, id);
       return CKT_OK;
     }
   } else if (own) {
@@ -490,9 +487,8 @@ int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loop
     return fail(CKT_ERR_BUDGET, "circuit needs " + std::to_string(lay.total) +
                                     " bytes; budget has " + std::to_string(budget_ - in_use_) + " left");
   void* slab = nullptr;
-  const bool pooled = pool_ok_ && lay.total <= kPooledSlab;
-  hipError_t e = pooled ? hipMallocAsync(&slab, lay.total, stream_) : hipMalloc(&slab, lay.total);
-  if (e != hipSuccess) return hip_fail(e, "allocating a circuit");
+  hipError_t e = hipMalloc(&slab, lay.total);
+  if (e != hipSuccess) return hip_fail(e, "hipMalloc(circuit)");
   std::vector<ckt_piece_t> pieces;
   void *scratch = nullptr, *own = nullptr;
   const size_t need = devgen_scratch_bytes(N, W);
@@ -504,10 +500,10 @@ int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loop
   if (!st && e != hipSuccess) st = hip_fail(e, "device generator");
   if (own) (void)hipFree(own);
   if (st) {
-    (void)(pooled ? hipFreeAsync(slab, stream_) : hipFree(slab));
+    (void)hipFree(slab);
     return st;
   }
-  attach(slab, lay, N, W, P, pieces, loops, id, pooled);
+  attach(slab, lay, N, W, P, pieces, loops, id);
   return CKT_OK;
 }
 
@@ -669,6 +665,19 @@ int Engine::store(uint32_t id, ckt_node_t* nodes, ckt_wire_t* wires) {
   if (!c) return fail(CKT_ERR_NOT_FOUND, "no circuit with id " + std::to_string(id));
   CKT_HIP(hipSetDevice(device_));
   int st;
+  const size_t wire_bytes = sizeof(ckt_wire_t) * (size_t)c->num_wires,
+               node_bytes = sizeof(ckt_node_t) * (size_t)c->num_nodes;
+  if (wires && nodes && wire_bytes + node_bytes <= HostRing::kSlotBytes)
+    return ring_.get(wire_bytes + node_bytes, stream_,
+                     [&](void* slot) {
+                       return launch_pack_all((ckt_wire_t*)slot,
+                                              (ckt_node_t*)((uint8_t*)slot + wire_bytes), c->dev,
+                                              stream_);
+                     },
+                     [&](const unsigned char* b) {
+                       std::memcpy(wires, b, wire_bytes);
+                       std::memcpy(nodes, b + wire_bytes, node_bytes);
+                     });
   if (wires &&
       (st = ring_.out(wires, sizeof(ckt_wire_t), c->num_wires, device_, stream_,
                       [&](void* slot, uint32_t first, uint32_t n) {

@@ -65,6 +65,19 @@ class HostRing {
     return mark(sl, s);
   }
 
+  // One slot of `bytes` (kSlotBytes at most): launch(slot) enqueues the kernel
+  // that writes it, drain(slot) reads it when that has run.
+  template <class Launch, class Drain>
+  int get(size_t bytes, hipStream_t s, Launch launch, Drain drain) {
+    Slot& sl = *small_slot();
+    if (int st = acquire(sl, bytes)) return st;
+    if (hipError_t e = launch(sl.p)) return hip_fail(e, "writing records");
+    if (int st = mark(sl, s)) return st;
+    if (int st = wait(sl)) return st;
+    drain((const unsigned char*)sl.p);
+    return CKT_OK;
+  }
+
   // Calls launch(slot, first, n) for the kernels that write records into
   // slots on `s`, and copies each slot to `dst` when its kernel has run.
   // Returns when all records are there.

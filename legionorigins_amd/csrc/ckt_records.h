@@ -36,6 +36,12 @@ int index_sort(const DevCircuit& c, const IndexScratch& sc, hipStream_t s);
 hipError_t launch_index_rows(const DevCircuit& c, const IndexScratch& sc, const LoadFaults* faults,
                              LoadFaults* host_faults, hipStream_t s);
 
+// Circuits of up to 4096 wires and 2^15 nodes: the whole index, from the
+// circuit's pointers, in one workgroup (faults as for launch_index_rows).
+bool index_is_small(uint32_t N, uint32_t W);
+hipError_t launch_index_small(const DevCircuit& c, const LoadFaults* faults,
+                              LoadFaults* host_faults, hipStream_t s);
+
 // What a load reads besides the wires, in one piece of pinned memory: nodes,
 // locator (if `locator`), pieces, and the pieces' first workgroups, each on a
 // 16-byte boundary.
@@ -76,6 +82,9 @@ hipError_t launch_pack_nodes(ckt_node_t* host, uint32_t first, uint32_t n, const
                              hipStream_t s);
 hipError_t launch_pack_wires(ckt_wire_t* host, uint32_t first, uint32_t n, const DevCircuit& c,
                              hipStream_t s);
+// All of a small circuit's wires and nodes in one launch.
+hipError_t launch_pack_all(ckt_wire_t* wires, ckt_node_t* nodes, const DevCircuit& c,
+                           hipStream_t s);
 hipError_t launch_pack_locator(int32_t* host, uint32_t first, uint32_t n, const DevCircuit& c,
                                hipStream_t s);
 hipError_t launch_copy_words(uint32_t* host, const uint32_t* dev, uint32_t n, hipStream_t s);

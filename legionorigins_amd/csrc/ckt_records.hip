@@ -120,10 +120,10 @@ __global__ __launch_bounds__(256) void unpack_wires_kernel(const uint4* __restri
   }
 }
 
-__global__ __launch_bounds__(256) void pack_wires_kernel(uint4* __restrict__ host, uint32_t first,
-                                                         uint32_t n, DevCircuit c) {
+__device__ __forceinline__ void pack_tile(uint4* __restrict__ host, uint32_t tile, uint32_t first,
+                                          uint32_t n, const DevCircuit& c) {
   __shared__ uint32_t rec[kWords * kRow];
-  const uint32_t base = blockIdx.x * kTile;
+  const uint32_t base = tile * kTile;
   const uint32_t here = n - base < kTile ? n - base : kTile;
   const uint32_t t = threadIdx.x;
   if (t < here) {
@@ -153,6 +153,23 @@ __global__ __launch_bounds__(256) void pack_wires_kernel(uint4* __restrict__ hos
           make_uint4(rec[(part + 0) * kRow + w], rec[(part + 1) * kRow + w],
                      rec[(part + 2) * kRow + w], rec[(part + 3) * kRow + w]);
   }
+}
+
+__global__ __launch_bounds__(256) void pack_wires_kernel(uint4* __restrict__ host, uint32_t first,
+                                                         uint32_t n, DevCircuit c) {
+  pack_tile(host, blockIdx.x, first, n, c);
+}
+
+// Workgroups [0, wire_tiles) pack wires, the others nodes.
+__global__ __launch_bounds__(256) void pack_all_kernel(uint4* __restrict__ wires,
+                                                       float4* __restrict__ nodes,
+                                                       uint32_t wire_tiles, DevCircuit c) {
+  if (blockIdx.x < wire_tiles) {
+    pack_tile(wires, blockIdx.x, 0, c.num_wires, c);
+    return;
+  }
+  const uint32_t i = (blockIdx.x - wire_tiles) * 256u + threadIdx.x;
+  if (i < c.num_nodes) nodes[i] = make_float4(c.charge[i], c.voltage[i], c.ncap[i], c.leak[i]);
 }
 
 __global__ __launch_bounds__(256) void unpack_locator_kernel(const int32_t* __restrict__ host,
@@ -273,6 +290,14 @@ hipError_t launch_pack_wires(ckt_wire_t* host, uint32_t first, uint32_t n, const
                              hipStream_t s) {
   hipLaunchKernelGGL(pack_wires_kernel, dim3(grid_for(n)), dim3(256), 0, s, (uint4*)host, first, n,
                      c);
+  return hipGetLastError();
+}
+
+hipError_t launch_pack_all(ckt_wire_t* wires, ckt_node_t* nodes, const DevCircuit& c,
+                           hipStream_t s) {
+  const uint32_t tiles = grid_for(c.num_wires);
+  hipLaunchKernelGGL(pack_all_kernel, dim3(tiles + grid_for(c.num_nodes)), dim3(256), 0, s,
+                     (uint4*)wires, (float4*)nodes, tiles, c);
   return hipGetLastError();
 }
 

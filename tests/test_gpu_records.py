@@ -28,8 +28,12 @@ def _circuit(C, N, W, seed):
     return C.HostCircuit(n, w, np.zeros(N, np.int32), p)
 
 
-# tiles of 256 records, slots of 16384 wires, 131072 nodes and 524288 words
-@pytest.mark.parametrize("N,W", [(1, 0), (1, 1), (3, 63), (255, 257), (700, 16384), (64, 16385),
+# tiles of 256 records, slots of 16384 wires, 131072 nodes and 524288 words;
+# the host path below 512 wires, the one-workgroup index up to 4096 wires of
+# 32768 nodes
+@pytest.mark.parametrize("N,W", [(1, 0), (1, 1), (3, 63), (255, 511), (1, 512), (300, 769),
+                                 (32768, 4096), (32769, 4096), (5, 4095), (2000, 4097),
+                                 (700, 16384), (64, 16385),
                                  (131073, 49153), (131072, 262145), (300000, 300001)])
 def test_round_trip_and_index(C, N, W):
     c = _circuit(C, N, W, N + W)
