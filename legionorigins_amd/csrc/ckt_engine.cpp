@@ -1260,19 +1260,33 @@ int Engine::run_graph(const std::vector<PieceRef>& refs, int policy, int mode, i
                            wires_per_lane_,  tile_span_, tile_order_,     all_steps_,
                            (int64_t)generation_};
   key = fnv(key, cfg, sizeof(cfg));
+  // Every buffer the launches use is created before any capture (an allocation
+  // during capture is not allowed).
+  if ((st = prefetch_tiles(refs, policy, mode))) return st;
+  const bool timing = timing_;  // no events are recorded in this form
+  timing_ = false;
+  st = replay_loops(key, refs, policy, mode, times);
+  timing_ = timing;
+  return st;
+}
+
+// A graph of one loop takes 4 to 6 us a loop longer than its launches, one of
+// kGraphLoops as long as they do, and capturing one takes as long as several
+// loops of a small circuit; so fewer loops than that are launched directly.
+int Engine::replay_loops(uint64_t key, const std::vector<PieceRef>& refs, int policy, int mode,
+                         int times) {
+  int st;
+  for (int i = 0; i < times % kGraphLoops; i++)
+    if ((st = launch_loop(refs, policy, mode))) return st;
+  if (times < kGraphLoops) return CKT_OK;
   auto it = graphs_.find(key);
   hipGraphExec_t exec = nullptr;
   if (it == graphs_.end()) {
-    // Every buffer the captured launches use is created before capture (an
-    // allocation during capture is not allowed).
-    if ((st = prefetch_tiles(refs, policy, mode))) return st;
-    const bool timing = timing_;
-    timing_ = false;
     CKT_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-    st = launch_loop(refs, policy, mode);
+    st = CKT_OK;
+    for (int i = 0; i < kGraphLoops && !st; i++) st = launch_loop(refs, policy, mode);
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(stream_, &graph);
-    timing_ = timing;
     if (st) {
       if (graph) (void)hipGraphDestroy(graph);
       return st;
@@ -1285,7 +1299,7 @@ int Engine::run_graph(const std::vector<PieceRef>& refs, int policy, int mode, i
   } else {
     exec = it->second;
   }
-  for (int i = 0; i < times; i++) CKT_HIP(hipGraphLaunch(exec, stream_));
+  for (int i = 0; i < times / kGraphLoops; i++) CKT_HIP(hipGraphLaunch(exec, stream_));
   return CKT_OK;
 }
 

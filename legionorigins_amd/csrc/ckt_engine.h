@@ -140,9 +140,12 @@ class Engine {
   // Waits for the engine stream; recycles the staging memory of tile lists.
   int sync();
 
-  // One loop (cnc, dsc, upv) of `refs` captured in a graph and replayed
-  // `times` times.
+  // `times` loops (cnc, dsc, upv) of `refs`: kGraphLoops at a time by a captured
+  // graph, the rest launched.
+  static constexpr int kGraphLoops = 16;
   int run_graph(const std::vector<PieceRef>& refs, int policy, int mode, int times);
+  int replay_loops(uint64_t key, const std::vector<PieceRef>& refs, int policy, int mode,
+                   int times);
   // One loop of `refs`: calc_new_currents, distribute_charge, update_voltages
   // in two or three launches (loop_form).
   int loop_once(const std::vector<PieceRef>& refs, int policy, int mode);

@@ -60,9 +60,11 @@ struct Rec {
   ckt_request_result_t res{};
 };
 
+// Arrays left uninitialised until the store fills them.
 struct KeptState {
-  std::vector<ckt_node_t> nodes;
-  std::vector<ckt_wire_t> wires;
+  uint32_t num_nodes = 0, num_wires = 0;
+  std::unique_ptr<ckt_node_t[]> nodes;
+  std::unique_ptr<ckt_wire_t[]> wires;
 };
 
 }  // namespace
@@ -312,9 +314,11 @@ void schedule(ckt_server* s) {
       if (s->keep_state && rec(ri).wires <= s->keep_max_wires) {
         Circuit* c = E.find(id);
         KeptState k;
-        k.nodes.resize(c->num_nodes);
-        k.wires.resize(c->num_wires);
-        if ((st = E.store(id, k.nodes.data(), k.wires.data()))) break;
+        k.num_nodes = c->num_nodes;
+        k.num_wires = c->num_wires;
+        k.nodes.reset(new ckt_node_t[c->num_nodes]);
+        k.wires.reset(new ckt_wire_t[c->num_wires]);
+        if ((st = E.store(id, k.nodes.get(), k.wires.get()))) break;
         std::lock_guard<std::mutex> g(s->mu);
         s->kept[ri] = std::move(k);
       }
@@ -520,8 +524,9 @@ int ckt_server_fetch(ckt_server_t* s, uint32_t index, ckt_node_t* nodes, ckt_wir
   auto k = s->kept.find(index);
   if (k == s->kept.end())
     return fail(CKT_ERR_NOT_FOUND, "no kept state for request " + std::to_string(index));
-  if (nodes) std::copy(k->second.nodes.begin(), k->second.nodes.end(), nodes);
-  if (wires) std::copy(k->second.wires.begin(), k->second.wires.end(), wires);
+  const KeptState& kept = k->second;
+  if (nodes) std::copy(kept.nodes.get(), kept.nodes.get() + kept.num_nodes, nodes);
+  if (wires) std::copy(kept.wires.get(), kept.wires.get() + kept.num_wires, wires);
   return CKT_OK;
 }
 
