@@ -140,7 +140,7 @@ __global__ __launch_bounds__(kSmallLanes) void index_small(DevCircuit c, unsigne
 // wires, one dependent LDS read each) gives where it enters the next one and how
 // many wires it started.  For 4.2 M wires the spans take 69 us, their composition
 // 61 and the wires 98, bound by the walks' latency and the draws' 64-bit
-// multiplies; the whole circuit is built in 1.4 ms, where one host core's walk of
+// multiplies; the whole circuit is built in 1.0 ms, where one host core's walk of
 // the chain made it 26.
 constexpr uint32_t kSpan = 1024, kSubs = 8, kSub = kSpan / kSubs, kEntries = 7;
 

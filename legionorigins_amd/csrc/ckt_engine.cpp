@@ -225,8 +225,11 @@ static uint64_t piece_key(const ckt_piece_t& p) {
   return fnv(1469598103934665603ull, &p, sizeof(p));
 }
 
-// Build scratch up to this size is kept with the engine for the next build.
-constexpr size_t kKeepScratch = 64u << 20;
+// Build scratch up to this size is kept with the engine for the next build; above
+// it, scratch is allocated and freed by each.  A circuit of 64 x 65536 wires needs
+// about 170 MB, nearly all of it for the index's sort: generating it on the device
+// again takes 1.02 ms with the scratch kept and 1.31 without.
+constexpr size_t kKeepScratch = 192u << 20;
 constexpr uint32_t kDeviceLoadWires = 512;
 
 Engine::~Engine() {
@@ -945,9 +948,11 @@ int Engine::cnc(const std::vector<PieceRef>& refs, int policy, bool fuse_dsc) {
   // Launch shape unless set with OPT_CNC_BLOCK / OPT_PERSISTENT /
   // OPT_WAVES_PER_SIMD.  With the early end a launch is bound by the wires'
   // bytes, and a plain grid of 256-lane workgroups is best: on the 64 x 16384 x
-  // 65536 circuit 170 us for SCALED, FAST and RECIP (172-190 with 64, 128 or
-  // 512 lanes; a tile queue 190-980), EXACT 239 (stable) and 169 (reference
-  // profile) against 228-374 and 179-185.  With every step: on the 64 x 16384 x 65536 circuit a persistent tile
+  // 65536 circuit 157 us for SCALED, FAST and RECIP, and 217 for EXACT (stable
+  // profile).  With ordinary instead of nontemporal accesses, where the shapes
+  // were compared: 170 us for the first three (172-190 with 64, 128 or 512 lanes;
+  // a tile queue 190-980), EXACT 239 (stable) and 169 (reference profile) against
+  // 228-374 and 179-185.  With every step: on the same circuit a persistent tile
   // queue of 256-lane workgroups with 4 resident waves per SIMD beats the
   // plain grid by 6% for SCALED and 1-2% for FAST and RECIP.  For EXACT (71
   // VGPRs, at most 7 resident waves) a queue of 64-lane workgroups at 7 waves
@@ -1020,7 +1025,8 @@ int Engine::launch_loop(const std::vector<PieceRef>& refs, int policy, int mode)
 // and with the early end the index is the faster way to it too, except in small
 // launches (us a loop with the index / with the atomics in calc_new_currents /
 // with the LDS reduction as its own launch: 64 x 65536 wires 230 / 417 / 234, 16 x
-// 16384 21 / 34 / 29, 4 x 4096 11.9 / 10.7 / 18.7).  Where every step runs, the
+// 16384 21 / 34 / 29, 4 x 4096 11.9 / 10.7 / 18.7; the first of these is 201 now
+// that calc_new_currents leaves the index its cached currents).  Where every step runs, the
 // atomics hide behind the steps of other waves and stay fused.  The options that
 // name an ATOMIC form get it.
 constexpr uint64_t kIndexSumWires = 32768;
@@ -1193,7 +1199,8 @@ int Engine::sync() {
 
 // Copies `bytes` into pinned staging memory (new chunks as needed, 1 MiB and
 // then twice the last one: pinning 64 MiB at the first tile list took 203 us
-// and freeing it 692, 1 MiB takes 80 and 47) and returns its address, valid until the next sync().
+// and freeing it 692, 1 MiB takes 80 and 47) and returns its address, valid until
+// the next sync().
 int Engine::stage(const void* src, size_t bytes, void** out) {
   while (staging_chunk_ < staging_.size() &&
          staging_off_ + bytes > staging_[staging_chunk_].cap) {

@@ -18,7 +18,9 @@ namespace ckt {
 // While a kernel reads or writes one slot over the bus, host threads copy
 // others: one core copies about 10 GB/s to or from pageable memory, the bus
 // carries about 50.  One transfer at a time (the caller's lock).  Slots are
-// allocated as large as they are first needed and kept, 38 MiB at most.
+// allocated as large as they are first needed, kept, and freed with the ring:
+// 16 of at most 2 MiB, two for each of eight threads, and three for transfers
+// that one slot holds.
 class HostRing {
  public:
   HostRing() = default;

@@ -94,11 +94,11 @@ __device__ __forceinline__ bool wave_all(bool p) { return __all(p); }
 // changes by a bit.  It happens early: in the generator's circuits every wire
 // repeats itself (period 1, in a fifth of the wires 2, seldom 4) after at most
 // 18 of a loop's 10000 steps in the stable profile, and in the reference
-// profile its NaN has reached every current after 17.  For 64 x 65536 wires a
-// SCALED launch takes 0.50 instead of 10.5 ms, FAST 0.50 instead of 16.9, RECIP
-// 0.50 instead of 28.5 and EXACT 0.96 instead of 93 ms (reference profile; the
-// stable one alike), most of it no longer the steps but the launch's tile queue
-// and the fused charge atomics.
+// profile its NaN has reached every current after 17.  For 64 x 65536 wires of
+// the stable profile a SCALED, FAST or RECIP launch takes 157 us instead of 10.5,
+// 16.9 and 28.5 ms, and an EXACT one 217 us instead of 93 ms.  The first three are
+// bound by the wires' bytes (0.76 GB: the same accesses without a step take 148
+// us, a large library copy of as many bytes 122); EXACT by its divisions.
 //
 // One check costs about one step.  Windows of kWin steps are compared one
 // after another up to step kDense, then one window of kWide steps every
@@ -1223,7 +1223,8 @@ __device__ __forceinline__ float upv_one(float v, float q, float C, float lk) {
 //
 // Bound by the gathers of currents: a cache line from L2 per contribution (40 of
 // 68 us for 64 x 65536 wires and 64 x 16384 nodes; with the same bytes read in
-// order it takes 29).  A tile's contributions are one contiguous range of the
+// order it takes 29).  It takes 49.5 us behind a calc_new_currents that leaves
+// those currents cached.  A tile's contributions are one contiguous range of the
 // index: the workgroup gathers them kChunk at a time into LDS, eight independent
 // loads in flight per lane, and each lane then adds its node's own part in
 // order.  (One lane walking its node's list by itself keeps one dependent pair
