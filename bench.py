@@ -782,6 +782,7 @@ def main():
         early = {}
         for prof, cx in (("reference", ctx), ("stable", ctx_s)):
             cx.set_option(C.OPT_ALL_STEPS, 0)
+            cx.set_option(C.OPT_FUSE_DSC, -1)
             for name in ("exact", "recip", "fast", "scaled"):
                 cx.run_loops(2, policy=policy_of(C, name), mode=mode)
                 r7, w7, k7 = time_loops(C, cx, 10, policy_of(C, name), mode)
