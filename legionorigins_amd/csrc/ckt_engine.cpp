@@ -948,7 +948,7 @@ int Engine::cnc(const std::vector<PieceRef>& refs, int policy, bool fuse_dsc) {
   // Launch shape unless set with OPT_CNC_BLOCK / OPT_PERSISTENT /
   // OPT_WAVES_PER_SIMD.  With the early end a launch is bound by the wires'
   // bytes, and a plain grid of 256-lane workgroups is best: on the 64 x 16384 x
-  // 65536 circuit 157 us for SCALED, FAST and RECIP, and 217 for EXACT (stable
+  // 65536 circuit 157 us for SCALED, FAST and RECIP, and 183 to 358 for EXACT (stable
   // profile).  With ordinary instead of nontemporal accesses, where the shapes
   // were compared: 170 us for the first three (172-190 with 64, 128 or 512 lanes;
   // a tile queue 190-980), EXACT 239 (stable) and 169 (reference profile) against

@@ -96,7 +96,8 @@ __device__ __forceinline__ bool wave_all(bool p) { return __all(p); }
 // 18 of a loop's 10000 steps in the stable profile, and in the reference
 // profile its NaN has reached every current after 17.  For 64 x 65536 wires of
 // the stable profile a SCALED, FAST or RECIP launch takes 157 us instead of 10.5,
-// 16.9 and 28.5 ms, and an EXACT one 217 us instead of 93 ms.  The first three are
+// 16.9 and 28.5 ms, and an EXACT one 358 (in the first loop) to 183 us (from the
+// hundredth on) instead of 93 ms.  The first three are
 // bound by the wires' bytes (0.76 GB: the same accesses without a step take 148
 // us, a large library copy of as many bytes 122); EXACT by its divisions.
 //
@@ -157,14 +158,16 @@ struct Settle {
 // for another reason.  Returns n if that was found in every active lane --
 // the state is then that after step n -- and `limit` otherwise.  The state at
 // j need not be a function of the currents: no window starts there.
-template <bool kOn, int kWin, int kWide, int kDense, int kPlain, class Run, class Save, class Over>
+// The first window has kFirst steps, and those that start before step kFine two.
+template <bool kOn, int kWin, int kWide, int kDense, int kPlain, int kFirst = kWin, int kFine = 0,
+          class Run, class Save, class Over>
 __device__ __forceinline__ int advance(int j, int limit, int n, Run run, Save save, Over over) {
   if constexpr (!kOn) {
     run(limit - j);
     return limit;
   }
   bool on = true, probe = false, settled = false;
-  int k = min(kWin, limit - j);
+  int k = min(kFirst, limit - j);
   while (j < limit) {
     if (probe) save();
     run(k);
@@ -176,7 +179,8 @@ __device__ __forceinline__ int advance(int j, int limit, int n, Run run, Save sa
     }
     const bool dense = j < kDense;
     probe = on && (dense || !probe);
-    k = on ? min(dense ? kWin : probe ? kWide : kPlain, limit - j) : limit - j;
+    const int win = j < kFine ? 2 : kWin;
+    k = on ? min(dense ? win : probe ? kWide : kPlain, limit - j) : limit - j;
   }
   return settled ? n : limit;
 }
@@ -196,6 +200,9 @@ struct SplitDivisor {
   __device__ __forceinline__ explicit SplitDivisor(float divisor) : b(divisor) {
     make_div_split(divisor, &zh, &zl);
   }
+  // A divisor whose split is known.
+  __device__ __forceinline__ constexpr SplitDivisor(float divisor, float h, float l)
+      : b(divisor), zh(h), zl(l) {}
 };
 
 // Correctly rounded a[i] / b for N dividends, FP32 only: q = RN(a zh - u),
@@ -277,7 +284,10 @@ __device__ __forceinline__ float state_max(const float (&ni)[kSeg], const float 
 }
 
 // One step of the reference (circuit_gpu.cu:114-129) with every division by
-// the FP64 reciprocal of its divisor (div_fixed_group): no per-wire set-up.
+// the FP64 reciprocal of its divisor (div_fixed_group): no per-wire set-up.  The
+// split of dt is known, so with kSplitDt (EXACT) its ten divisions are by that:
+// 20 fmas and two guards instead of 30 instructions on the FP64 pipe and one.
+template <bool kSplitDt>
 __device__ __forceinline__ void reciprocal_step(float (&ni)[kSeg], float (&nv)[kSeg + 1],
                                                 const float (&I0)[kSeg],
                                                 const float (&V0)[kSeg - 1], float L, float R,
@@ -287,7 +297,13 @@ __device__ __forceinline__ void reciprocal_step(float (&ni)[kSeg], float (&nv)[k
   float t[kSeg], q[kSeg], u[kSeg - 1], w[kSeg - 1];
 #pragma unroll
   for (int i = 0; i < kSeg; i++) t[i] = L * (ni[i] - I0[i]);
-  div_fixed_group(q, t, rdt, dt);
+  // What make_div_split(dt) returns: RN(1/dt), RN(1/dt - RN(1/dt)).
+  constexpr float zh = (float)rdt, zl = (float)(rdt - (double)zh);
+  static_assert(zh == 0x1.e848p+19f && zl == 0x1.4aecccp-9f, "the split of dt");
+  if constexpr (kSplitDt)
+    div_split_group<kSeg, true>(q, t, SplitDivisor(dt, zh, zl));
+  else
+    div_fixed_group(q, t, rdt, dt);
 #pragma unroll
   for (int i = 0; i < kSeg; i++) t[i] = (nv[i + 1] - nv[i]) - q[i];
   div_fixed_group(ni, t, rR, R);
@@ -318,6 +334,14 @@ __device__ __forceinline__ void write_back(const float (&ni)[kSeg], const float 
 // of the wire's divisors first.  So with the early end on, the split comes
 // only after kSplitAfter steps, which most wires never reach; the steps are
 // the same bit for bit.
+//   EXACT's launch is bound by these steps, each as long as several checks, and a
+// wave's wires have repeated themselves after 12 to 18 of them, with period 1 or
+// 2 but for a few: so its windows have two steps there, which ends a wave after
+// 12.6 to 18.7 steps on average instead of 16 to 21.4 (CPU count over the
+// generator's circuits, twelve loops, both profiles).  64 x 65536 wires, stable
+// profile, us a launch in the first loop / the third / the average of the second
+// hundred: 420 / 375 / 222 with windows of four and all divisions by reciprocals, 395 /
+// 322 / 193 with these windows, 358 / 295 / 183 with the split of dt.
 constexpr int kSplitAfter = 64;
 
 template <bool kSplit, class St>
@@ -327,10 +351,10 @@ __device__ __forceinline__ void reference_steps(float (&ni)[kSeg], float (&nv)[k
   int j = 0;
   if constexpr (!kSplit || St::on) {
     const double rR = 1.0 / (double)R, rC = 1.0 / (double)C;
-    j = advance<St::on, 4, 12, 64, 1020>(
+    j = advance<St::on, 4, 12, 64, 1020, kSplit ? 6 : 4, kSplit ? 24 : 0>(
         0, kSplit ? min(steps, kSplitAfter) : steps, steps,
         [&](int k) {
-          for (int i = 0; i < k; i++) reciprocal_step(ni, nv, I0, V0, L, R, C, rR, rC);
+          for (int i = 0; i < k; i++) reciprocal_step<kSplit>(ni, nv, I0, V0, L, R, C, rR, rC);
         },
         [&] { st.save(ni); }, [&] { return st.same(ni); });
   }
@@ -555,7 +579,7 @@ __device__ __forceinline__ void finish_in_reference_order(float (&I)[kSeg], floa
   for (int i = 0; i < kSeg - 1; i++) nv[i + 1] = V[i] + div_fixed(dt * (x[i] - x[i + 1]), rC, C);
   nv[kSeg] = vout;
   const double rR = 1.0 / (double)R;
-  for (int j = 0; j < kTail; j++) reciprocal_step(x, nv, I, V, L, R, C, rR, rC);
+  for (int j = 0; j < kTail; j++) reciprocal_step<false>(x, nv, I, V, L, R, C, rR, rC);
   write_back(x, nv, I, V);
 }
 
