@@ -145,9 +145,11 @@ __global__ __launch_bounds__(kSmallLanes) void index_small(DevCircuit c, unsigne
 constexpr uint32_t kSpan = 1024, kSubs = 8, kSub = kSpan / kSubs, kEntries = 7;
 
 struct SpanScratch {
-  uint8_t cross[kSpan];                   // whether a wire that starts here is cross-piece
+  // whether a wire that starts here is cross-piece; a lane writes four as a word
+  alignas(4) uint8_t cross[kSpan];
   uint16_t step[kSubs][kEntries + 1];     // count << 3 | entry into the next sub-span
 };
+static_assert(alignof(SpanScratch) >= 4, "word stores into cross");
 
 // Fills `sp` for span b: lane t takes positions 4 t .. 4 t + 3.  With `states`,
 // also each position's state (before its draw).
