@@ -347,17 +347,7 @@ int Engine::build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, cons
   // private nodes of other pieces that their wires reach.
   std::vector<uint32_t> blocks(1, 0u);
   uint32_t good = 0;
-  uint64_t total = 0;
-  while (good < P && (uint64_t)pieces[good].first_wire + pieces[good].num_wires <= W &&
-         (uint64_t)pieces[good].first_node + pieces[good].num_nodes <= N &&
-         total + ((uint64_t)pieces[good].num_wires + 255) / 256 <= 0x7fffffffu) {
-    total += ((uint64_t)pieces[good].num_wires + 255) / 256;
-    blocks.push_back((uint32_t)total);
-    good++;
-  }
-  const bool fits = good == P || (uint64_t)pieces[good].first_wire + pieces[good].num_wires > W ||
-                    (uint64_t)pieces[good].first_node + pieces[good].num_nodes > N;
-  if (!fits) return CKT_ERR_UNSUPPORTED;  // overlapping pieces past the grid's limit
+  if (!piece_check_blocks(pieces, P, N, W, &blocks, &good)) return CKT_ERR_UNSUPPORTED;
   const LoadRest rest(N, locator != nullptr, P, good + 1);
   if (rest.bytes <= HostRing::kSlotBytes) {
     if ((st = ring_.put(rest.bytes, stream_,
@@ -401,7 +391,7 @@ int Engine::build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, cons
     return st;
   if (!locator) CKT_HIP(launch_derive_locator(c, stream_));
   const PieceIndex ix{c.pieces, d_blocks, good};
-  CKT_HIP(launch_check_pieces(ix, (uint32_t)total, c, faults, stream_));
+  CKT_HIP(launch_check_pieces(ix, blocks.back(), c, faults, stream_));
   LoadFaults f;
   if (index_is_small(N, W)) {
     st = ring_.out(&f, sizeof(f), 1, device_, stream_, [&](void* slot, uint32_t, uint32_t) {

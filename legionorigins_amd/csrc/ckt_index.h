@@ -41,6 +41,32 @@ __host__ __device__ inline uint32_t piece_of_block(const uint32_t* first_block, 
   return lo;
 }
 
+// HIP refuses a launch of 2^32 lanes or more in one dimension: the most
+// workgroups of 256 lanes in one.
+constexpr uint64_t kMaxBlocks256 = 0xffffffffu / 256u;
+
+// The piece table of a load's check (one lane per wire of each piece): appends
+// to `first_block` (which holds the 0 of the first piece) the end of every
+// piece's workgroups, up to the first piece that exceeds N nodes or W wires, and
+// sets *good to the number of pieces before that one.  False if they take more
+// workgroups than a launch can have: pieces may overlap, so their wires can be
+// many times W.
+template <class Piece>
+bool piece_check_blocks(const Piece* pieces, uint32_t P, uint32_t N, uint32_t W,
+                        std::vector<uint32_t>* first_block, uint32_t* good) {
+  uint64_t total = 0;
+  uint32_t k = 0;
+  for (; k < P; k++) {
+    const Piece& p = pieces[k];
+    if ((uint64_t)p.first_wire + p.num_wires > W || (uint64_t)p.first_node + p.num_nodes > N) break;
+    total += ((uint64_t)p.num_wires + 255) / 256;
+    if (total > kMaxBlocks256) return false;
+    first_block->push_back((uint32_t)total);
+  }
+  *good = k;
+  return true;
+}
+
 // Wire subrange si of `splits` of a piece's num_wires wires in the LDS
 // reduction: whole 1024-wire blocks, [*k0, *k1); trailing subranges may be
 // empty.
