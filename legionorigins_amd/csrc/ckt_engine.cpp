@@ -351,12 +351,10 @@ int Engine::build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, cons
   const LoadRest rest(N, locator != nullptr, P, good + 1);
   if (rest.bytes <= HostRing::kSlotBytes) {
     if ((st = ring_.put(rest.bytes, stream_,
-                        [&](unsigned char* b) {
-                          std::memcpy(b, nodes, sizeof(ckt_node_t) * (size_t)N);
-                          if (locator) std::memcpy(b + rest.locator_at, locator, 4 * (size_t)N);
-                          std::memcpy(b + rest.pieces_at, pieces, sizeof(ckt_piece_t) * (size_t)P);
-                          std::memcpy(b + rest.blocks_at, blocks.data(), 4 * blocks.size());
-                        },
+                        {{0, nodes, sizeof(ckt_node_t) * (size_t)N},
+                         {rest.locator_at, locator, locator ? 4 * (size_t)N : 0},
+                         {rest.pieces_at, pieces, sizeof(ckt_piece_t) * (size_t)P},
+                         {rest.blocks_at, blocks.data(), 4 * blocks.size()}},
                         [&](void* slot) {
                           return launch_unpack_rest(slot, rest, c, d_blocks, faults, stream_);
                         })))
@@ -667,10 +665,7 @@ int Engine::store(uint32_t id, ckt_node_t* nodes, ckt_wire_t* wires) {
                                               (ckt_node_t*)((uint8_t*)slot + wire_bytes), c->dev,
                                               stream_);
                      },
-                     [&](const unsigned char* b) {
-                       std::memcpy(wires, b, wire_bytes);
-                       std::memcpy(nodes, b + wire_bytes, node_bytes);
-                     });
+                     {{0, wires, wire_bytes}, {wire_bytes, nodes, node_bytes}});
   if (wires &&
       (st = ring_.out(wires, sizeof(ckt_wire_t), c->num_wires, device_, stream_,
                       [&](void* slot, uint32_t first, uint32_t n) {

@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <initializer_list>
 #include <string>
 #include <system_error>
 #include <thread>
@@ -20,7 +21,9 @@ namespace ckt {
 // carries about 50.  One transfer at a time (the caller's lock).  Slots are
 // allocated as large as they are first needed, kept, and freed with the ring:
 // 16 of at most 2 MiB, two for each of eight threads, and three for transfers
-// that one slot holds.
+// that one slot holds.  Where no pinned memory can be had a slot is device
+// memory of the same size, filled and read with synchronous copies: slower, but
+// a circuit can still be loaded and stored.
 class HostRing {
  public:
   HostRing() = default;
@@ -29,7 +32,7 @@ class HostRing {
   ~HostRing() {
     for (Slot& sl : slots_) {
       if (sl.busy) (void)hipEventSynchronize(sl.ev);
-      if (sl.p) (void)hipHostFree(sl.p);
+      (void)release(sl);
       if (sl.ev) (void)hipEventDestroy(sl.ev);
     }
   }
@@ -48,7 +51,7 @@ class HostRing {
         const uint32_t first = c * p.per, n = std::min(p.per, count - first);
         Slot& sl = own[2 * t + side];
         if (int st = acquire(sl, n * size)) return st;
-        std::memcpy(sl.p, (const char*)src + (size_t)first * size, n * size);
+        if (int st = write(sl, 0, (const char*)src + (size_t)first * size, n * size, s)) return st;
         if (hipError_t e = launch(sl.p, first, n)) return hip_fail(e, "reading records");
         if (int st = mark(sl, s)) return st;
       }
@@ -56,27 +59,41 @@ class HostRing {
     });
   }
 
-  // One slot of `bytes` (kSlotBytes at most): fill(slot) writes it, launch(slot)
-  // enqueues the kernel that reads it.
-  template <class Fill, class Launch>
-  int put(size_t bytes, hipStream_t s, Fill fill, Launch launch) {
+  // A part of a slot and the host memory it is copied from or to.
+  struct Source {
+    size_t at;
+    const void* p;
+    size_t bytes;
+  };
+  struct Sink {
+    size_t at;
+    void* p;
+    size_t bytes;
+  };
+
+  // One slot of `bytes` (kSlotBytes at most): `parts` are copied into it, and
+  // launch(slot) enqueues the kernel that reads it.
+  template <class Launch>
+  int put(size_t bytes, hipStream_t s, std::initializer_list<Source> parts, Launch launch) {
     Slot& sl = *small_slot();
     if (int st = acquire(sl, bytes)) return st;
-    fill((unsigned char*)sl.p);
+    for (const Source& x : parts)
+      if (int st = write(sl, x.at, x.p, x.bytes, s)) return st;
     if (hipError_t e = launch(sl.p)) return hip_fail(e, "reading records");
     return mark(sl, s);
   }
 
   // One slot of `bytes` (kSlotBytes at most): launch(slot) enqueues the kernel
-  // that writes it, drain(slot) reads it when that has run.
-  template <class Launch, class Drain>
-  int get(size_t bytes, hipStream_t s, Launch launch, Drain drain) {
+  // that writes it, and `parts` are copied from it when that has run.
+  template <class Launch>
+  int get(size_t bytes, hipStream_t s, Launch launch, std::initializer_list<Sink> parts) {
     Slot& sl = *small_slot();
     if (int st = acquire(sl, bytes)) return st;
     if (hipError_t e = launch(sl.p)) return hip_fail(e, "writing records");
     if (int st = mark(sl, s)) return st;
     if (int st = wait(sl)) return st;
-    drain((const unsigned char*)sl.p);
+    for (const Sink& x : parts)
+      if (int st = read(sl, x.at, x.p, x.bytes, s)) return st;
     return CKT_OK;
   }
 
@@ -103,7 +120,7 @@ class HostRing {
         Slot& sl = own[2 * t + side];
         if ((st = wait(sl))) break;
         const uint32_t first = c * p.per, n = std::min(p.per, count - first);
-        std::memcpy((char*)dst + (size_t)first * size, sl.p, n * size);
+        st = read(sl, 0, (char*)dst + (size_t)first * size, n * size, s);
       }
       return st;
     });
@@ -117,7 +134,8 @@ class HostRing {
     void* p = nullptr;
     size_t cap = 0;
     hipEvent_t ev = nullptr;
-    bool busy = false;  // ev is recorded and not yet waited for
+    bool busy = false;    // ev is recorded and not yet waited for
+    bool pinned = false;  // host memory, else device memory
   };
   Slot slots_[kSlots + kSmall];
   int next_ = 0;
@@ -153,13 +171,40 @@ class HostRing {
     if (int st = wait(sl)) return st;
     if (!sl.ev) CKT_HIP(hipEventCreateWithFlags(&sl.ev, hipEventDisableTiming));
     if (bytes > sl.cap) {
-      if (sl.p) CKT_HIP(hipHostFree(sl.p));
-      sl.p = nullptr;
-      sl.cap = 0;
+      CKT_HIP(release(sl));
       const size_t cap = std::min(kSlotBytes, std::max<size_t>(2 * bytes, 64u << 10));
-      CKT_HIP(hipHostMalloc(&sl.p, cap, hipHostMallocDefault));
+      sl.pinned = hipHostMalloc(&sl.p, cap, hipHostMallocDefault) == hipSuccess;
+      if (!sl.pinned) {
+        (void)hipGetLastError();
+        sl.p = nullptr;
+        CKT_HIP(hipMalloc(&sl.p, cap));
+      }
       sl.cap = cap;
     }
+    return CKT_OK;
+  }
+  static hipError_t release(Slot& sl) {
+    void* p = sl.p;
+    sl.p = nullptr;
+    sl.cap = 0;
+    if (!p) return hipSuccess;
+    return sl.pinned ? hipHostFree(p) : hipFree(p);
+  }
+  static int write(const Slot& sl, size_t at, const void* src, size_t bytes, hipStream_t s) {
+    return move(sl, (char*)sl.p + at, src, bytes, hipMemcpyHostToDevice, s);
+  }
+  static int read(const Slot& sl, size_t at, void* dst, size_t bytes, hipStream_t s) {
+    return move(sl, dst, (const char*)sl.p + at, bytes, hipMemcpyDeviceToHost, s);
+  }
+  static int move(const Slot& sl, void* dst, const void* src, size_t bytes, hipMemcpyKind kind,
+                  hipStream_t s) {
+    if (!bytes) return CKT_OK;
+    if (sl.pinned) {
+      std::memcpy(dst, src, bytes);
+      return CKT_OK;
+    }
+    CKT_HIP(hipMemcpyAsync(dst, src, bytes, kind, s));
+    CKT_HIP(hipStreamSynchronize(s));
     return CKT_OK;
   }
   static int mark(Slot& sl, hipStream_t s) {
