@@ -225,11 +225,13 @@ static uint64_t piece_key(const ckt_piece_t& p) {
   return fnv(1469598103934665603ull, &p, sizeof(p));
 }
 
-// Build scratch up to this size is kept with the engine for the next build; above
-// it, scratch is allocated and freed by each.  A circuit of 64 x 65536 wires needs
-// about 170 MB, nearly all of it for the index's sort: generating it on the device
-// again takes 1.02 ms with the scratch kept and 1.31 without.
-constexpr size_t kKeepScratch = 192u << 20;
+// Build scratch up to this share of the budget is kept with the engine for the
+// next build, within the budget beside the circuits; other scratch is allocated
+// and freed by each build.  A circuit's scratch is about a quarter of its slab,
+// nearly all of it for the index's sort (64 x 65536 wires 170 MB), and
+// allocating it costs such a build 0.3 ms of 1.3.  The default budget's share (1
+// GB) is the scratch of 25 M wires.
+constexpr uint64_t kKeepShare = 256;
 constexpr uint32_t kDeviceLoadWires = 512;
 
 Engine::~Engine() {
@@ -289,8 +291,10 @@ int Engine::add(SlabImage& img, int32_t loops, uint32_t* id) {
   if (budget_ && in_use_ + img.lay.total > budget_)
     return fail(CKT_ERR_BUDGET, "circuit needs " + std::to_string(img.lay.total) +
                                     " bytes; budget has " + std::to_string(budget_ - in_use_) + " left");
+  int st = trim_scratch(img.lay.total);
+  if (st) return st;
   void* slab = nullptr;
-  hipError_t e = hipMalloc(&slab, img.lay.total);
+  hipError_t e = alloc_slab(img.lay.total, &slab);
   if (e != hipSuccess) return hip_fail(e, "hipMalloc(circuit)");
   e = hipMemcpy(slab, img.bytes.data(), img.lay.total, hipMemcpyHostToDevice);
   if (e != hipSuccess) {
@@ -315,14 +319,11 @@ struct RecordScratch {
 };
 }  // namespace
 
-int Engine::build_scratch(size_t need, void** scratch, void** own) {
+int Engine::build_scratch(size_t need, bool keep, void** scratch, void** own) {
   *scratch = *own = nullptr;
-  if (need > devgen_scratch_cap_ && need <= kKeepScratch) {
-    // Builds already enqueued use the old scratch.
-    CKT_HIP(hipStreamSynchronize(stream_));
-    if (devgen_scratch_) CKT_HIP(hipFree(devgen_scratch_));
-    devgen_scratch_ = nullptr;
-    devgen_scratch_cap_ = 0;
+  int st;
+  if (need > devgen_scratch_cap_ && keep) {
+    if ((st = drop_scratch())) return st;
     if (hipMalloc(&devgen_scratch_, need) == hipSuccess) devgen_scratch_cap_ = need;
     else devgen_scratch_ = nullptr;
   }
@@ -331,6 +332,31 @@ int Engine::build_scratch(size_t need, void** scratch, void** own) {
   else *own = nullptr;
   (void)hipGetLastError();
   return CKT_OK;
+}
+
+int Engine::drop_scratch() {
+  if (!devgen_scratch_) return CKT_OK;
+  // Builds already enqueued use it.
+  CKT_HIP(hipStreamSynchronize(stream_));
+  CKT_HIP(hipFree(devgen_scratch_));
+  devgen_scratch_ = nullptr;
+  devgen_scratch_cap_ = 0;
+  return CKT_OK;
+}
+
+int Engine::trim_scratch(uint64_t bytes) {
+  if (!budget_ || in_use_ + bytes + devgen_scratch_cap_ <= budget_) return CKT_OK;
+  return drop_scratch();
+}
+
+hipError_t Engine::alloc_slab(size_t bytes, void** slab) {
+  hipError_t e = hipMalloc(slab, bytes);
+  if (e != hipSuccess && devgen_scratch_) {  // it may fit in the scratch's place
+    (void)hipGetLastError();
+    if (drop_scratch() == CKT_OK) e = hipMalloc(slab, bytes);
+  }
+  if (e != hipSuccess) *slab = nullptr;
+  return e;
 }
 
 int Engine::build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, const int32_t* locator,
@@ -428,20 +454,18 @@ int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* w
   CKT_HIP(hipSetDevice(device_));
   int st;
   const SlabLayout lay = SlabLayout::make(N, W, P);
-  const Circuit* old = replaced ? find(*replaced) : nullptr;
-  const uint64_t in_use = in_use_ - (old ? old->lay.total : 0);
   // The device path holds the new circuit and its scratch beside the replaced
-  // one.  Where that does not fit, the records are unpacked and checked on the
-  // host and the replaced circuit leaves first; so are the smallest circuits,
-  // for which that is faster (256 wires 30 us against 54, 1024 wires 110 against
-  // 56).
-  void *slab = nullptr, *own = nullptr;
-  const size_t need = RecordScratch(N, W, P).bytes;
-  bool fits = W >= kDeviceLoadWires && need && (!budget_ || in_use + lay.total <= budget_);
-  void* scratch = nullptr;
-  if (fits && (st = build_scratch(need, &scratch, &own))) return st;
-  fits = fits && scratch;
-  fits = fits && hipMalloc(&slab, lay.total) == hipSuccess;
+  // one.  Where the budget or the memory has no room for that, the records are
+  // unpacked and checked on the host and the replaced circuit leaves first; so
+  // are the smallest circuits, for which that is faster (256 wires 30 us against
+  // 54, 1024 wires 110 against 56).
+  void *slab = nullptr, *own = nullptr, *scratch = nullptr;
+  const size_t need = RecordScratch(N, W, P).bytes, kept = devgen_scratch_cap_;
+  const bool keep = need <= budget_ / kKeepShare;
+  const uint64_t held = in_use_ + lay.total + (need <= kept ? kept : keep ? need : kept + need);
+  bool fits = W >= kDeviceLoadWires && need && (!budget_ || held <= budget_);
+  if (fits && (st = build_scratch(need, keep, &scratch, &own))) return st;
+  fits = fits && scratch && hipMalloc(&slab, lay.total) == hipSuccess;
   (void)hipGetLastError();
   if (fits) {
     st = build_records(nodes, wires, locator, pieces, device_view(slab, lay, N, W, P),
@@ -450,7 +474,7 @@ int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* w
     if (!st && e != hipSuccess) st = hip_fail(e, "load");
     if (own) (void)hipFree(own);
     if (st) (void)hipFree(slab);
-    if (st && st != CKT_ERR_UNSUPPORTED) return st;
+    if (st && st != CKT_ERR_UNSUPPORTED && st != CKT_ERR_NO_MEMORY) return st;
     if (!st && replaced && (st = remove(*replaced))) {
       (void)hipFree(slab);
       return st;
@@ -459,6 +483,7 @@ int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* w
       attach(slab, lay, N, W, P, std::vector<ckt_piece_t>(pieces, pieces + P), loops, id);
       return CKT_OK;
     }
+    (void)hipGetLastError();
   } else if (own) {
     (void)hipFree(own);
   }
@@ -477,14 +502,17 @@ int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loop
   if (budget_ && in_use_ + lay.total > budget_)
     return fail(CKT_ERR_BUDGET, "circuit needs " + std::to_string(lay.total) +
                                     " bytes; budget has " + std::to_string(budget_ - in_use_) + " left");
+  const size_t need = devgen_scratch_bytes(N, W);
+  if (!need) return fail(CKT_ERR_HIP, "device generator scratch size query failed");
+  if ((st = trim_scratch(lay.total))) return st;
   void* slab = nullptr;
-  hipError_t e = hipMalloc(&slab, lay.total);
+  hipError_t e = alloc_slab(lay.total, &slab);
   if (e != hipSuccess) return hip_fail(e, "hipMalloc(circuit)");
   std::vector<ckt_piece_t> pieces;
   void *scratch = nullptr, *own = nullptr;
-  const size_t need = devgen_scratch_bytes(N, W);
-  if (!need) st = fail(CKT_ERR_HIP, "device generator scratch size query failed");
-  else if (!(st = build_scratch(need, &scratch, &own)) && !scratch)
+  const bool keep =
+      need <= budget_ / kKeepShare && (!budget_ || in_use_ + lay.total + need <= budget_);
+  if (!(st = build_scratch(need, keep, &scratch, &own)) && !scratch)
     st = fail(CKT_ERR_NO_MEMORY, "device generator: no memory for its scratch");
   if (!st) st = devgen_enqueue(params, lay, slab, scratch, stream_, pieces);
   e = hipStreamSynchronize(stream_);

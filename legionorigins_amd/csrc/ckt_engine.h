@@ -173,11 +173,17 @@ class Engine {
               bool stream_ordered = false);
   static DevCircuit device_view(void* slab, const SlabLayout& L, uint32_t N, uint32_t W,
                                 uint32_t P);
-  // Scratch of `need` bytes for a build: the engine's own (grown, after the
-  // builds already enqueued) up to kKeepScratch, else, or where that fails, an
-  // allocation in *own that the caller frees; NULL if there is no memory.
-  int build_scratch(size_t need, void** scratch, void** own);
-  // add_records' build into `slab`; `scratch` as record_scratch_bytes says.
+  // Scratch of `need` bytes for a build: the engine's own where it is large
+  // enough or, with `keep`, can be grown (after the builds already enqueued), else
+  // an allocation in *own that the caller frees; NULL if there is no memory.
+  int build_scratch(size_t need, bool keep, void** scratch, void** own);
+  // Frees the engine's own scratch, the second only if it does not fit in the
+  // budget beside the circuits and `bytes` more.
+  int drop_scratch();
+  int trim_scratch(uint64_t bytes);
+  // A circuit's memory; takes the scratch's place if there is no other.
+  hipError_t alloc_slab(size_t bytes, void** slab);
+  // add_records' build into the slab of `c`; `scratch` as RecordScratch says.
   int build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, const int32_t* locator,
                     const ckt_piece_t* pieces, const DevCircuit& c, void* scratch);
   int ensure_table();
@@ -248,9 +254,9 @@ class Engine {
   bool timing_ = false;
   std::vector<Pending> pending_;
   std::vector<hipEvent_t> event_pool_;
-  // Device scratch of circuit builds (grow-only; the builds on the stream run
-  // one after another), and pinned staging chunks for tile lists and the
-  // descriptor table, recycled at sync().
+  // Device scratch of circuit builds (the builds on the stream run one after
+  // another), and pinned staging chunks for tile lists and the descriptor table,
+  // recycled at sync().
   bool pool_ok_ = false;  // the device's default memory pool is usable
   void* devgen_scratch_ = nullptr;
   size_t devgen_scratch_cap_ = 0;
