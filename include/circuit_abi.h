@@ -431,13 +431,15 @@ int ckt_batch_store(ckt_batch_t* b, uint32_t id, ckt_node_t* nodes, ckt_wire_t* 
  * *best: first the launch shape (workgroup size x plain grid or persistent
  * queue x resident waves), then, with that shape, the tile schedule (wires
  * per lane x tile span x tile order).  Only calc_new_currents is timed, with
- * `probe_steps` inner steps per candidate; circuit state is restored
- * afterwards. */
+ * loops of `probe_steps` inner steps, each from the circuits' own state, which is
+ * restored afterwards.  Waves whose wires repeat themselves end before that many
+ * steps here as in a run (CKT_OPT_ALL_STEPS). */
 int ckt_batch_autotune(ckt_batch_t* b, int32_t policy, int32_t probe_steps,
                        ckt_batch_config_t* best, double* best_ms);
 /* The probe ckt_batch_autotune times, for one configuration: milliseconds of
- * calc_new_currents over every circuit at `probe_steps` inner steps (the
- * faster of two launches); circuit state is restored afterwards. */
+ * calc_new_currents over every circuit with a loop of `probe_steps` inner steps
+ * (the faster of two launches from the same state); circuit state is restored
+ * afterwards. */
 int ckt_batch_probe(ckt_batch_t* b, const ckt_batch_config_t* config, int32_t probe_steps,
                     double* ms);
 

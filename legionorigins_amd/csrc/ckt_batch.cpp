@@ -68,9 +68,11 @@ int apply_config(ckt_batch_t* b, const ckt_batch_config_t& cfg) { return apply_c
 
 // The probes of ckt_batch_autotune / ckt_batch_probe: calc_new_currents over
 // every circuit at a shortened step count, timed with events on the engine
-// stream.  The constructor saves each circuit's currents and internal
-// voltages (one contiguous region of its slab) and the engine options; the
-// destructor puts both back.
+// stream.  begin() saves each circuit's currents and internal voltages (one
+// contiguous region of its slab) and the engine options; the destructor puts
+// both back.  The state is put back before every timed launch too: with the
+// early end the steps that a launch executes depend on it, and fewer are left
+// from one launch's result than from the state before.
 class Prober {
  public:
   explicit Prober(Engine& E) : E_(E) {}
@@ -90,12 +92,14 @@ class Prober {
     CKT_HIP(hipEventCreate(&z_));
     return E_.set_option(OPT_STEPS, probe_steps);
   }
-  // The faster of two launches under `cfg`'s launch shape and schedule.
+  // The faster of two launches under `cfg`'s launch shape and schedule, each
+  // from the saved state.
   int time(int32_t policy, const ckt_batch_config_t& cfg, double* ms) {
     int st;
     if ((st = apply_config(E_, cfg))) return st;
     double t = 1e30;
     for (int rep = 0; rep < 2; rep++) {
+      CKT_HIP(restore());
       if ((st = E_.sync())) return st;
       CKT_HIP(hipEventRecord(a_, E_.stream()));
       if ((st = E_.cnc(refs_, policy))) return st;
@@ -113,17 +117,24 @@ class Prober {
     if (z_) (void)hipEventDestroy(z_);
     if (began_)
       for (int o = 0; o < kOpts; o++) (void)E_.set_option(kOptIds[o], opts_[o]);
-    hipStream_t s = E_.stream();
-    for (size_t i = 0; i < saved_.size(); i++) {
-      Circuit* c = E_.slots()[i];
-      (void)hipMemcpyAsync((uint8_t*)c->slab + c->lay.cur, saved_[i], c->lay.ind - c->lay.cur,
-                           hipMemcpyDeviceToDevice, s);
-    }
-    (void)hipStreamSynchronize(s);
+    (void)restore();
+    (void)hipStreamSynchronize(E_.stream());
     for (void* p : saved_) (void)hipFree(p);
   }
 
  private:
+  hipError_t restore() {
+    hipError_t bad = hipSuccess;
+    for (size_t i = 0; i < saved_.size(); i++) {
+      Circuit* c = E_.slots()[i];
+      const hipError_t e =
+          hipMemcpyAsync((uint8_t*)c->slab + c->lay.cur, saved_[i], c->lay.ind - c->lay.cur,
+                         hipMemcpyDeviceToDevice, E_.stream());
+      if (e != hipSuccess) bad = e;
+    }
+    return bad;
+  }
+
   static constexpr int kOpts = 7;
   static constexpr int kOptIds[kOpts] = {OPT_STEPS,          OPT_CNC_BLOCK, OPT_PERSISTENT,
                                          OPT_WAVES_PER_SIMD, OPT_WIRES_PER_LANE,
