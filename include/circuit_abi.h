@@ -127,7 +127,8 @@ enum {
  *           FAST's step.
  * Every policy stops stepping a wave of wires early where their states repeat
  * themselves, with the same bits as if every step were executed
- * (CKT_OPT_ALL_STEPS); a server with EXACT executes every step.
+ * (CKT_OPT_ALL_STEPS); a server with EXACT executes every step unless told not to
+ * (ckt_server_set_option).
  * RECIP, FAST and SCALED are not bit-exact; their error is checked against
  * 1e-5.  FAST and SCALED write a wire whose currents left the finite range as
  * all NaN, which is where the reference recurrence ends such a wire. */
@@ -331,7 +332,7 @@ typedef struct ckt_loop_report {
 int ckt_run_loops(ckt_ctx_t* ctx, int num_loops, const ckt_loop_config_t* config,
                   ckt_loop_report_t* report);
 
-/* Tuning and test options (context and batch). */
+/* Tuning and test options (context, batch and server). */
 enum {
   CKT_OPT_STEPS = 0,             /* inner steps per loop (default CKT_STEPS) */
   CKT_OPT_CNC_BLOCK = 1,         /* calc_new_currents workgroup size: 64/128/256/512;
@@ -526,6 +527,10 @@ int ckt_server_set_keep_state(ckt_server_t* s, int keep_state);
 /* Keep only the states of requests with at most max_wires wires (default:
  * all). */
 int ckt_server_set_keep_limit(ckt_server_t* s, uint32_t max_wires);
+/* A CKT_OPT_* for every request (set before a start or a trace).  A server with
+ * EXACT is created with CKT_OPT_ALL_STEPS 1; 0 ends its requests' loops early,
+ * with the same bits. */
+int ckt_server_set_option(ckt_server_t* s, int option, int64_t value);
 int ckt_server_fetch(ckt_server_t* s, uint32_t index, ckt_node_t* nodes, ckt_wire_t* wires);
 
 /* Debug builds (CKT_BOUNDS_CHECKS, the counterpart of the reference's

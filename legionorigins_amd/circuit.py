@@ -212,6 +212,7 @@ def _declare(L):
         "ckt_server_set_keep_state": ([vp, i32], i32),
         "ckt_server_fetch": ([vp, u32, vp, vp], i32),
         "ckt_server_set_keep_limit": ([vp, u32], i32),
+        "ckt_server_set_option": ([vp, i32, ctypes.c_int64], i32),
         "ckt_server_start": ([vp], i32),
         "ckt_server_stop": ([vp, i32], i32),
         "ckt_server_submit": ([vp, P(_GenParams), i32, ctypes.c_double, P(u32)], i32),
@@ -662,6 +663,9 @@ class Server:
         _check(lib().ckt_server_set_keep_state(self.h, int(keep)))
         _check(lib().ckt_server_set_keep_limit(self.h, 0xFFFFFFFF if max_wires is None
                                                else int(max_wires)))
+
+    def set_option(self, opt, value):
+        _check(lib().ckt_server_set_option(self.h, opt, value))
 
     # Online serving (ckt_server_start/submit/poll/wait/cancel/stop).
     def start(self):

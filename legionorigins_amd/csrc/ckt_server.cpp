@@ -476,9 +476,9 @@ int ckt_server_create(int device, const ckt_server_config_t* config, ckt_server_
     delete s;
     return st;
   }
-  // EXACT requests execute every step.  The early end would serve a 500-loop
-  // request of 16384 wires in under 50 ms, and callers (the online test of
-  // wait's time limit and of cancel) count on it running longer than that.
+  // EXACT requests execute every step unless ckt_server_set_option says
+  // otherwise, so that a request lasts as long as it always did: time limits,
+  // deadlines and cancels that callers chose for EXACT requests rely on it.
   if (cfg.policy == CKT_POLICY_EXACT) st = s->eng.set_option(OPT_ALL_STEPS, 1);
   if (st) {
     delete s;
@@ -516,6 +516,13 @@ int ckt_server_set_keep_limit(ckt_server_t* s, uint32_t max_wires) {
   if (s->running) return fail(CKT_ERR_STATE, "server: set the keep limit before starting");
   s->keep_max_wires = max_wires;
   return CKT_OK;
+}
+
+int ckt_server_set_option(ckt_server_t* s, int option, int64_t value) {
+  if (!s) return fail(CKT_ERR_INVALID_ARG, "null server");
+  std::lock_guard<std::mutex> g(s->mu);
+  if (s->running) return fail(CKT_ERR_STATE, "server: set options before starting");
+  return s->eng.set_option(option, value);
 }
 
 int ckt_server_fetch(ckt_server_t* s, uint32_t index, ckt_node_t* nodes, ckt_wire_t* wires) {
