@@ -824,6 +824,24 @@ constexpr int kUpvTile = 2048;
 constexpr uint64_t kUpvBytesPerNode = 24;
 constexpr uint64_t kLastLevelCacheBytes = 256ull << 20;
 
+// Whether calc_new_currents with the early end moves its wires' state with
+// ordinary accesses, so that the last-level cache holds it from loop to loop:
+// where the state, the pointers and the index entries (104 bytes a wire) fit that
+// cache but not twice the L2s (8 x 4 MB), else nontemporal (load_once).  Larger
+// circuits push each other's lines out, and below the L2s the ordinary accesses
+// push out what the loop's other launch reads.  Microseconds a SCALED loop,
+// nontemporal / ordinary, 16384 wires to 4096 nodes or 65536 to 16384: 128k wires
+// 15.7 / 15.7, 256k 19.3 / 20.3, 384k 27.3 / 27.8, 512k 36.0 / 36.9; 768k 45.8 /
+// 41.2, 1024k 59.3 / 51.7, 2048k 109 / 89.5, 2304k 119 / 101; 2560k 132 / 144, 4096k
+// 200 / 230.  FAST and RECIP alike, EXACT with smaller steps in the same places.
+constexpr uint64_t kL2Bytes = 8 * (4ull << 20);
+constexpr uint64_t kCncBytesPerWire = 104;
+
+static bool cnc_state_cached(uint64_t wires) {
+  const uint64_t bytes = wires * kCncBytesPerWire;
+  return bytes > 2 * kL2Bytes && bytes <= kLastLevelCacheBytes;
+}
+
 int Engine::tiles_for(int kind, const std::vector<PieceRef>& refs, int block, DevBuf* out) {
   uint64_t key = fnv(1469598103934665603ull, &kind, sizeof(kind));
   key = fnv(key, &block, sizeof(block));
@@ -975,16 +993,20 @@ int Engine::cnc(const std::vector<PieceRef>& refs, int policy, bool fuse_dsc) {
   const bool persistent =
       persistent_ >= 0 ? persistent_ != 0
                        : all_steps_ && (policy != CKT_POLICY_EXACT || cnc_block_ < 0);
+  uint64_t wires = 0;
+  for (const PieceRef& r : refs) wires += slots_[r.slot]->pieces[r.piece].num_wires;
+  const CncSteps how = all_steps_ ? kEveryStep
+                       : cnc_state_cached(wires) ? kEarlyEnd
+                                                 : kEarlyEndStream;
   const int waves = waves_per_simd_ > 0 ? waves_per_simd_ : (policy == CKT_POLICY_EXACT ? 7 : 4);
   if (persistent) {
     const int waves_per_block = block / 64;
     int grid = num_cus_ * 4 * waves / waves_per_block;
     if (grid > (int)t.n) grid = (int)t.n;
     e = launch_cnc_persistent(policy, fuse_dsc, d_table_, (const Tile*)t.p, t.n, block, grid,
-                              d_counters_, steps_, all_steps_ != 0, stream_);
+                              d_counters_, steps_, how, stream_);
   } else {
-    e = launch_cnc(policy, fuse_dsc, d_table_, (const Tile*)t.p, t.n, block, steps_,
-                   all_steps_ != 0, stream_);
+    e = launch_cnc(policy, fuse_dsc, d_table_, (const Tile*)t.p, t.n, block, steps_, how, stream_);
   }
   if (e != hipSuccess) return hip_fail(e, "calc_new_currents launch");
   return timed_end(CKT_CALC_NEW_CURRENTS, a);

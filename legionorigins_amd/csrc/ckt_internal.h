@@ -57,13 +57,15 @@ struct PieceTile {
 
 // Host launchers (defined in ckt_kernels.hip).  All are asynchronous on `s`.
 // fuse_dsc adds each wire's two charge contributions with float atomics at the
-// end of the relaxation (the ATOMIC distribute_charge, fused); all_steps
-// executes every step also where the state repeats itself.
+// end of the relaxation (the ATOMIC distribute_charge, fused); `how` says
+// whether steps are executed where the state repeats itself, and without those
+// whether the wires' state is moved past the caches.
+enum CncSteps { kEveryStep, kEarlyEnd, kEarlyEndStream };
 hipError_t launch_cnc(int policy, bool fuse_dsc, const DevCircuit* circuits, const Tile* tiles,
-                      uint32_t ntiles, int block, int steps, bool all_steps, hipStream_t s);
+                      uint32_t ntiles, int block, int steps, CncSteps how, hipStream_t s);
 hipError_t launch_cnc_persistent(int policy, bool fuse_dsc, const DevCircuit* circuits,
                                  const Tile* tiles, uint32_t ntiles, int block, int grid,
-                                 uint32_t* counters, int steps, bool all_steps, hipStream_t s);
+                                 uint32_t* counters, int steps, CncSteps how, hipStream_t s);
 hipError_t launch_dsc_atomic(const DevCircuit* circuits, const Tile* tiles, uint32_t ntiles,
                              int block, hipStream_t s);
 // Dynamic LDS bytes of the LDS-privatised reduction for pieces of up to

@@ -120,7 +120,7 @@ __device__ __forceinline__ bool same_value(float a, float b) {
 // bare loops (SCALED 10.98 against 10.45 ms, EXACT 94.7 against 92.3 ms for
 // 64 x 65536 wires with every step executed).
 struct EveryStep {
-  static constexpr bool on = false;
+  static constexpr bool on = false, stream = false;
   __device__ __forceinline__ EveryStep(lfloat*, uint32_t) {}
   template <int kRow = 0, int N>
   __device__ __forceinline__ void save(const float (&)[N]) const {}
@@ -131,7 +131,7 @@ struct EveryStep {
 };
 
 struct Settle {
-  static constexpr bool on = true;
+  static constexpr bool on = true, stream = false;
   lfloat* snap;     // this lane's column, kSeg rows of `stride` floats
   uint32_t stride;
   __device__ __forceinline__ Settle(lfloat* lane_column, uint32_t row_stride)
@@ -150,6 +150,12 @@ struct Settle {
     for (int i = 0; i < N; i++) eq &= same_value(snap[(kRow + i) * stride], x[i]);
     return eq;
   }
+};
+
+// With the wires' state moved past the caches (load_once).
+struct SettleStream : Settle {
+  static constexpr bool stream = true;
+  using Settle::Settle;
 };
 
 // Takes the state from step j to step `limit` of n by run(k), which takes k
@@ -988,11 +994,13 @@ struct Relax<CKT_POLICY_SCALED> {
 typedef __attribute__((address_space(1))) float gfloat;
 typedef __attribute__((address_space(1))) const uint32_t gcu32;
 
-// A wire's state is read and written once per loop, so with the early end, where
-// the launch is bound by those bytes, they are nontemporal: 64 x 65536 wires 157
-// us instead of 171 (stores alone gain nothing).  The two currents that the
-// charge reduction reads next stay ordinary stores, and are then still cached:
-// its launch takes 49.5 instead of 68 us, and the loop 201 instead of 230.
+// A wire's state is read and written once per loop.  With the early end, where
+// the launch is bound by those bytes, they are nontemporal (SettleStream) unless
+// the last-level cache holds them from loop to loop (cnc_state_cached):
+// 64 x 65536 wires 157 us instead of 171 (stores alone gain nothing).  The two
+// currents that the charge reduction reads next stay ordinary stores, and are
+// then still cached: its launch takes 49.5 instead of 68 us, and the loop 201
+// instead of 230.
 template <bool kNt, class T>
 __device__ __forceinline__ T load_once(const __attribute__((address_space(1))) T* p) {
   if constexpr (kNt) return __builtin_nontemporal_load(p);
@@ -1017,9 +1025,9 @@ __device__ __forceinline__ void cnc_one(const DevCircuit& c, uint32_t w, int ste
     return;
   float I[kSeg], V[kSeg - 1];
 #pragma unroll
-  for (int s = 0; s < kSeg; s++) I[s] = load_once<St::on>(&cur[s * ws + w]);
+  for (int s = 0; s < kSeg; s++) I[s] = load_once<St::stream>(&cur[s * ws + w]);
 #pragma unroll
-  for (int s = 0; s < kSeg - 1; s++) V[s] = load_once<St::on>(&vol[s * ws + w]);
+  for (int s = 0; s < kSeg - 1; s++) V[s] = load_once<St::stream>(&vol[s * ws + w]);
   const float L = ((gfloat*)c.ind)[w], R = ((gfloat*)c.res)[w], C = ((gfloat*)c.wcap)[w];
   const float vin = ((gfloat*)c.voltage)[((gcu32*)c.in_ptr)[w]];
   const float vout = ((gfloat*)c.voltage)[((gcu32*)c.out_ptr)[w]];
@@ -1028,10 +1036,10 @@ __device__ __forceinline__ void cnc_one(const DevCircuit& c, uint32_t w, int ste
 #pragma unroll
   for (int s = 0; s < kSeg; s++) {
     if (s == 0 || s == kSeg - 1) cur[s * ws + w] = I[s];
-    else store_once<St::on>(I[s], &cur[s * ws + w]);
+    else store_once<St::stream>(I[s], &cur[s * ws + w]);
   }
 #pragma unroll
-  for (int s = 0; s < kSeg - 1; s++) store_once<St::on>(V[s], &vol[s * ws + w]);
+  for (int s = 0; s < kSeg - 1; s++) store_once<St::stream>(V[s], &vol[s * ws + w]);
   if (FUSE) {
     const float dt = CKT_DT_F;
     unsafeAtomicAdd(&c.charge[c.in_ptr[w]], -dt * I[0]);
@@ -1710,47 +1718,55 @@ static hipError_t cnc_by_block(bool persistent, const DevCircuit* c, const Tile*
 
 template <int POLICY, bool FUSE>
 static hipError_t cnc_by_steps(bool persistent, const DevCircuit* c, const Tile* t, uint32_t n,
-                               int block, int grid, uint32_t* ctr, int steps, bool all,
+                               int block, int grid, uint32_t* ctr, int steps, CncSteps how,
                                hipStream_t s) {
-  return all ? cnc_by_block<POLICY, FUSE, EveryStep>(persistent, c, t, n, block, grid, ctr, steps, s)
-             : cnc_by_block<POLICY, FUSE, Settle>(persistent, c, t, n, block, grid, ctr, steps, s);
+  switch (how) {
+    case kEveryStep:
+      return cnc_by_block<POLICY, FUSE, EveryStep>(persistent, c, t, n, block, grid, ctr, steps, s);
+    case kEarlyEnd:
+      return cnc_by_block<POLICY, FUSE, Settle>(persistent, c, t, n, block, grid, ctr, steps, s);
+    case kEarlyEndStream:
+      return cnc_by_block<POLICY, FUSE, SettleStream>(persistent, c, t, n, block, grid, ctr, steps,
+                                                      s);
+  }
+  return hipErrorInvalidValue;
 }
 
 template <int POLICY>
 static hipError_t cnc_by_fuse(bool fuse, bool persistent, const DevCircuit* c, const Tile* t,
-                              uint32_t n, int block, int grid, uint32_t* ctr, int steps, bool all,
-                              hipStream_t s) {
-  return fuse ? cnc_by_steps<POLICY, true>(persistent, c, t, n, block, grid, ctr, steps, all, s)
-              : cnc_by_steps<POLICY, false>(persistent, c, t, n, block, grid, ctr, steps, all, s);
+                              uint32_t n, int block, int grid, uint32_t* ctr, int steps,
+                              CncSteps how, hipStream_t s) {
+  return fuse ? cnc_by_steps<POLICY, true>(persistent, c, t, n, block, grid, ctr, steps, how, s)
+              : cnc_by_steps<POLICY, false>(persistent, c, t, n, block, grid, ctr, steps, how, s);
 }
 
 static hipError_t cnc_launch(int policy, bool fuse, bool persistent, const DevCircuit* c,
                              const Tile* t, uint32_t n, int block, int grid, uint32_t* ctr,
-                             int steps, bool all, hipStream_t s) {
+                             int steps, CncSteps how, hipStream_t s) {
   if (n == 0) return hipSuccess;
   if (persistent && grid < 1) return hipErrorInvalidValue;
   switch (policy) {
     case CKT_POLICY_EXACT:
-      return cnc_by_fuse<CKT_POLICY_EXACT>(fuse, persistent, c, t, n, block, grid, ctr, steps, all, s);
+      return cnc_by_fuse<CKT_POLICY_EXACT>(fuse, persistent, c, t, n, block, grid, ctr, steps, how, s);
     case CKT_POLICY_RECIP:
-      return cnc_by_fuse<CKT_POLICY_RECIP>(fuse, persistent, c, t, n, block, grid, ctr, steps, all, s);
+      return cnc_by_fuse<CKT_POLICY_RECIP>(fuse, persistent, c, t, n, block, grid, ctr, steps, how, s);
     case CKT_POLICY_FAST:
-      return cnc_by_fuse<CKT_POLICY_FAST>(fuse, persistent, c, t, n, block, grid, ctr, steps, all, s);
+      return cnc_by_fuse<CKT_POLICY_FAST>(fuse, persistent, c, t, n, block, grid, ctr, steps, how, s);
     case CKT_POLICY_SCALED:
-      return cnc_by_fuse<CKT_POLICY_SCALED>(fuse, persistent, c, t, n, block, grid, ctr, steps, all, s);
+      return cnc_by_fuse<CKT_POLICY_SCALED>(fuse, persistent, c, t, n, block, grid, ctr, steps, how, s);
     default: return hipErrorInvalidValue;
   }
 }
 
 hipError_t launch_cnc(int policy, bool fuse_dsc, const DevCircuit* c, const Tile* t, uint32_t n,
-                      int block, int steps, bool all, hipStream_t s) {
-  return cnc_launch(policy, fuse_dsc, false, c, t, n, block, 0, nullptr, steps, all, s);
+                      int block, int steps, CncSteps how, hipStream_t s) {
+  return cnc_launch(policy, fuse_dsc, false, c, t, n, block, 0, nullptr, steps, how, s);
 }
 
 hipError_t launch_cnc_persistent(int policy, bool fuse_dsc, const DevCircuit* c, const Tile* t,
                                  uint32_t n, int block, int grid, uint32_t* ctr, int steps,
-                                 bool all, hipStream_t s) {
-  return cnc_launch(policy, fuse_dsc, true, c, t, n, block, grid, ctr, steps, all, s);
+                                 CncSteps how, hipStream_t s) {
+  return cnc_launch(policy, fuse_dsc, true, c, t, n, block, grid, ctr, steps, how, s);
 }
 
 hipError_t launch_dsc_atomic(const DevCircuit* c, const Tile* t, uint32_t n, int block,
