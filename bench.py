@@ -192,11 +192,11 @@ def batched_measure(C, policy_name, loops=5):
     b.add_generated_many(shapes, [loops] * len(shapes), threads=min(16, host_threads()))
     log(f"[batched] {len(shapes)} circuits, {W_total} wires, added in "
         f"{time.perf_counter() - t0:.1f} s")
-    # The library's default schedule (256-thread persistent workgroups, 4
-    # resident waves per SIMD, one tile per 256 wires of a piece, pieces in
-    # order) against the autotuned one, as probes and as whole runs.
-    default = C.Batch.config(policy=pol, mode=C.REDUCE_ATOMIC, block_threads=256, persistent=1,
-                             waves_per_simd=4, wires_per_lane=1, tile_span=0, tile_order=0)
+    # The library's default schedule (a plain grid of 256-thread workgroups, one
+    # tile per 256 wires of a piece, pieces in order) against the autotuned one,
+    # as probes and as whole runs.  A probe's steps end early like a run's.
+    default = C.Batch.config(policy=pol, mode=C.REDUCE_ATOMIC, block_threads=256, persistent=0,
+                             wires_per_lane=1, tile_span=0, tile_order=0)
     default_probe_ms = b.probe(default, probe_steps=2000)
     best, _ = b.autotune(pol, probe_steps=2000)
     best_probe_ms = b.probe(best, probe_steps=2000)
@@ -216,7 +216,8 @@ def batched_measure(C, policy_name, loops=5):
     #  (a) one launch per piece per task with a wait after each (how the
     #      reference runtime runs GPU point tasks);
     #  (b) plain launches: one per task over all pieces, no fusion, no graph;
-    #  (c) this library's own loop driver: fused epilogue, graph-captured.
+    #  (c) this library's own loop driver with its defaults: the second and
+    #      third task joined, graphs of sixteen loops where there are as many.
     seq_piece = seq_plain = seq_task = 0.0
     ctx = C.Context(0)
     for i, s in enumerate(shapes):
@@ -226,7 +227,7 @@ def batched_measure(C, policy_name, loops=5):
                                    per_piece=True)["elapsed_s"]
         seq_plain += ctx.run_loops(loops, policy=pol,
                                    mode=C.REDUCE_ATOMIC)["elapsed_s"]
-        ctx.set_option(C.OPT_FUSE_DSC, 1)
+        ctx.set_option(C.OPT_FUSE_DSC, -1)
         seq_task += ctx.run_loops(loops, policy=pol, mode=C.REDUCE_ATOMIC,
                                   use_graph=True)["elapsed_s"]
         if i % 128 == 127:
@@ -236,7 +237,7 @@ def batched_measure(C, policy_name, loops=5):
     return {"workload": "512 circuits, wires log-uniform in [2^10, 2^18], nodes = wires/4, "
                         "pieces = ceil(nodes/4096), 95% in-piece, 10000 inner steps, "
                         f"{loops} loops each, {policy_name.upper()} policy, ATOMIC reduction, "
-                        "hipGraph per loop",
+                        "use_graph on",
             "total_wires": W_total,
             "autotuned": best.describe(),
             "wire_updates_per_s": rep["wire_updates_per_s"], "elapsed_s": rep["elapsed_s"],
@@ -248,10 +249,10 @@ def batched_measure(C, policy_name, loops=5):
             "autotune_gain": rep_default["elapsed_s"] / rep["elapsed_s"],
             "sequential_per_piece": {"elapsed_s": seq_piece, "wire_updates_per_s": wu / seq_piece},
             "sequential_plain": {"elapsed_s": seq_plain, "wire_updates_per_s": wu / seq_plain},
-            "sequential_fused_graph": {"elapsed_s": seq_task, "wire_updates_per_s": wu / seq_task},
+            "sequential_own_loop": {"elapsed_s": seq_task, "wire_updates_per_s": wu / seq_task},
             "speedup_vs_sequential_per_piece": seq_piece / rep["elapsed_s"],
             "speedup_vs_sequential_plain": seq_plain / rep["elapsed_s"],
-            "speedup_vs_sequential_fused_graph": seq_task / rep["elapsed_s"]}
+            "speedup_vs_sequential_own_loop": seq_task / rep["elapsed_s"]}
 
 
 def run_batched(C, args):
@@ -321,7 +322,7 @@ def served_measure(C, policy_name, rate, seconds, cap_wires, timeout_s=0.0,
            "per_loop_s_by_wires": {str(int(w)): t for w, t in zip(sizes, t_loop)}}
     # The most any batching of these requests can gain over that: all of
     # their work at the rate one circuit that fills the GPU runs at in the
-    # library's own loop (4,194,304 wires, fused epilogue, graph-captured).
+    # library's own loop (4,194,304 wires).
     ctx = C.Context(0)
     ctx.generate_device(C.shape_for_wires(1 << 22, 95, 78, C.PROFILE_REFERENCE))
     ctx.run_loops(1, policy=pol, mode=C.REDUCE_ATOMIC, use_graph=True)

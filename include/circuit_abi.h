@@ -318,7 +318,8 @@ typedef struct ckt_loop_config {
   int32_t policy;
   int32_t reduce_mode;
   int32_t sync;      /* -sync: 0 none, 1 wait after every launch, 2 NOP launches only */
-  int32_t use_graph; /* capture one loop in a hipGraph and replay it */
+  int32_t use_graph; /* 1: sixteen loops at a time are replayed from a hipGraph; fewer
+                        loops, and the rest, are launched directly */
   int32_t per_piece; /* 1: one launch per piece per task with a wait after each,
                         as the reference runtime runs GPU point tasks
                         (lowlevel_gpu.cc:117-160); 0: one launch per task */
@@ -378,7 +379,8 @@ typedef struct ckt_batch ckt_batch_t;
 typedef struct ckt_batch_config {
   int32_t policy;
   int32_t reduce_mode;
-  int32_t use_graph;        /* capture each loop's launches in a hipGraph */
+  int32_t use_graph;        /* as in ckt_loop_config_t, while the set of active
+                               circuits stays the same */
   int32_t block_threads;    /* 64..1024, multiple of 64; 0 = autotuned/default */
   int32_t persistent;       /* 1: calc_new_currents as a persistent tile-queue kernel */
   int32_t waves_per_simd;   /* persistent grid size = CUs * 4 * waves_per_simd */

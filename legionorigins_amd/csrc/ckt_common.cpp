@@ -266,7 +266,9 @@ static int noalloc_scratch(unsigned char** out) {
 // 65536 wires, 168 with the LDS form, 121 and 62 for 64 x 16384.  The
 // LDS form has two launches, and an atomic per node with a contribution, so it
 // wants large tables with several wires per node; its two sums per node have
-// to fit in LDS, and the rows in 64 MiB.
+// to fit in LDS, and the rows in 64 MiB.  The forms meet at 2^18 wires (us a call,
+// LDS / atomics: 64 x 2048 wires 38 / 28, 64 x 4096 39 / 41, 16 x 16384 42 / 42, 64
+// x 8192 45 / 69).
 struct ChargePlan {
   uint32_t splits = 0, stride = 0;
   size_t bytes = 0;

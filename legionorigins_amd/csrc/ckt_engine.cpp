@@ -1062,8 +1062,9 @@ int Engine::launch_loop(const std::vector<PieceRef>& refs, int policy, int mode)
 // with the LDS reduction as its own launch: 64 x 65536 wires 230 / 417 / 234, 16 x
 // 16384 21 / 34 / 29, 4 x 4096 11.9 / 10.7 / 18.7; the first of these is 201 now
 // that calc_new_currents leaves the index its cached currents).  Where every step runs, the
-// atomics hide behind the steps of other waves and stay fused.  The options that
-// name an ATOMIC form get it.
+// atomics hide behind the steps of other waves and stay fused.  OPT_FUSE_DSC names the
+// form; where it does not, a named OPT_DSC_ATOMIC_IMPL, which is about launches of
+// distribute_charge alone, leaves the loops the fused atomics.
 constexpr uint64_t kIndexSumWires = 32768;
 
 Engine::LoopForm Engine::loop_form(const std::vector<PieceRef>& refs, int mode) const {

@@ -103,6 +103,9 @@ struct PieceIndex {
 
 // The piece table as a kernel argument: tables of up to kInlinePieces by
 // value (no copy to the device goes before the launch), longer ones by `ix`.
+// 64 pieces make 1.3 KB of arguments.  Microseconds a call over 64 / 65 pieces of
+// 64 wires: calc_new_currents 19.2 / 49.7, distribute_charge 16.3 / 46.9,
+// update_voltages 15.3 / 37.8.
 constexpr uint32_t kInlinePieces = 64;
 struct PieceArgs {
   PieceIndex ix;

@@ -103,8 +103,15 @@ __device__ __forceinline__ bool wave_all(bool p) { return __all(p); }
 //
 // One check costs about one step.  Windows of kWin steps are compared one
 // after another up to step kDense, then one window of kWide steps every
-// kPlain steps, so that a wire that never repeats itself pays under 1%.  A
-// wave ends when all its active lanes do.  The state at a window's start is
+// kPlain steps, so that the checks of a wire that never repeats itself cost
+// little (undamped wires, EXACT, 64 x 65536: 109 ms a launch with them, without
+// those after the first 64 steps, and with every step in the same grid).  What such
+// wires do lose is the launch shape, which Engine::cnc chooses for wires that
+// end early: EXACT takes 105 ms where every step executed in its queue takes 100;
+// SCALED, FAST and RECIP run undamped wires in reference order and lose nothing
+// (135, 133 and 134 ms for 136, 135 and 136).  A wire that repeats itself later than
+// step 64 is found within about 1030 steps of that (L = 0.97 R dt: 13 to 16 ms a
+// launch instead of 100 and 131).  A wave ends when all its active lanes do.  The state at a window's start is
 // kept in LDS (one column per lane, no barrier), not in registers: ten more
 // live registers in the step loops would cost EXACT an occupancy step.
 typedef __attribute__((address_space(3))) float lfloat;
@@ -115,10 +122,9 @@ __device__ __forceinline__ bool same_value(float a, float b) {
 
 //
 // A kernel takes the early end with Settle and executes every step with
-// EveryStep: a template parameter, because the step loops with the checks
-// around them allocate 10 to 30 more registers and ran 3-5% slower than the
-// bare loops (SCALED 10.98 against 10.45 ms, EXACT 94.7 against 92.3 ms for
-// 64 x 65536 wires with every step executed).
+// EveryStep: a template parameter, because with a run-time flag the step loops
+// that execute every step ran 3-5% slower than the bare ones (SCALED 10.98 against
+// 10.45 ms, EXACT 94.7 against 92.3 ms for 64 x 65536 wires, in the same queue).
 struct EveryStep {
   static constexpr bool on = false, stream = false;
   __device__ __forceinline__ EveryStep(lfloat*, uint32_t) {}
@@ -1551,8 +1557,9 @@ __global__ __launch_bounds__(256) void dsc_aos_kernel(PieceArgs ix,
 // all others to memory with atomics, and the sums are written as rows of
 // `partial` (`stride` private sums, then `stride` shared ones), which
 // dsc_aos_sum_kernel adds to the instances -- with atomics, because calls on
-// other streams may add to the same nodes.  Bound by the records: 64 bytes of
-// each cross the bus for the 24 in use.
+// other streams may add to the same nodes.  Bound by the records' memory
+// traffic: whole 128-byte lines cross the bus, one per record for the 24 bytes in
+// use (64 x 65536 wires: 0.57 GB with the rows in 111 us, 5.1 TB/s).
 __global__ __launch_bounds__(1024) void dsc_aos_lds_kernel(PieceArgs ix, uint32_t splits,
                                                            const ckt_wire_t* __restrict__ wires,
                                                            ckt_node_t* pvt, float* owned_fold,
