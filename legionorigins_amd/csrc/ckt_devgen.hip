@@ -89,28 +89,24 @@ __global__ __launch_bounds__(256) void gen_nodes(uint32_t N, uint64_t seed_state
 // The index of a small circuit in one workgroup: entry and node packed into
 // 32 bits and sorted by node in LDS (stable, so entries keep their order), then
 // each entry that starts a new node fills the rows up to it.  One launch for
-// the device-wide sort's eight and the rows': adding a circuit of 1600 wires
-// takes 66 us instead of 93.
+// the device-wide sort's eight and the rows': generating 4 x 1024 wires takes 77
+// us instead of 85.
 constexpr uint32_t kSmallLanes = 512, kSmallEach = 16, kSmallEntries = kSmallLanes * kSmallEach;
 constexpr unsigned kEntryBits = 13;
 static_assert(kSmallEntries == 1u << kEntryBits, "an entry fits its bits");
 
-__global__ __launch_bounds__(kSmallLanes) void index_small(DevCircuit c, unsigned bits,
-                                                           const LoadFaults* faults,
-                                                           LoadFaults* host_faults) {
+__global__ __launch_bounds__(kSmallLanes) void index_small(DevCircuit c, unsigned bits) {
   using Sort = rocprim::block_radix_sort<uint32_t, kSmallLanes, kSmallEach>;
   __shared__ typename Sort::storage_type storage;
   __shared__ uint32_t last[kSmallLanes];
   const uint32_t t = threadIdx.x, E = 2 * c.num_wires;
-  if (t == 0 && faults) *host_faults = *faults;
   uint32_t item[kSmallEach];
 #pragma unroll
   for (uint32_t u = 0; u < kSmallEach; u++) {
-    // Past the end: the largest node, after every real entry of it.  An
-    // invalid pointer is refused after the build; here it has to stay in range.
+    // Past the end: the largest node, after every real entry of it.
     const uint32_t e = t * kSmallEach + u;
     uint32_t n = c.num_nodes - 1;
-    if (e < E) n = min(n, (e & 1u) ? c.out_ptr[e >> 1] : c.in_ptr[e >> 1]);
+    if (e < E) n = (e & 1u) ? c.out_ptr[e >> 1] : c.in_ptr[e >> 1];
     item[u] = n << kEntryBits | e;
   }
   Sort().sort(item, storage, kEntryBits, kEntryBits + bits);
@@ -473,6 +469,13 @@ unsigned key_bits(uint32_t N) {
   return bits;
 }
 
+// Circuits of up to 4096 wires and 2^15 nodes (with many more nodes than entries
+// the rows between them, written by one lane, would take longer than the launches
+// saved).
+bool index_is_small(uint32_t N, uint32_t W) {
+  return 2ull * W <= kSmallEntries && N <= 1u << 15;
+}
+
 // Locations, then the index (from the entries, or for a small circuit from
 // the pointers).
 int enqueue_index(const ckt_gen_params_t* p, uint32_t N, uint32_t W, const SlabView& v,
@@ -492,7 +495,8 @@ int enqueue_index(const ckt_gen_params_t* p, uint32_t N, uint32_t W, const SlabV
   c.in_ptr = v.u(v.L.in_ptr);
   c.out_ptr = v.u(v.L.out_ptr);
   if (index_is_small(N, W)) {
-    CKT_HIP(launch_index_small(c, nullptr, nullptr, s));
+    hipLaunchKernelGGL(index_small, dim3(1), dim3(kSmallLanes), 0, s, c, key_bits(N));
+    CKT_HIP(hipGetLastError());
     return CKT_OK;
   }
   if (int st = index_sort(c, sc, s)) return st;
@@ -520,19 +524,6 @@ int index_scratch(uint32_t N, uint32_t W, void* base, IndexScratch* sc, size_t* 
     sc->sort_bytes = sort_bytes;
   }
   return CKT_OK;
-}
-
-// With many more nodes than entries the rows between them, written by one
-// lane, would take longer than the launches saved.
-bool index_is_small(uint32_t N, uint32_t W) {
-  return 2ull * W <= kSmallEntries && N <= 1u << 15;
-}
-
-hipError_t launch_index_small(const DevCircuit& c, const LoadFaults* faults,
-                              LoadFaults* host_faults, hipStream_t s) {
-  hipLaunchKernelGGL(index_small, dim3(1), dim3(kSmallLanes), 0, s, c, key_bits(c.num_nodes), faults,
-                     host_faults);
-  return hipGetLastError();
 }
 
 int index_sort(const DevCircuit& c, const IndexScratch& sc, hipStream_t s) {

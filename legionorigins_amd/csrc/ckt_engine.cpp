@@ -115,19 +115,29 @@ int image_from_aos(SlabImage& img, const ckt_node_t* nodes, uint32_t N, const ck
   float *ind = img.at<float>(L.ind), *res = img.at<float>(L.res), *wcap = img.at<float>(L.wcap);
   uint32_t *in_ptr = img.at<uint32_t>(L.in_ptr), *out_ptr = img.at<uint32_t>(L.out_ptr);
   uint8_t *in_loc = img.at<uint8_t>(L.in_loc), *out_loc = img.at<uint8_t>(L.out_loc);
-  for (uint32_t w = 0; w < W; w++) {
-    const ckt_wire_t& x = wires[w];
-    for (int s = 0; s < kSeg; s++) cur[s * ws + w] = x.current[s];
-    for (int s = 0; s < kSeg - 1; s++) vol[s * ws + w] = x.voltage[s];
-    ind[w] = x.inductance;
-    res[w] = x.resistance;
-    wcap[w] = x.capacitance;
-    in_ptr[w] = x.in_ptr;
-    out_ptr[w] = x.out_ptr;
-    if (x.in_loc < 0 || x.in_loc > 2 || x.out_loc < 0 || x.out_loc > 2)
-      return fail(CKT_ERR_INVALID_ARG, "wire " + std::to_string(w) + " has an invalid PointerLocation");
-    in_loc[w] = (uint8_t)x.in_loc;
-    out_loc[w] = (uint8_t)x.out_loc;
+  // A block of records at a time, array by array: the arrays lie a multiple of
+  // the wire stride apart, and where that is a power of two, 26 of them written in
+  // turn push each other out of the cache (4096 wires took 376 us, 4097 took 64).
+  constexpr uint32_t kBlock = 64;
+  for (uint32_t first = 0; first < W; first += kBlock) {
+    const ckt_wire_t* x = wires + first;
+    const uint32_t n = std::min(kBlock, W - first);
+    for (int s = 0; s < kSeg; s++)
+      for (uint32_t k = 0; k < n; k++) cur[s * ws + first + k] = x[k].current[s];
+    for (int s = 0; s < kSeg - 1; s++)
+      for (uint32_t k = 0; k < n; k++) vol[s * ws + first + k] = x[k].voltage[s];
+    for (uint32_t k = 0; k < n; k++) ind[first + k] = x[k].inductance;
+    for (uint32_t k = 0; k < n; k++) res[first + k] = x[k].resistance;
+    for (uint32_t k = 0; k < n; k++) wcap[first + k] = x[k].capacitance;
+    for (uint32_t k = 0; k < n; k++) in_ptr[first + k] = x[k].in_ptr;
+    for (uint32_t k = 0; k < n; k++) out_ptr[first + k] = x[k].out_ptr;
+    for (uint32_t k = 0; k < n; k++) {
+      if ((uint32_t)x[k].in_loc > 2 || (uint32_t)x[k].out_loc > 2)
+        return fail(CKT_ERR_INVALID_ARG,
+                    "wire " + std::to_string(first + k) + " has an invalid PointerLocation");
+      in_loc[first + k] = (uint8_t)x[k].in_loc;
+      out_loc[first + k] = (uint8_t)x[k].out_loc;
+    }
   }
   float *charge = img.at<float>(L.charge), *voltage = img.at<float>(L.voltage);
   float *ncap = img.at<float>(L.ncap), *leak = img.at<float>(L.leak);
@@ -232,7 +242,17 @@ static uint64_t piece_key(const ckt_piece_t& p) {
 // allocating it costs such a build 0.3 ms of 1.3.  The default budget's share (1
 // GB) is the scratch of 25 M wires.
 constexpr uint64_t kKeepShare = 256;
-constexpr uint32_t kDeviceLoadWires = 512;
+
+// How a load goes, by the slab's size (us a load with its wait, nodes = wires / 4).
+// Up to kHostLoadBytes the host unpacks and checks the records and the slab goes up
+// whole: 1500 wires 34 against 90 on the device, 3000 50 / 101, 6000 84 / 115, 8000
+// 110 / 118; 9500 147 / 137, 11000 160 / 149.  It goes through a pinned slot, because
+// the runtime's copy from pageable memory is slow for its first 10 MB or so in a
+// process (6000 wires 340, then 76; the very first one sets the runtime up in 9 ms,
+// a slot in 1); slabs up to kPageableLoadBytes are copied by the runtime all the
+// same (700 wires 51, then 23, against 26).
+constexpr size_t kHostLoadBytes = 1 << 20;
+constexpr size_t kPageableLoadBytes = 128 << 10;
 
 Engine::~Engine() {
   if (device_ < 0) return;
@@ -286,7 +306,7 @@ int Engine::init(int device, uint64_t budget_bytes) {
   return CKT_OK;
 }
 
-int Engine::add(SlabImage& img, int32_t loops, uint32_t* id) {
+int Engine::add(SlabImage& img, int32_t loops, uint32_t* id, bool pinned) {
   CKT_HIP(hipSetDevice(device_));
   if (budget_ && in_use_ + img.lay.total > budget_)
     return fail(CKT_ERR_BUDGET, "circuit needs " + std::to_string(img.lay.total) +
@@ -296,10 +316,20 @@ int Engine::add(SlabImage& img, int32_t loops, uint32_t* id) {
   void* slab = nullptr;
   hipError_t e = alloc_slab(img.lay.total, &slab);
   if (e != hipSuccess) return hip_fail(e, "hipMalloc(circuit)");
-  e = hipMemcpy(slab, img.bytes.data(), img.lay.total, hipMemcpyHostToDevice);
-  if (e != hipSuccess) {
+  if (pinned) {
+    st = ring_.in(img.bytes.data(), 16, (uint32_t)(img.lay.total / 16), device_, stream_,
+                  [&](void* slot, uint32_t first, uint32_t n) {
+                    return launch_copy_words((uint32_t*)slab + 4 * (size_t)first, (uint32_t*)slot,
+                                             4 * n, stream_);
+                  });
+    e = hipStreamSynchronize(stream_);
+  } else {
+    e = hipMemcpy(slab, img.bytes.data(), img.lay.total, hipMemcpyHostToDevice);
+  }
+  if (!st && e != hipSuccess) st = hip_fail(e, "circuit upload");
+  if (st) {
     (void)hipFree(slab);
-    return hip_fail(e, "hipMemcpy(circuit upload)");
+    return st;
   }
   attach(slab, img.lay, img.N, img.W, img.P, img.pieces, loops, id);
   return CKT_OK;
@@ -417,16 +447,11 @@ int Engine::build_records(const ckt_node_t* nodes, const ckt_wire_t* wires, cons
   const PieceIndex ix{c.pieces, d_blocks, good};
   CKT_HIP(launch_check_pieces(ix, blocks.back(), c, faults, stream_));
   LoadFaults f;
-  if (index_is_small(N, W)) {
-    st = ring_.out(&f, sizeof(f), 1, device_, stream_, [&](void* slot, uint32_t, uint32_t) {
-      return launch_index_small(c, faults, (LoadFaults*)slot, stream_);
-    });
-  } else if (!(st = index_sort(c, sc, stream_))) {
-    st = ring_.out(&f, sizeof(f), 1, device_, stream_, [&](void* slot, uint32_t, uint32_t) {
-      return launch_index_rows(c, sc, faults, (LoadFaults*)slot, stream_);
-    });
-  }
-  if (st) return st;
+  if ((st = index_sort(c, sc, stream_)) ||
+      (st = ring_.out(&f, sizeof(f), 1, device_, stream_, [&](void* slot, uint32_t, uint32_t) {
+         return launch_index_rows(c, sc, faults, (LoadFaults*)slot, stream_);
+       })))
+    return st;
   // In the order in which a pass over wires, then pieces, meets them.
   if (~f.location)
     return fail(CKT_ERR_INVALID_ARG,
@@ -457,13 +482,12 @@ int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* w
   // The device path holds the new circuit and its scratch beside the replaced
   // one.  Where the budget or the memory has no room for that, the records are
   // unpacked and checked on the host and the replaced circuit leaves first; so
-  // are the smallest circuits, for which that is faster (256 wires 30 us against
-  // 54, 1024 wires 110 against 56).
+  // are small circuits.
   void *slab = nullptr, *own = nullptr, *scratch = nullptr;
   const size_t need = RecordScratch(N, W, P).bytes, kept = devgen_scratch_cap_;
   const bool keep = need <= budget_ / kKeepShare;
   const uint64_t held = in_use_ + lay.total + (need <= kept ? kept : keep ? need : kept + need);
-  bool fits = W >= kDeviceLoadWires && need && (!budget_ || held <= budget_);
+  bool fits = lay.total > kHostLoadBytes && need && (!budget_ || held <= budget_);
   if (fits && (st = build_scratch(need, keep, &scratch, &own))) return st;
   fits = fits && scratch && hipMalloc(&slab, lay.total) == hipSuccess;
   (void)hipGetLastError();
@@ -490,7 +514,7 @@ int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* w
   SlabImage img;
   if ((st = image_from_aos(img, nodes, N, wires, W, locator, pieces, P))) return st;
   if (replaced && (st = remove(*replaced))) return st;
-  return add(img, loops, id);
+  return add(img, loops, id, lay.total > kPageableLoadBytes && lay.total <= HostRing::kSlotBytes);
 }
 
 int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loops, uint32_t* id) {
@@ -834,6 +858,9 @@ constexpr uint64_t kLastLevelCacheBytes = 256ull << 20;
 // 15.7 / 15.7, 256k 19.3 / 20.3, 384k 27.3 / 27.8, 512k 36.0 / 36.9; 768k 45.8 /
 // 41.2, 1024k 59.3 / 51.7, 2048k 109 / 89.5, 2304k 119 / 101; 2560k 132 / 144, 4096k
 // 200 / 230.  FAST and RECIP alike, EXACT with smaller steps in the same places.
+// Circuits that together exceed the cache and run one loop in turn lose by it (8 of
+// 1024k wires 75 / 79), with two loops each they gain as much as they lose (67 / 66),
+// with five they gain (62 / 58).
 constexpr uint64_t kL2Bytes = 8 * (4ull << 20);
 constexpr uint64_t kCncBytesPerWire = 104;
 

@@ -36,11 +36,6 @@ int index_sort(const DevCircuit& c, const IndexScratch& sc, hipStream_t s);
 hipError_t launch_index_rows(const DevCircuit& c, const IndexScratch& sc, const LoadFaults* faults,
                              LoadFaults* host_faults, hipStream_t s);
 
-// Circuits of up to 4096 wires and 2^15 nodes: the whole index, from the
-// circuit's pointers, in one workgroup (faults as for launch_index_rows).
-bool index_is_small(uint32_t N, uint32_t W);
-hipError_t launch_index_small(const DevCircuit& c, const LoadFaults* faults,
-                              LoadFaults* host_faults, hipStream_t s);
 
 // What a load reads besides the wires, in one piece of pinned memory: nodes,
 // locator (if `locator`), pieces, and the pieces' first workgroups, each on a

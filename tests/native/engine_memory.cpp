@@ -73,7 +73,6 @@ int devgen_enqueue(const ckt_gen_params_t* p, const SlabLayout&, void*, void*, h
   pieces.assign(1, ckt_piece_t{0, (uint32_t)p->wires_per_piece, 0, (uint32_t)p->nodes_per_piece});
   return CKT_OK;
 }
-bool index_is_small(uint32_t, uint32_t) { return false; }
 int index_sort(const DevCircuit&, const IndexScratch&, hipStream_t) { return CKT_OK; }
 hipError_t launch_index_rows(const DevCircuit&, const IndexScratch&, const LoadFaults*,
                              LoadFaults* host, hipStream_t) {
@@ -114,7 +113,7 @@ static void expect(bool ok, const char* what, uint64_t a, uint64_t b) {
   fails++;
 }
 
-constexpr uint32_t N = 500, W = 4000;
+constexpr uint32_t N = 500, W = 40000;  // enough for a load on the device
 constexpr size_t kFixed = 4096;  // the engine's counters
 static const size_t kSlab = SlabLayout::make(N, W, 1).total;
 static const size_t kScratch = scratch_of(W) + 4096;
