@@ -245,14 +245,11 @@ constexpr uint64_t kKeepShare = 256;
 
 // How a load goes, by the slab's size (us a load with its wait, nodes = wires / 4).
 // Up to kHostLoadBytes the host unpacks and checks the records and the slab goes up
-// whole: 1500 wires 34 against 90 on the device, 3000 50 / 101, 6000 84 / 115, 8000
-// 110 / 118; 9500 147 / 137, 11000 160 / 149.  It goes through a pinned slot, because
-// the runtime's copy from pageable memory is slow for its first 10 MB or so in a
-// process (6000 wires 340, then 76; the very first one sets the runtime up in 9 ms,
-// a slot in 1); slabs up to kPageableLoadBytes are copied by the runtime all the
-// same (700 wires 51, then 23, against 26).
-constexpr size_t kHostLoadBytes = 1 << 20;
-constexpr size_t kPageableLoadBytes = 128 << 10;
+// whole: 700 wires 22 against 77 on the device, 1500 30 / 83, 3000 45 / 94, 6000 77 /
+// 108, 9500 120 / 135, 11000 137 / 143; 13000 158 / 152, 14500 173 / 160.  It goes up
+// from pinned memory, because the runtime's copy from pageable memory is slow for
+// its first 10 MB or so in a process (3000 wires 175, then 45; 9500 320, then 130).
+constexpr size_t kHostLoadBytes = 1408 << 10;
 
 Engine::~Engine() {
   if (device_ < 0) return;
@@ -316,20 +313,13 @@ int Engine::add(SlabImage& img, int32_t loops, uint32_t* id, bool pinned) {
   void* slab = nullptr;
   hipError_t e = alloc_slab(img.lay.total, &slab);
   if (e != hipSuccess) return hip_fail(e, "hipMalloc(circuit)");
-  if (pinned) {
-    st = ring_.in(img.bytes.data(), 16, (uint32_t)(img.lay.total / 16), device_, stream_,
-                  [&](void* slot, uint32_t first, uint32_t n) {
-                    return launch_copy_words((uint32_t*)slab + 4 * (size_t)first, (uint32_t*)slot,
-                                             4 * n, stream_);
-                  });
-    e = hipStreamSynchronize(stream_);
-  } else {
-    e = hipMemcpy(slab, img.bytes.data(), img.lay.total, hipMemcpyHostToDevice);
-  }
-  if (!st && e != hipSuccess) st = hip_fail(e, "circuit upload");
-  if (st) {
+  const void* from = img.bytes.data();
+  if (void* slot = pinned ? ring_.pinned(img.lay.total) : nullptr)
+    from = std::memcpy(slot, from, img.lay.total);
+  e = hipMemcpy(slab, from, img.lay.total, hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
     (void)hipFree(slab);
-    return st;
+    return hip_fail(e, "hipMemcpy(circuit upload)");
   }
   attach(slab, img.lay, img.N, img.W, img.P, img.pieces, loops, id);
   return CKT_OK;
@@ -514,7 +504,7 @@ int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* w
   SlabImage img;
   if ((st = image_from_aos(img, nodes, N, wires, W, locator, pieces, P))) return st;
   if (replaced && (st = remove(*replaced))) return st;
-  return add(img, loops, id, lay.total > kPageableLoadBytes && lay.total <= HostRing::kSlotBytes);
+  return add(img, loops, id, lay.total <= HostRing::kSlotBytes);
 }
 
 int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loops, uint32_t* id) {

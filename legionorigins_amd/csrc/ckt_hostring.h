@@ -97,6 +97,13 @@ class HostRing {
     return CKT_OK;
   }
 
+  // `bytes` (kSlotBytes at most) of pinned memory until the next call here, or
+  // NULL if there is none.
+  void* pinned(size_t bytes) {
+    Slot& sl = *small_slot();
+    return acquire(sl, bytes) == CKT_OK && sl.pinned ? sl.p : nullptr;
+  }
+
   // Calls launch(slot, first, n) for the kernels that write records into
   // slots on `s`, and copies each slot to `dst` when its kernel has run.
   // Returns when all records are there.
