@@ -250,6 +250,11 @@ constexpr uint64_t kKeepShare = 256;
 // from pinned memory, because the runtime's copy from pageable memory is slow for
 // its first 10 MB or so in a process (3000 wires 175, then 45; 9500 320, then 130).
 constexpr size_t kHostLoadBytes = 1408 << 10;
+// Slabs up to this size are stored with one copy of the slab and a pass on the
+// host (300 wires 16 us against 20 for a launch that packs the records, 500 18 / 20,
+// 900 22 / 23; in a process's first 200 stores or so 30 and 20, for the same reason,
+// but a copy to pinned memory takes 21 at any time).
+constexpr size_t kHostStoreBytes = 64 << 10;
 
 Engine::~Engine() {
   if (device_ < 0) return;
@@ -691,13 +696,47 @@ void Engine::all_refs(std::vector<PieceRef>& refs, bool only_active) const {
   }
 }
 
+// The records of the slab `b`, in host memory; either array may be NULL.
+static void aos_from_slab(const uint8_t* b, const SlabLayout& L, ckt_node_t* nodes, uint32_t N,
+                          ckt_wire_t* wires, uint32_t W) {
+  auto real = [&](size_t off) { return (const float*)(b + off); };
+  auto word = [&](size_t off) { return (const uint32_t*)(b + off); };
+  constexpr uint32_t kBlock = 64;  // array by array, as in image_from_aos
+  for (uint32_t first = 0; wires && first < W; first += kBlock) {
+    ckt_wire_t* x = wires + first;
+    const uint32_t n = std::min(kBlock, W - first);
+    std::memset(x, 0, n * sizeof(ckt_wire_t));
+    for (uint32_t k = 0; k < n; k++) x[k].in_ptr = word(L.in_ptr)[first + k];
+    for (uint32_t k = 0; k < n; k++) x[k].out_ptr = word(L.out_ptr)[first + k];
+    for (uint32_t k = 0; k < n; k++) x[k].in_loc = b[L.in_loc + first + k];
+    for (uint32_t k = 0; k < n; k++) x[k].out_loc = b[L.out_loc + first + k];
+    for (uint32_t k = 0; k < n; k++) x[k].inductance = real(L.ind)[first + k];
+    for (uint32_t k = 0; k < n; k++) x[k].resistance = real(L.res)[first + k];
+    for (uint32_t k = 0; k < n; k++) x[k].capacitance = real(L.wcap)[first + k];
+    for (int s = 0; s < kSeg; s++)
+      for (uint32_t k = 0; k < n; k++) x[k].current[s] = real(L.cur)[s * L.ws + first + k];
+    for (int s = 0; s < kSeg - 1; s++)
+      for (uint32_t k = 0; k < n; k++) x[k].voltage[s] = real(L.vol)[s * L.ws + first + k];
+  }
+  for (uint32_t i = 0; nodes && i < N; i++)
+    nodes[i] = ckt_node_t{real(L.charge)[i], real(L.voltage)[i], real(L.ncap)[i], real(L.leak)[i]};
+}
+
 // The records are put together on the device and written straight into
-// pinned slots; waits for the stream, behind which the kernels are queued.
+// pinned slots; waits for the stream, behind which the kernels are queued.  The
+// smallest circuits' slabs are copied out whole instead.
 int Engine::store(uint32_t id, ckt_node_t* nodes, ckt_wire_t* wires) {
   Circuit* c = find(id);
   if (!c) return fail(CKT_ERR_NOT_FOUND, "no circuit with id " + std::to_string(id));
   CKT_HIP(hipSetDevice(device_));
   int st;
+  if (c->lay.total <= kHostStoreBytes) {
+    std::vector<uint8_t> slab(c->lay.total);
+    CKT_HIP(hipStreamSynchronize(stream_));
+    CKT_HIP(hipMemcpy(slab.data(), c->slab, c->lay.total, hipMemcpyDeviceToHost));
+    aos_from_slab(slab.data(), c->lay, nodes, c->num_nodes, wires, c->num_wires);
+    return CKT_OK;
+  }
   const size_t wire_bytes = sizeof(ckt_wire_t) * (size_t)c->num_wires,
                node_bytes = sizeof(ckt_node_t) * (size_t)c->num_nodes;
   if (wires && nodes && wire_bytes + node_bytes <= HostRing::kSlotBytes)
