@@ -246,14 +246,12 @@ constexpr uint64_t kKeepShare = 256;
 // How a load goes, by the slab's size (us a load with its wait, nodes = wires / 4).
 // Up to kHostLoadBytes the host unpacks and checks the records and the slab goes up
 // whole: 700 wires 22 against 77 on the device, 1500 30 / 83, 3000 45 / 94, 6000 77 /
-// 108, 9500 120 / 135, 11000 137 / 143; 13000 158 / 152, 14500 173 / 160.  It goes up
-// from pinned memory, because the runtime's copy from pageable memory is slow for
-// its first 10 MB or so in a process (3000 wires 175, then 45; 9500 320, then 130).
+// 108, 9500 120 / 135, 11000 137 / 143; 13000 158 / 152, 14500 173 / 160.
 constexpr size_t kHostLoadBytes = 1408 << 10;
 // Slabs up to this size are stored with one copy of the slab and a pass on the
 // host (300 wires 16 us against 20 for a launch that packs the records, 500 18 / 20,
-// 900 22 / 23; in a process's first 200 stores or so 30 and 20, for the same reason,
-// but a copy to pinned memory takes 21 at any time).
+// 900 22 / 23; in a process's first 200 stores or so 30 and 20, see Engine::add,
+// but with a copy to pinned memory 21 at any time).
 constexpr size_t kHostStoreBytes = 64 << 10;
 
 Engine::~Engine() {
@@ -308,7 +306,7 @@ int Engine::init(int device, uint64_t budget_bytes) {
   return CKT_OK;
 }
 
-int Engine::add(SlabImage& img, int32_t loops, uint32_t* id, bool pinned) {
+int Engine::add(SlabImage& img, int32_t loops, uint32_t* id) {
   CKT_HIP(hipSetDevice(device_));
   if (budget_ && in_use_ + img.lay.total > budget_)
     return fail(CKT_ERR_BUDGET, "circuit needs " + std::to_string(img.lay.total) +
@@ -318,8 +316,12 @@ int Engine::add(SlabImage& img, int32_t loops, uint32_t* id, bool pinned) {
   void* slab = nullptr;
   hipError_t e = alloc_slab(img.lay.total, &slab);
   if (e != hipSuccess) return hip_fail(e, "hipMalloc(circuit)");
+  // From pinned memory where a slot holds it: the runtime's copy from pageable
+  // memory is slow for its first 10 MB or so in a process (loads of 3000 wires 175
+  // us, then 45; 9500 wires 320, then 130).
+  const bool fits = img.lay.total <= HostRing::kSlotBytes;
   const void* from = img.bytes.data();
-  if (void* slot = pinned ? ring_.pinned(img.lay.total) : nullptr)
+  if (void* slot = fits ? ring_.pinned(img.lay.total) : nullptr)
     from = std::memcpy(slot, from, img.lay.total);
   e = hipMemcpy(slab, from, img.lay.total, hipMemcpyHostToDevice);
   if (e != hipSuccess) {
@@ -509,7 +511,7 @@ int Engine::add_records(const ckt_node_t* nodes, uint32_t N, const ckt_wire_t* w
   SlabImage img;
   if ((st = image_from_aos(img, nodes, N, wires, W, locator, pieces, P))) return st;
   if (replaced && (st = remove(*replaced))) return st;
-  return add(img, loops, id, lay.total <= HostRing::kSlotBytes);
+  return add(img, loops, id);
 }
 
 int Engine::add_generated_on_device(const ckt_gen_params_t* params, int32_t loops, uint32_t* id) {

@@ -101,8 +101,7 @@ class Engine {
   int num_cus() const { return num_cus_; }
 
   // Circuits.
-  // `pinned`: uploaded through the ring's slots, else by the runtime.
-  int add(SlabImage& img, int32_t loops, uint32_t* id, bool pinned = false);
+  int add(SlabImage& img, int32_t loops, uint32_t* id);
   // A circuit from reference-layout records (ckt_ctx_load): streamed to the
   // device, unpacked, checked and indexed there.  `replaced`, if not NULL, is
   // the id of a circuit to remove once the new one is known to be valid.
