@@ -249,10 +249,11 @@ constexpr uint64_t kKeepShare = 256;
 // 108, 9500 120 / 135, 11000 137 / 143; 13000 158 / 152, 14500 173 / 160.
 constexpr size_t kHostLoadBytes = 1408 << 10;
 // Slabs up to this size are stored with one copy of the slab and a pass on the
-// host (300 wires 16 us against 20 for a launch that packs the records, 500 18 / 20,
-// 900 22 / 23; in a process's first 200 stores or so 30 and 20, see Engine::add,
-// but with a copy to pinned memory 21 at any time).
-constexpr size_t kHostStoreBytes = 64 << 10;
+// host, record by record (300 wires 16 us against 20 to 25 for a launch that packs the
+// records, on two cards; 500 18 / 20 to 25, 900 22 / 23 to 29; in a process's first 200
+// stores or so 30, see Engine::add, but with a copy to pinned memory 21 at any time).
+// From 1024 wires on strides are multiples of 4 KB, for which that pass is slow.
+constexpr size_t kHostStoreBytes = 104 << 10;
 
 Engine::~Engine() {
   if (device_ < 0) return;
@@ -703,22 +704,18 @@ static void aos_from_slab(const uint8_t* b, const SlabLayout& L, ckt_node_t* nod
                           ckt_wire_t* wires, uint32_t W) {
   auto real = [&](size_t off) { return (const float*)(b + off); };
   auto word = [&](size_t off) { return (const uint32_t*)(b + off); };
-  constexpr uint32_t kBlock = 64;  // array by array, as in image_from_aos
-  for (uint32_t first = 0; wires && first < W; first += kBlock) {
-    ckt_wire_t* x = wires + first;
-    const uint32_t n = std::min(kBlock, W - first);
-    std::memset(x, 0, n * sizeof(ckt_wire_t));
-    for (uint32_t k = 0; k < n; k++) x[k].in_ptr = word(L.in_ptr)[first + k];
-    for (uint32_t k = 0; k < n; k++) x[k].out_ptr = word(L.out_ptr)[first + k];
-    for (uint32_t k = 0; k < n; k++) x[k].in_loc = b[L.in_loc + first + k];
-    for (uint32_t k = 0; k < n; k++) x[k].out_loc = b[L.out_loc + first + k];
-    for (uint32_t k = 0; k < n; k++) x[k].inductance = real(L.ind)[first + k];
-    for (uint32_t k = 0; k < n; k++) x[k].resistance = real(L.res)[first + k];
-    for (uint32_t k = 0; k < n; k++) x[k].capacitance = real(L.wcap)[first + k];
-    for (int s = 0; s < kSeg; s++)
-      for (uint32_t k = 0; k < n; k++) x[k].current[s] = real(L.cur)[s * L.ws + first + k];
-    for (int s = 0; s < kSeg - 1; s++)
-      for (uint32_t k = 0; k < n; k++) x[k].voltage[s] = real(L.vol)[s * L.ws + first + k];
+  for (uint32_t w = 0; wires && w < W; w++) {
+    ckt_wire_t& x = wires[w];
+    std::memset(&x, 0, sizeof(x));
+    x.in_ptr = word(L.in_ptr)[w];
+    x.out_ptr = word(L.out_ptr)[w];
+    x.in_loc = b[L.in_loc + w];
+    x.out_loc = b[L.out_loc + w];
+    x.inductance = real(L.ind)[w];
+    x.resistance = real(L.res)[w];
+    x.capacitance = real(L.wcap)[w];
+    for (int s = 0; s < kSeg; s++) x.current[s] = real(L.cur)[s * L.ws + w];
+    for (int s = 0; s < kSeg - 1; s++) x.voltage[s] = real(L.vol)[s * L.ws + w];
   }
   for (uint32_t i = 0; nodes && i < N; i++)
     nodes[i] = ckt_node_t{real(L.charge)[i], real(L.voltage)[i], real(L.ncap)[i], real(L.leak)[i]};

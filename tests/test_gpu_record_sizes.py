@@ -1,5 +1,5 @@
 """Loads and stores either side of the slab sizes at which they change their way:
-64 KiB (stored by a pass on the host or on the device) and 1408 KiB (unpacked on
+104 KiB (stored by a pass on the host or on the device) and 1408 KiB (unpacked on
 the host or on the device), with few and with many nodes."""
 import numpy as np
 import pytest
@@ -21,7 +21,7 @@ def _largest(C, fits, hi):
     return lo
 
 
-@pytest.mark.parametrize("limit", [64 << 10, 1408 << 10])
+@pytest.mark.parametrize("limit", [104 << 10, 1408 << 10])
 @pytest.mark.parametrize("many_nodes", [False, True])
 def test_either_side(C, limit, many_nodes):
     if many_nodes:
