@@ -383,7 +383,10 @@ hipError_t Engine::alloc_slab(size_t bytes, void** slab) {
     (void)hipGetLastError();
     if (drop_scratch() == CKT_OK) e = hipMalloc(slab, bytes);
   }
-  if (e != hipSuccess) *slab = nullptr;
+  if (e != hipSuccess) {
+    *slab = nullptr;
+    (void)hipGetLastError();  // not the next launch's
+  }
   return e;
 }
 
