@@ -344,7 +344,8 @@ enum {
                                     set */
   CKT_OPT_WAVES_PER_SIMD = 3,    /* persistent grid: waves resident per SIMD (1..8);
                                     -1 (default): 7 for EXACT, 4 otherwise */
-  CKT_OPT_DSC_ATOMIC_IMPL = 4,   /* ATOMIC reduction: 0 auto, 1 global atomics, 2 LDS */
+  CKT_OPT_DSC_ATOMIC_IMPL = 4,   /* ATOMIC distribute_charge as a launch of its own: 0 auto,
+                                    1 global atomics, 2 LDS */
   CKT_OPT_FUSE_DSC = 5,          /* the ATOMIC distribute_charge in ckt_run_loops (sync 0,
                                     per_piece 0), batches and servers: 1: done by
                                     calc_new_currents' epilogue from registers; 0: a launch of
