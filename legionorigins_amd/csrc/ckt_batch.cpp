@@ -349,6 +349,7 @@ int ckt_batch_run(ckt_batch_t* b, const ckt_batch_config_t* config, ckt_batch_re
     int32_t k = INT32_MAX;
     for (Circuit* c : E.slots())
       if (c->loops_left > 0) k = std::min(k, c->loops_left);
+    const Engine::LoopsInARow row(E, k);
     if (cfg.use_graph) {
       if ((st = E.run_graph(refs, cfg.policy, cfg.reduce_mode, k))) return st;
     } else {

@@ -292,6 +292,7 @@ int ckt_run_loops(ckt_ctx_t* ctx, int num_loops, const ckt_loop_config_t* config
     return CKT_OK;
   };
 
+  const Engine::LoopsInARow row(E, num_loops);
   if ((st = E.sync())) return st;
   const double t0 = now_s();
   if (cfg.use_graph && !cfg.sync && !cfg.per_piece) {

@@ -888,16 +888,21 @@ constexpr uint64_t kLastLevelCacheBytes = 256ull << 20;
 // nontemporal / ordinary, 16384 wires to 4096 nodes or 65536 to 16384: 128k wires
 // 15.7 / 15.7, 256k 19.3 / 20.3, 384k 27.3 / 27.8, 512k 36.0 / 36.9; 768k 45.8 /
 // 41.2, 1024k 59.3 / 51.7, 2048k 109 / 89.5, 2304k 119 / 101; 2560k 132 / 144, 4096k
-// 200 / 230.  FAST and RECIP alike, EXACT with smaller steps in the same places.
-// Circuits that together exceed the cache and run one loop in turn lose by it (8 of
-// 1024k wires 75 / 79), with two loops each they gain as much as they lose (67 / 66),
-// with five they gain (62 / 58).
+// 200 / 230.  FAST and RECIP alike; EXACT, whose launch its divisions bind, gains 2% there
+// and stays nontemporal.
+//   It takes loops in a row: on a state that is not in the cache yet the ordinary
+// accesses are slower.  Whole calls with the voltages read back, on states that take
+// turns, 1024k and 2048k wires, us: 1 loop 335 / 338 and 576 / 589, 2 loops 416 / 426
+// and 679 / 693, 3 loops 486 / 486 and 796 / 772, 5 loops 631 / 600 and 1083 / 1055, 8 loops
+// 831 / 772 and 1555 / 1425.
 constexpr uint64_t kL2Bytes = 8 * (4ull << 20);
 constexpr uint64_t kCncBytesPerWire = 104;
+constexpr int kCachedLoops = 3;
 
-static bool cnc_state_cached(uint64_t wires) {
+static bool cnc_state_cached(uint64_t wires, int policy, int loops) {
   const uint64_t bytes = wires * kCncBytesPerWire;
-  return bytes > 2 * kL2Bytes && bytes <= kLastLevelCacheBytes;
+  return loops >= kCachedLoops && policy != CKT_POLICY_EXACT && bytes > 2 * kL2Bytes &&
+         bytes <= kLastLevelCacheBytes;
 }
 
 int Engine::tiles_for(int kind, const std::vector<PieceRef>& refs, int block, DevBuf* out) {
@@ -1054,7 +1059,7 @@ int Engine::cnc(const std::vector<PieceRef>& refs, int policy, bool fuse_dsc) {
   uint64_t wires = 0;
   for (const PieceRef& r : refs) wires += slots_[r.slot]->pieces[r.piece].num_wires;
   const CncSteps how = all_steps_ ? kEveryStep
-                       : cnc_state_cached(wires) ? kEarlyEnd
+                       : cnc_state_cached(wires, policy, loops_in_a_row_) ? kEarlyEnd
                                                  : kEarlyEndStream;
   const int waves = waves_per_simd_ > 0 ? waves_per_simd_ : (policy == CKT_POLICY_EXACT ? 7 : 4);
   if (persistent) {
@@ -1356,10 +1361,10 @@ int Engine::run_graph(const std::vector<PieceRef>& refs, int policy, int mode, i
   int st;
   if ((st = ensure_table())) return st;
   uint64_t key = fnv(1469598103934665603ull, refs.data(), refs.size() * sizeof(PieceRef));
-  const int64_t cfg[13] = {policy,           mode,       steps_,          cnc_block_,
+  const int64_t cfg[14] = {policy,           mode,       steps_,          cnc_block_,
                            persistent_,      waves_per_simd_, dsc_atomic_impl_, fuse_dsc_,
                            wires_per_lane_,  tile_span_, tile_order_,     all_steps_,
-                           (int64_t)generation_};
+                           (int64_t)generation_, loops_in_a_row_ >= kCachedLoops};
   key = fnv(key, cfg, sizeof(cfg));
   // Every buffer the launches use is created before any capture (an allocation
   // during capture is not allowed).

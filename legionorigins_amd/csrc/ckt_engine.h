@@ -153,6 +153,19 @@ class Engine {
   int set_option(int opt, int64_t value);
   int64_t option(int opt) const;
 
+  // While one lives, its driver runs `loops` loops in a row over the same
+  // circuits (where none does, a launch is taken to be on its own).
+  class LoopsInARow {
+   public:
+    LoopsInARow(Engine& e, int loops) : e_(e) { e_.loops_in_a_row_ = loops; }
+    ~LoopsInARow() { e_.loops_in_a_row_ = 1; }
+    LoopsInARow(const LoopsInARow&) = delete;
+    LoopsInARow& operator=(const LoopsInARow&) = delete;
+
+   private:
+    Engine& e_;
+  };
+
   // Event timing per task id.
   void set_timing(bool on) { timing_ = on; }
   int kernel_time(int task, double* ms, uint64_t* launches);
@@ -251,6 +264,7 @@ class Engine {
   int tile_span_ = 0;
   int tile_order_ = 0;
   int all_steps_ = 0;
+  int loops_in_a_row_ = 1;
   bool timing_ = false;
   std::vector<Pending> pending_;
   std::vector<hipEvent_t> event_pool_;

@@ -182,6 +182,7 @@ void schedule(ckt_server* s) {
   const ckt_server_config_t cfg = s->cfg;
   int st = CKT_OK;
   if (hipSetDevice(E.device()) != hipSuccess) st = fail(CKT_ERR_HIP, "server: hipSetDevice");
+  const Engine::LoopsInARow row(E, INT32_MAX);  // iterations follow one another
   std::deque<uint32_t> queue;       // arrived, not admitted
   uint64_t reserved = 0;            // bytes of admitted, not retired requests
   uint64_t admitted_wires = 0;      // wires of admitted, not retired requests
